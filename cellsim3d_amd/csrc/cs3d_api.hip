@@ -349,16 +349,9 @@ extern "C" cs3d_status cs3d_ctx_create(int device, const cs3d_mesh* mesh, int64_
     // angle gather table and mesh consistency (every bond listed from both ends)
     MeshDev md;
     std::memset(&md, 0, sizeof(md));
-    std::memcpy(md.nn, mesh->nn, sizeof(md.nn));
-    std::memcpy(md.sign, mesh->sign, sizeof(md.sign));
-    std::memcpy(md.faces, mesh->faces, sizeof(md.faces));
-    std::memcpy(md.R0, mesh->R0, sizeof(md.R0));
-    // reciprocals of the rest lengths for the kernels' quotients (IEEE division here;
-    // NaN where quot_ok fails sends those bonds to the kernels' division path)
-    for (int i = 0; i < 3 * kSlots; ++i)
-        md.R0inv[i] = quot_ok(mesh->R0[i]) ? 1.0f / mesh->R0[i] : std::numeric_limits<float>::quiet_NaN();
-    std::memcpy(md.theta0, mesh->theta0, sizeof(md.theta0));
+    md.theta = kTheta;
     for (int p = 0; p < kNodes; ++p) {
+        int gather[6];
         for (int q = 0; q < 3; ++q) {
             const int n = mesh->nn[q * kSlots + p];
             if (n < 0 || n >= kNodes) return fail(CS3D_INVALID_ARG, "mesh neighbour out of range");
@@ -368,12 +361,27 @@ extern "C" cs3d_status cs3d_ctx_create(int device, const cs3d_mesh* mesh, int64_
             else if (a1 == p) { e0 = (n * 3 + 0) * 6 + 3; e1 = (n * 3 + 1) * 6 + 0; }
             else if (a2 == p) { e0 = (n * 3 + 2) * 6 + 3; e1 = (n * 3 + 1) * 6 + 3; }
             else return fail(CS3D_INVALID_ARG, "mesh neighbour lists are not symmetric");
-            md.gather[p * 6 + 2 * q] = e0;
-            md.gather[p * 6 + 2 * q + 1] = e1;
+            gather[2 * q] = e0;
+            gather[2 * q + 1] = e1;
+            md.th[p].w |= (uint32_t)n << (8 * q);
         }
+        md.r0[p].w = (uint32_t)gather[0] | (uint32_t)gather[1] << 16;
+        md.ir0[p].w = (uint32_t)gather[2] | (uint32_t)gather[3] << 16;
+        md.gs[p].w = (uint32_t)gather[4] | (uint32_t)gather[5] << 16;
+        md.gs[p].sign = (float)mesh->sign[p];
     }
+    for (int k = 0; k < 3; ++k)
+        for (int i = 0; i < kSlots; ++i) {
+            const float r = mesh->R0[k * kSlots + i];
+            md.r0[i].f[k] = r;
+            // reciprocals of the rest lengths for the kernels' quotients (IEEE division here;
+            // NaN where quot_ok fails sends those bonds to the kernels' division path)
+            md.ir0[i].f[k] = quot_ok(r) ? 1.0f / r : std::numeric_limits<float>::quiet_NaN();
+            md.th[i].f[k] = mesh->theta0[3 * i + k];
+        }
     for (int i = 0; i < CS3D_FACES * 7; ++i)
         if (mesh->faces[i] < 0 || mesh->faces[i] >= kNodes) return fail(CS3D_INVALID_ARG, "mesh face index out of range");
+        else md.face[i / 7] |= (uint64_t)mesh->faces[i] << (8 * (i % 7));
 
     cs3d_ctx* c = new cs3d_ctx();
     c->mesh_host = *mesh;
@@ -700,6 +708,10 @@ extern "C" cs3d_status cs3d_get(cs3d_ctx* c, cs3d_sys s, cs3d_field f, void* hos
     }
     HIPCHK(hipMemcpyAsync(host, L.ptr, bytes, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    if (f == CS3D_F_CANDCOUNT) {  // the counts without the list offsets kept above them
+        int32_t* w = static_cast<int32_t*>(host);
+        for (size_t i = 0; i < bytes / 4; ++i) w[i] &= (1 << kCandBits) - 1;
+    }
     return CS3D_OK;
 }
 

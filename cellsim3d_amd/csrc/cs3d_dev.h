@@ -11,7 +11,8 @@
 //                ascending, k-major per cell so lanes access consecutive words
 //                int32[cap_cells * 192]  partner count per node
 //                int32[cap_cells * kPMax * 192]  contact candidates (within attraction_range + skin
-//                at the last search), same layout, + count per node
+//                at the last search): per cell one flat list, node after node, + per node the
+//                count (low kCandBits bits) and the index of its first entry (above them)
 //                float[cap_cells * 192] x3  node positions at the last search
 //   voxel pool   int32                   per system: counts[budget] then lists[budget * capacity]
 //                                        (the reference's 2.9-wide cell grid)
@@ -22,14 +23,20 @@
 // A system (tissue) owns a contiguous range of cell slots [base, base + cap), a voxel
 // region and a bin region; its live cells are base .. base + n - 1 (local 0 .. n - 1).
 #pragma once
+#include <hip/hip_runtime.h>
 #include <stdint.h>
+
 #include "../../include/cs3d.h"
+#include "cs3d_theta.h"
 
 namespace cs3d {
 
 constexpr int kSlots = CS3D_SLOTS;   // 192
 constexpr int kNodes = CS3D_NODES;   // 180
+constexpr int kFacePad = 128;        // rows of the face table (CS3D_FACES, the rest zero)
 constexpr int kPMax = 40;            // contact candidates / partners stored per node
+constexpr int kCandBits = 8;         // low bits of an NCAND word that hold the count
+static_assert(kPMax < (1 << kCandBits), "a node's candidate count fits its bits");
 constexpr int kBCap = CS3D_BIN_CAP;  // nodes per search bin
 constexpr int kMaxSys = 4096;        // systems per context
 constexpr int kMaxPartial = 192;     // listed cells beyond which the next search is a full one (at most the
@@ -83,18 +90,29 @@ struct SysMeta {
 // checks them exhaustively (on the host; results are cached per (m, dt)).
 void kick_consts(float m, float dt, SysMeta& M);
 
-struct MeshDev {
-    int32_t nn[3 * kSlots];
-    int32_t sign[kSlots];
-    int32_t faces[CS3D_FACES * 7];
-    float R0[3 * kSlots];
-    float R0inv[3 * kSlots];  // RN(1/R0) where quot_ok(R0), NaN elsewhere
-    float theta0[3 * kSlots];
-    // angle gather table: for node p, six offsets (in floats) into the per-cell
-    // angle-force array, in the summation order of CalculateAngleForce
-    // (propagate.cu:124-178)
-    int32_t gather[kNodes * 6];
+// Mesh tables of a node in three 16-byte records and one of 8 bytes, so that a lane
+// gets its whole topology and rest state from four loads that depend on nothing but
+// the kernel arguments and are issued with the cell's own node data.
+struct alignas(16) MeshRec {
+    float f[3];
+    uint32_t w;
 };
+struct MeshDev {
+    MeshRec th[kSlots];   // rest angles; w: the three neighbours, 8 bits each
+    MeshRec r0[kSlots];   // rest lengths; w: angle gather offsets 0, 1 (16 bits each)
+    MeshRec ir0[kSlots];  // RN(1/R0) where quot_ok(R0), NaN elsewhere; w: gather offsets 2, 3
+    struct alignas(8) {
+        uint32_t w;       // gather offsets 4, 5
+        float sign;       // orientation of the friction normal (C180NN)
+    } gs[kSlots];
+    // The angle gather table: for a node, six offsets (in floats) into the per-cell
+    // angle-force array, in the summation order of CalculateAngleForce
+    // (propagate.cu:124-178).
+    // face[f]: the 7 entries of a C180_pentahexa row, 8 bits each
+    uint64_t face[kFacePad];
+    ThetaCoeffs theta;  // kTheta
+};
+__host__ __device__ inline int mesh_nn(uint32_t w, int k) { return (int)((w >> (8 * k)) & 0xffu); }
 
 struct Pool {
     float *X, *Y, *Z;

@@ -82,6 +82,17 @@ __device__ __forceinline__ float sqrt_cr(float x) {
     return tiny ? t * 0x1p-16f : t;
 }
 
+// sqrt_cr without its scaling of inputs below 2^-96: the same steps on the same
+// values for every other input.  A smaller input gives a result below 2^-40 (or
+// the exact 0), so quot_ok of the result is false; the callers then take sqrt_cr.
+__device__ __forceinline__ float sqrt_normal(float x) {
+    const float s = __builtin_amdgcn_sqrtf(x);
+    const float sm = __int_as_float(__float_as_int(s) - 1), sp = __int_as_float(__float_as_int(s) + 1);
+    const float rm = fmaf(-sm, s, x), rp = fmaf(-sp, s, x);
+    const float t = rm <= 0.f ? sm : s;
+    return rp > 0.f ? sp : t;
+}
+
 // RN(1/b) for quot_ok(b): the hardware reciprocal estimate and one Newton step
 // with an fma residual.  Equal to 1.0f / b for every float b with quot_ok(b)
 // (cs3d_check_div).
@@ -102,6 +113,17 @@ __device__ __forceinline__ float inv_rn(float b) {
     if (!quot_ok(b)) {
         slow_path();
         y = 1.0f / b;
+    }
+    return y;
+}
+
+// 1.0f / sqrt_cr(x2)
+__device__ __forceinline__ float inv_sqrt_rn(float x2) {
+    const float r = sqrt_normal(x2);
+    float y = rcp_rn(r);
+    if (!quot_ok(r)) {
+        slow_path();
+        y = 1.0f / sqrt_cr(x2);
     }
     return y;
 }
@@ -162,6 +184,7 @@ typedef __attribute__((address_space(4))) const cs3d_params* CParams;
 typedef __attribute__((address_space(4))) const SysMeta* CMeta;
 __device__ __forceinline__ CParams cparams(const cs3d_params* q) { return (CParams)q; }
 __device__ __forceinline__ CMeta cmeta(const SysMeta* q) { return (CMeta)q; }
+typedef __attribute__((address_space(4))) const ThetaCoeffs* CTheta;
 template <class T> __device__ __forceinline__ T cld(const T* q) {
     return *(__attribute__((address_space(4))) const T*)q;
 }
@@ -721,9 +744,14 @@ __device__ __forceinline__ void angle_quotients(float idk, float ra2, float ya2,
     }
 }
 
+// cs3d_acos as a call: for paths that hardly ever run, where inlining it would take
+// registers for its constants from the common path.
+__attribute__((noinline)) __device__ double acos_call(double x) { return cs3d_acos(x); }
+
 // Shared GetAngleForce pair (propagate.cu:26-60): Fa = F(a-v, b-v), Fb = F(b-v, a-v).
 // dot, |.|^2, c1 and theta are symmetric in the two arguments, so both come from
 // one evaluation with bit-identical values.
+template <bool kRare = false>
 __device__ __forceinline__ uint32_t angle_pair(float ax, float ay, float az, float bx, float by, float bz,
                                                float th0, float k, float* out) {
     const float idk = ax * bx + ay * by + az * bz;
@@ -732,7 +760,8 @@ __device__ __forceinline__ uint32_t angle_pair(float ax, float ay, float az, flo
     const float inner = (float)((double)(ra2 * rb2 - idk * idk) + 1e-3);
     const float c1 = -inv_rn(sqrt_cr(inner));
     const float den = sqrt_cr(ra2) * sqrt_cr(rb2);
-    const float theta = (float)cs3d_acos((double)idk / ((double)den + 1e-3));
+    const double x = (double)idk / ((double)den + 1e-3);
+    const float theta = (float)(kRare ? acos_call(x) : cs3d_acos(x));
     const float s = ((-k) * c1) * (theta - th0);
     float ca, cb;
     angle_quotients(idk, ra2, rcp_rn(ra2), rb2, rcp_rn(rb2), ca, cb);
@@ -743,37 +772,80 @@ __device__ __forceinline__ uint32_t angle_pair(float ax, float ay, float az, flo
     return ok ? 0u : (uint32_t)CS3D_SYS_ANGLE_NONFINITE;
 }
 
-// GetAngleForce pair (as angle_pair) with the squared lengths ra2, rb2 of the two
-// bond vectors and their square roots la, lb computed by the caller: the same
-// operations on the same vectors as in angle_pair (the springs of the node use
-// them too), so every bit is the same.  Its three quotients stay divisions here:
-// from reciprocals, with the division path kept for operands out of range, they
-// would keep more values live across the acos than the six-wave register budget
-// of k_con_dis holds.
-__device__ __forceinline__ uint32_t angle_pair_l(float ax, float ay, float az, float ra2, float la, float bx, float by,
-                                                 float bz, float rb2, float lb, float th0, float k, float* out) {
+// angle_pair for bonds with squared lengths ra2, rb2 in [2^-20, 2^20] (checked by the
+// caller), their roots la, lb (which the node's springs use too) and
+// the reciprocals ya2, yb2 = rcp_rn of them: the angle from cs3d_theta, the square
+// root without scaling and the quotients from reciprocals.  Returns whether every
+// operand was in the range of those steps (cs3d_theta's, c1's root in quot_ok's
+// range, |idk| at least 2^-40, |s| at most 2^70); then every bit equals
+// angle_pair's, and no component overflows: |b| <= 2^10 and |idk / ra2| <= 2^40
+// bound them below 2^121.
+__device__ __forceinline__ bool angle_pair_fast(float ax, float ay, float az, float ra2, float ya2, float la, float bx,
+                                                float by, float bz, float rb2, float yb2, float lb, float th0, float k,
+                                                CTheta c, float* out) {
     const float idk = ax * bx + ay * by + az * bz;
     const float inner = (float)((double)(ra2 * rb2 - idk * idk) + 1e-3);
-    const float c1 = -1.0f / sqrt_cr(inner);
+    const float root = sqrt_normal(inner);
+    const float c1 = -rcp_rn(root);
     const float den = la * lb;
-    const float theta = (float)cs3d_acos((double)idk / ((double)den + 1e-3));
+    float theta;
+    bool ok = cs3d_theta(idk, den, c, &theta);
     const float s = ((-k) * c1) * (theta - th0);
-    const float ca = idk / ra2, cb = idk / rb2;
+    const float ca = quot_rn(idk, ra2, ya2), cb = quot_rn(idk, rb2, yb2);
     out[0] = s * (bx - ca * ax); out[1] = s * (by - ca * ay); out[2] = s * (bz - ca * az);
     out[3] = s * (ax - cb * bx); out[4] = s * (ay - cb * by); out[5] = s * (az - cb * bz);
-    bool ok = isfinite(out[0]) && isfinite(out[1]) && isfinite(out[2]) && isfinite(out[3]) && isfinite(out[4]) &&
-              isfinite(out[5]);
-    return ok ? 0u : (uint32_t)CS3D_SYS_ANGLE_NONFINITE;
+    ok &= quot_ok(root);
+    ok &= fabsf(idk) >= 0x1p-40f;
+    ok &= fabsf(s) <= 0x1p70f;
+    return ok;
+}
+
+// The three angles of node tid, (n0,n1), (n1,n2), (n0,n2) (propagate.cu:26-60), to
+// out[18] from its bond vectors, squared lengths b2 and lengths bl: by
+// angle_pair_fast, and where an operand is out of its range again by angle_pair
+// (a loop that is not unrolled, on vectors read again from the positions in LDS:
+// it adds nothing to the registers live in the common path).
+__device__ __forceinline__ uint32_t node_angles(const float* bx, const float* by, const float* bz, const float* b2,
+                                                const float* bl, const MeshRec& mt, float k, const MeshDev* mesh,
+                                                const float* sx, const float* sy, const float* sz, int tid,
+                                                float* out) {
+    const float y2[3] = {rcp_rn(b2[0]), rcp_rn(b2[1]), rcp_rn(b2[2])};
+    // a NaN length leaves idk NaN in two of the angles, which their checks catch
+    bool in = fminf(fminf(b2[0], b2[1]), b2[2]) >= 0x1p-20f;
+    in &= fmaxf(fmaxf(b2[0], b2[1]), b2[2]) <= 0x1p20f;
+    uint32_t bad = in ? 0u : 7u;
+    CTheta c = (CTheta)&mesh->theta;
+    asm volatile("" : "+s"(c));  // read here, not kept across cells
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        const int a = q == 1 ? 1 : 0, b = q == 0 ? 1 : 2;
+        const bool ok = angle_pair_fast(bx[a], by[a], bz[a], b2[a], y2[a], bl[a], bx[b], by[b], bz[b], b2[b], y2[b],
+                                        bl[b], mt.f[q], k, c, out + 6 * q);
+        bad |= ok ? 0u : 1u << q;
+    }
+    uint32_t st = 0;
+    if (bad) {
+        slow_path();
+        const float X = lds_reread(sx, tid), Y = lds_reread(sy, tid), Z = lds_reread(sz, tid);
+        const float* th0 = reinterpret_cast<const float*>(mesh->th) + 4 * tid;
+#pragma unroll 1
+        for (int q = 0; q < 3; ++q) {
+            if (!(bad >> q & 1u)) continue;
+            const int a = mesh_nn(mt.w, q == 1 ? 1 : 0), b = mesh_nn(mt.w, q == 0 ? 1 : 2);
+            st |= angle_pair<true>(sx[a] - X, sy[a] - Y, sz[a] - Z, sx[b] - X, sy[b] - Y, sz[b] - Z,
+                                   th0[q], k, out + 6 * q);
+        }
+    }
+    return st;
 }
 
 // friction normal of node tid (propagate.cu:558-572), positions in LDS
-__device__ __forceinline__ void node_normal(const float* sx, const float* sy, const float* sz, const MeshDev* mesh,
-                                            int tid, int N1, int N2, int N3, float& nx, float& ny, float& nz) {
+__device__ __forceinline__ void node_normal(const float* sx, const float* sy, const float* sz, float sg, int N1, int N2,
+                                            int N3, float& nx, float& ny, float& nz) {
     const float Ax = sx[N2] - sx[N1], Ay = sy[N2] - sy[N1], Az = sz[N2] - sz[N1];
     const float Bx = sx[N3] - sx[N1], By = sy[N3] - sy[N1], Bz = sz[N3] - sz[N1];
     const float cx = Ay * Bz - Az * By, cy = Az * Bx - Ax * Bz, cz = Ax * By - Ay * Bx;
-    const float inv = inv_rn(sqrt_cr(cx * cx + cy * cy + cz * cz));
-    const float sg = (float)ldu(mesh->sign, lane_index());
+    const float inv = inv_sqrt_rn(cx * cx + cy * cy + cz * cz);
     nx = sg * (inv * cx);
     ny = sg * (inv * cy);
     nz = sg * (inv * cz);
@@ -823,87 +895,137 @@ __device__ __forceinline__ void pair_friction(const int32_t* lst, int tid, int n
     }
 }
 
-// Reference tests over the node's candidates in stored (= reference) order:
-// distance (ConForce skips R^2 >= ar^2, DisForce R^2 > ar^2, propagate.cu:421,641)
-// and the candidate rule per partner cell.  Accepted keys go to rec (for the
-// second friction pass); contact (CON) and friction (DIS) are summed as in
-// propagate.cu:411-440 and 633-653.  The loop is software-pipelined: while one
-// candidate is tested, the partner data of the next and the key of the one after
-// are already loading, so the key -> position dependence of each candidate does
-// not serialise the loop.
-// Returns the number accepted.
-// cand, rec: the cell's lists (uniform), entries at i * 192 + tid; sX .. sVZ,
-// sVR, sBB: node arrays, voxel ranges and boxes from the system's first slot
-// (uniform).
+// The contact pass works on pairs, not on nodes: the candidates of a cell's nodes
+// lie one after another in the cell's list (node order, each node's keys ascending,
+// so reference order), and lane t of the workgroup takes entry c0 + t of the list,
+// kSlots entries per round.  A node has 1 to 2 candidates on average but some node
+// of every wave has 5 to 7, so a loop over each node's own candidates ran 5 to 7
+// rounds with most lanes idle.  The lane applies the reference's tests to its pair
+// and leaves the force terms in LDS; each node then adds the terms of its accepted
+// pairs in list order, so every sum has the reference's order.
+// NCAND holds a node's candidate count in its low kCandBits bits and the index of
+// its first entry above them.
+struct PairLds {
+    float t[9][kSlots];    // attraction, repulsion and friction terms of the round's pairs
+    int32_t key[kSlots];   // their partner keys
+    uint64_t ok[4];        // accepted pairs of the round, one bit each (the fourth word stays 0)
+};
+
+// owner[j] = node whose entry c0 + j is, for this lane's entries in the round
+__device__ __forceinline__ void fill_owners(uint8_t* owner, int tid, int first, int nc, int c0) {
+    const int lo = max(first, c0), hi = min(first + nc, c0 + kSlots);
+    for (int j = lo; j < hi; ++j) owner[j - c0] = (uint8_t)tid;
+}
+
+// The reference's tests and force terms for one pair (node at X with velocity
+// vi and normal n, partner at px with velocity w): distance (ConForce skips
+// R^2 >= ar^2, DisForce R^2 > ar^2, propagate.cu:421,641), the candidate rule of
+// the partner's cell, the contact terms of propagate.cu:411-440 and the friction
+// term of 633-653.  A term that does not apply stays 0: the sums start at +0 and
+// never become -0, so adding it changes nothing.  Returns whether the pair is
+// accepted.
 template <bool CON, bool DIS>
-__device__ __forceinline__ int accept_forces(const int32_t* cand, int tid, int nc, int32_t* rec, float X, float Y,
-                                             float Z, const RuleCtx& R, const int32_t* __restrict__ sVR,
-                                             const float* __restrict__ sBB, float vix,
-                                             float viy, float viz, float nx, float ny, float nz, const PairConsts& k,
-                                             const float* __restrict__ sX, const float* __restrict__ sY,
-                                             const float* __restrict__ sZ, const float* __restrict__ sVX,
-                                             const float* __restrict__ sVY, const float* __restrict__ sVZ,
-                                             float& cfx, float& cfy, float& cfz, float& fdx, float& fdy,
-                                             float& fdz) {
-    int np = 0;
-    int lastb = -1;
-    bool lastok = false;
-    int vx = -1, vy = -1, vz = -1;  // the node's voxel (propagate.cu:360-372), found at first use
-    int key_n = nc > 0 ? ldu(cand, (uint32_t)tid) : 0;
-    int key_nn = nc > 1 ? ldu(cand, (uint32_t)(kSlots + tid)) : 0;
-    float pxn = 0.f, pyn = 0.f, pzn = 0.f, wxn = 0.f, wyn = 0.f, wzn = 0.f;
-    if (nc > 0) {
-        const uint32_t g = (uint32_t)key_n;
-        pxn = ldu(sX, g); pyn = ldu(sY, g); pzn = ldu(sZ, g);
-        if (DIS) { wxn = ldu(sVX, g); wyn = ldu(sVY, g); wzn = ldu(sVZ, g); }
+__device__ __forceinline__ bool pair_terms(int key, float X, float Y, float Z, float px, float py, float pz, float vix,
+                                           float viy, float viz, float wx, float wy, float wz, float nx, float ny,
+                                           float nz, const RuleCtx& R, const PairConsts& k,
+                                           const int32_t* __restrict__ sVR, const float* __restrict__ sBB, float* t) {
+    const float dX = X - px, dY = Y - py, dZ = Z - pz;
+    const float R2 = dX * dX + dY * dY + dZ * dZ;
+    if (R2 > k.ar2) return false;
+    // the node's voxel (propagate.cu:360-372)
+    const int vx = vox1(X, R.gx, R.DL, R.xd), vy = vox1(Y, R.gy, R.DL, R.yd), vz = vox1(Z, R.gz, R.DL, R.zd);
+    if (!rule_ok(sVR, sBB, (uint32_t)(key / kSlots), vx, vy, vz, X, Y, Z, R.ar2)) return false;
+    if (CON && R2 < k.ar2) {
+        const float Rl = sqrt_cr(R2);
+        if (Rl < k.ar) {
+            t[0] = k.ka * (k.ar - Rl) / Rl * dX;
+            t[1] = k.ka * (k.ar - Rl) / Rl * dY;
+            t[2] = k.ka * (k.ar - Rl) / Rl * dZ;
+        }
+        if (Rl <= k.rr) {
+            t[3] = k.kr * (k.rr - Rl) / Rl * dX;
+            t[4] = k.kr * (k.rr - Rl) / Rl * dY;
+            t[5] = k.kr * (k.rr - Rl) / Rl * dZ;
+        }
     }
-    for (int i = 0; i < nc; ++i) {
-        const int key = key_n;
-        const float px = pxn, py = pyn, pz = pzn;
-        const float wx = wxn, wy = wyn, wz = wzn;
-        key_n = key_nn;
-        if (i + 1 < nc) {
-            const uint32_t g = (uint32_t)key_n;
-            pxn = ldu(sX, g); pyn = ldu(sY, g); pzn = ldu(sZ, g);
-            if (DIS) { wxn = ldu(sVX, g); wyn = ldu(sVY, g); wzn = ldu(sVZ, g); }
+    if (DIS) {
+        const float ux = vix - wx, uy = viy - wy, uz = viz - wz;
+        const float d = ux * nx + uy * ny + uz * nz;
+        t[6] = k.gext * (ux - d * nx);
+        t[7] = k.gext * (uy - d * ny);
+        t[8] = k.gext * (uz - d * nz);
+    }
+    return true;
+}
+
+// All pairs of a cell (every lane of the workgroup calls it).  cand, rec: the
+// cell's candidate list (flat) and accepted-partner lists (entries at i * 192 +
+// tid), uniform; key0: cand[tid]; first, nc: this lane's entries; total: entries of the cell;
+// owner: filled for the first round and visible; sX .. sVZ, sVR, sBB: node arrays,
+// voxel ranges and boxes from the system's first slot (uniform); sx .. snz: the
+// cell's own positions, velocities and normals in LDS.  u is written only after a
+// barrier that ends its previous use.  Returns the number accepted.
+template <bool CON, bool DIS>
+__device__ __forceinline__ int pair_pass(const int32_t* cand, int key0, int32_t* rec, int tid, int first, int nc, int total,
+                                         PairLds& u, uint8_t* owner, const RuleCtx& R, const PairConsts& k,
+                                         const float* sx, const float* sy, const float* sz, const float* svx,
+                                         const float* svy, const float* svz, const float* snx, const float* sny,
+                                         const float* snz, const int32_t* __restrict__ sVR,
+                                         const float* __restrict__ sBB, const float* __restrict__ sX,
+                                         const float* __restrict__ sY, const float* __restrict__ sZ,
+                                         const float* __restrict__ sVX, const float* __restrict__ sVY,
+                                         const float* __restrict__ sVZ, float& cfx, float& cfy, float& cfz, float& fdx,
+                                         float& fdy, float& fdz) {
+    int np = 0;
+    for (int c0 = 0; c0 < total; c0 += kSlots) {
+        const bool has = c0 + tid < total;
+        const int key = c0 == 0 ? key0 : (has ? ldu(cand, (uint32_t)(c0 + tid)) : 0);
+        float t[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        bool ok = false;
+        if (has) {
+            const uint32_t g = (uint32_t)key;
+            const float px = ldu(sX, g), py = ldu(sY, g), pz = ldu(sZ, g);
+            float wx = 0.f, wy = 0.f, wz = 0.f;
+            if (DIS) { wx = ldu(sVX, g); wy = ldu(sVY, g); wz = ldu(sVZ, g); }
+            const int o = owner[tid];
+            ok = pair_terms<CON, DIS>(key, sx[o], sy[o], sz[o], px, py, pz, DIS ? svx[o] : 0.f, DIS ? svy[o] : 0.f,
+                                      DIS ? svz[o] : 0.f, wx, wy, wz, DIS ? snx[o] : 0.f, DIS ? sny[o] : 0.f,
+                                      DIS ? snz[o] : 0.f, R, k, sVR, sBB, t);
         }
-        if (i + 2 < nc) key_nn = ldu(cand, (uint32_t)((i + 2) * kSlots + tid));
-        const int b = key / kSlots;
-        const float dX = X - px, dY = Y - py, dZ = Z - pz;
-        const float R2 = dX * dX + dY * dY + dZ * dZ;
-        if (R2 > k.ar2) continue;
-        if (b != lastb) {
-            if (vx < 0) {
-                vx = vox1(X, R.gx, R.DL, R.xd);
-                vy = vox1(Y, R.gy, R.DL, R.yd);
-                vz = vox1(Z, R.gz, R.DL, R.zd);
+        __syncthreads();  // the previous use of u, and this round's owners, are done
+        const uint64_t m = __ballot(ok);
+        if ((tid & 63) == 0) u.ok[tid >> 6] = m;
+        if (tid == 0) u.ok[3] = 0;
+        if (ok) {
+            u.key[tid] = key;
+            if (CON) {
+#pragma unroll
+                for (int a = 0; a < 6; ++a) u.t[a][tid] = t[a];
             }
-            lastb = b;
-            lastok = rule_ok(sVR, sBB, (uint32_t)b, vx, vy, vz, X, Y, Z, R.ar2);
-        }
-        if (!lastok) continue;
-        stu(rec, (uint32_t)(np * kSlots + tid), key);
-        ++np;
-        if (CON && R2 < k.ar2) {
-            const float Rl = sqrt_cr(R2);
-            if (Rl < k.ar) {
-                cfx += k.ka * (k.ar - Rl) / Rl * dX;
-                cfy += k.ka * (k.ar - Rl) / Rl * dY;
-                cfz += k.ka * (k.ar - Rl) / Rl * dZ;
-            }
-            if (Rl <= k.rr) {
-                cfx += k.kr * (k.rr - Rl) / Rl * dX;
-                cfy += k.kr * (k.rr - Rl) / Rl * dY;
-                cfz += k.kr * (k.rr - Rl) / Rl * dZ;
+            if (DIS) {
+#pragma unroll
+                for (int a = 6; a < 9; ++a) u.t[a][tid] = t[a];
             }
         }
-        if (DIS) {
-            const float ux = vix - wx, uy = viy - wy, uz = viz - wz;
-            const float d = ux * nx + uy * ny + uz * nz;
-            const float tx = ux - d * nx, ty = uy - d * ny, tz = uz - d * nz;
-            fdx = fdx - k.gext * tx;
-            fdy = fdy - k.gext * ty;
-            fdz = fdz - k.gext * tz;
+        if (c0 + kSlots < total) fill_owners(owner, tid, first, nc, c0 + kSlots);
+        __syncthreads();
+        const int lo = max(first, c0), hi = min(first + nc, c0 + kSlots);
+        if (lo < hi) {  // this node's accepted pairs of the round, in list order (at most kPMax < 64 bits)
+            const int j0 = lo - c0, w = j0 >> 6, sh = j0 & 63;
+            uint64_t bits = u.ok[w] >> sh;
+            if (sh) bits |= u.ok[w + 1] << (64 - sh);
+            bits &= (1ull << (hi - lo)) - 1;
+            while (bits) {
+                const int j = j0 + __ffsll((unsigned long long)bits) - 1;
+                bits &= bits - 1;
+                stu(rec, (uint32_t)(np * kSlots + tid), u.key[j]);
+                ++np;
+                if (CON) {
+                    cfx += u.t[0][j]; cfy += u.t[1][j]; cfz += u.t[2][j];
+                    cfx += u.t[3][j]; cfy += u.t[4][j]; cfz += u.t[5][j];
+                }
+                if (DIS) { fdx = fdx - u.t[6][j]; fdy = fdy - u.t[7][j]; fdz = fdz - u.t[8][j]; }
+            }
         }
     }
     return np;
@@ -919,6 +1041,7 @@ template <int kLive>
 __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always) {
     __shared__ int32_t lst[kPMax][kSlots];
     __shared__ float part[3][6];
+    __shared__ int32_t wsum[3];
     __shared__ int32_t near;
     const int tid = threadIdx.x;
     const bool node = tid < kNodes;
@@ -987,15 +1110,27 @@ __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always)
             // is kept for later partial searches
             box_of_cell(X, Y, Z, node, part, p.SBOX + (int64_t)slot * 6);
         }
-        if (node) {
-            uint32_t st = 0;
-            const int nc = find_candidates(p, MC, P, c, X, Y, Z, lst, tid, st);
-            int32_t* cstore = p.CAND + (size_t)slot * kPMax * kSlots;
-            for (int i = 0; i < nc; ++i) stu(cstore, (uint32_t)(i * kSlots) + ln, lst[i][tid]);
-            stu(p.NCAND + cb, ln, nc);
-            if (reset) { stu(p.XBX + cb, ln, X); stu(p.XBY + cb, ln, Y); stu(p.XBZ + cb, ln, Z); }
-            if (st) flag(M, st);
+        uint32_t st = 0;
+        const int nc = node ? find_candidates(p, MC, P, c, X, Y, Z, lst, tid, st) : 0;
+        // the cell's candidates one after another in node order: an exclusive scan of
+        // the counts (shuffles within a wave, then the wave totals)
+        int first = nc;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int t = __shfl_up(first, o);
+            if ((tid & 63) >= o) first += t;
         }
+        if ((tid & 63) == 63) wsum[tid >> 6] = first;
+        __syncthreads();
+        first -= nc;
+        if (tid >= 64) first += wsum[0];
+        if (tid >= 128) first += wsum[1];
+        int32_t* cstore = p.CAND + (size_t)slot * kPMax * kSlots;
+        for (int i = 0; i < nc; ++i) stu(cstore, (uint32_t)(first + i), lst[i][tid]);
+        stu(p.NCAND + cb, ln, (first << kCandBits) | nc);  // the padding lanes hold the cell's total
+        if (node && reset) { stu(p.XBX + cb, ln, X); stu(p.XBY + cb, ln, Y); stu(p.XBZ + cb, ln, Z); }
+        if (st) flag(M, st);
+        __syncthreads();  // wsum is rewritten by the next cell
     }
 }
 
@@ -1007,32 +1142,39 @@ __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always)
 // partners), M_CON / M_INIT (FC, accepted partners), M_BONDED (spring +
 // pressure + angle -> FC), M_PAIRS (accepted partners only).
 // ------------------------------------------------------------------------------
-// 6 waves per SIMD (80 VGPRs): 2048 workgroups fit on the chip at once, so 2000
-// cells run in one round instead of 1.5.  Measured against 4 waves (100 VGPRs):
-// this kernel 28.0 instead of 29.5 us, and k_dis_post, which reads its outputs
-// next, 11.5 instead of 12.8 us, even with 18 values spilled to scratch then.  The
-// spills are gone: the angles come before the springs, so the spring sums are not
-// live across them; the node's position is read again from LDS after them; the
-// neighbour, rest-length, rest-angle and gather tables are read at a uniform base
-// plus the opaque lane offset where they are used, not through per-lane 64-bit
-// pointers kept across the cell loop.
-// kLive: walk Pool::LIVE (a multi-system step) instead of the range's slots
-template <int kLive>
+// 6 waves per SIMD (80 VGPRs, 20,064 B of LDS): 2048 workgroups fit on the chip at
+// once, so 2000 cells run in one round instead of 1.5 (at 4 waves the kernel took
+// 29.5 instead of 28.0 us, and k_dis_post, which reads its outputs next, 12.8 instead
+// of 11.5).  No spills at that budget: the node's position is read again from LDS
+// after the angles, the mesh tables are read at a uniform base plus the opaque lane
+// offset where they are used, LDS indices are the opaque lane as well, and what the
+// angles hardly ever need (angle_pair, the general acos) is a loop and a call.
+// What bounds it: vector-ALU issue and the latency of each cell's chain of loads and
+// barriers.  Pairs on lanes instead of a loop over each node's candidates, and the
+// angles' short arithmetic, took it from 1577 to 1127 vector instructions per wave
+// at 2000 cells (2017 to 1088 at 20,000): 22.9 to 21.0 us and 248 to 224 us a launch.
+// kLive: walk Pool::LIVE (a multi-system step) instead of the range's slots; kStep:
+// mode is M_STEP (the fused step has code of its own: as a run-time value the mode
+// took scalar registers, spilled, throughout the kernel)
+template <int kLive, bool kStep>
 __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_con_dis(Pool p, Range r, int32_t mode, const float* __restrict__ rX,
                                                  const float* __restrict__ rY, const float* __restrict__ rZ,
                                                  const float* __restrict__ rVX, const float* __restrict__ rVY,
                                                  const float* __restrict__ rVZ, const float* __restrict__ rBB) {
     __shared__ float sx[kSlots], sy[kSlots], sz[kSlots];
     __shared__ float svx[kSlots], svy[kSlots], svz[kSlots];
-    __shared__ struct {
+    __shared__ float snx[kSlots], sny[kSlots], snz[kSlots];  // friction normals
+    __shared__ uint8_t owner[kSlots];
+    __shared__ union {
         float angF[kNodes * 18];
+        PairLds pr;
     } u;
     const int tid = threadIdx.x;
     const bool node = tid < kNodes;
     const MeshDev* mesh = p.mesh;
-    const bool fused = mode == M_STEP;
-    const bool forces = mode != M_PAIRS;
-    const bool search = mode != M_BONDED;
+    const bool fused = kStep;
+    const bool forces = kStep || mode != M_PAIRS;
+    const bool search = kStep || mode != M_BONDED;
     // a multi-system step walks the compact list of live slots (k_live)
     const int nit = kLive ? *p.n_live : r.slot_hi - r.slot_lo;
     for (int it = xcd_block(); it < nit; it += gridDim.x) {
@@ -1041,10 +1183,19 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
         // overlaps the metadata reads
         const size_t cb = (size_t)slot * kSlots;  // the cell's first node (uniform)
         const uint32_t ln = lane_index();
+        const int lt = (int)ln;  // for LDS indices as well: nothing per lane is kept across cells
         const float X = ldu(rX + cb, ln), Y = ldu(rY + cb, ln), Z = ldu(rZ + cb, ln);
         float vX = 0.f, vY = 0.f, vZ = 0.f;
         if (fused) { vX = ldu(rVX + cb, ln); vY = ldu(rVY + cb, ln); vZ = ldu(rVZ + cb, ln); }
-        const int nc_pre = search ? ldu(p.NCAND + cb, ln) : 0;
+        const int32_t* cand = p.CAND + (size_t)slot * kPMax * kSlots;  // the cell's candidate list (uniform)
+        int ncf = 0, key0 = 0, total = 0;
+        if (search) {
+            ncf = ldu(p.NCAND + cb, ln);
+            key0 = ldu(cand, ln);  // the first round's keys (in the list's room also where it is shorter)
+            total = cld(p.NCAND + cb + kNodes) >> kCandBits;  // entries of the list, from a padding lane
+        }
+        const MeshRec mt = ldu(mesh->th, ln);
+        const float sg = fused ? ldu(mesh->gs, ln).sign : 0.f;
         const int s = __builtin_amdgcn_readfirstlane(sys_of(p, r, slot));
         if (s < 0) continue;
         SysMeta* M = p.meta + s;
@@ -1056,8 +1207,8 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
         const int c = slot - sbase;
         if (c >= MC->n) continue;
         const CParams P = cparams(p.prm + s);
-        sx[tid] = X; sy[tid] = Y; sz[tid] = Z;
-        if (fused) { svx[tid] = vX; svy[tid] = vY; svz[tid] = vZ; }
+        sx[lt] = X; sy[lt] = Y; sz[lt] = Z;
+        if (fused) { svx[lt] = vX; svy[lt] = vY; svz[lt] = vZ; }
         if (fused && tid == 0) {  // the search of this step has used the reset list
             p.RESET[slot] = 0;
             if (c == 0) M->n_reset = 0;
@@ -1068,41 +1219,33 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
         float FX = 0.f, FY = 0.f, FZ = 0.f;
         if (forces) {
             if (node && (isnan(X) || isnan(Y) || isnan(Z))) st |= CS3D_SYS_NAN;  // propagate.cu:241-248
+            if (fused && node) {
+                float nx, ny, nz;
+                node_normal(sx, sy, sz, sg, mesh_nn(mt.w, 0), mesh_nn(mt.w, 1), mesh_nn(mt.w, 2), nx, ny, nz);
+                snx[lt] = nx; sny[lt] = ny; snz[lt] = nz;
+            }
             if (node) {
                 // the node's three bonds: vectors, squared lengths and lengths, used by the
                 // node's own three angles (propagate.cu:26-60) and by the springs
                 // (propagate.cu:298-314), which compute the same quantities from the same
-                // vectors.  The angles write to LDS only, so evaluating them before the
-                // springs leaves every sum in its reference order.
+                // vectors.  The angles write to LDS only and are summed after the pressure, as
+                // in the reference.
                 float bx[3], by[3], bz[3], b2[3], bl[3];
-                const uint32_t lb = lane_index();
 #pragma unroll
                 for (int i = 0; i < 3; ++i) {
-                    const int N1 = ldu(mesh->nn, (uint32_t)(i * kSlots) + lb);
+                    const int N1 = mesh_nn(mt.w, i);
                     bx[i] = sx[N1] - X; by[i] = sy[N1] - Y; bz[i] = sz[N1] - Z;
                     b2[i] = bx[i] * bx[i] + by[i] * by[i] + bz[i] * bz[i];
-                    bl[i] = sqrt_cr(b2[i]);
-                }
-                if (angles) {  // each angle once (propagate.cu:26-60): (n0,n1), (n1,n2), (n0,n2)
-                    const float k = P->angle_k;
-                    const uint32_t lt = lane_index();
-#pragma unroll
-                    for (int q = 0; q < 3; ++q) {
-                        const int a = q == 1 ? 1 : 0;
-                        const int b = q == 0 ? 1 : 2;
-                        st |= angle_pair_l(bx[a], by[a], bz[a], b2[a], bl[a], bx[b], by[b], bz[b], b2[b], bl[b],
-                                           ldu(mesh->theta0, 3 * lt + q), k, u.angF + (tid * 3 + q) * 6);
-                    }
+                    bl[i] = sqrt_normal(b2[i]);
                 }
                 // ---- springs, propagate.cu:298-314
                 const float stiffness = cld(p.E + slot);
+                const MeshRec r0 = ldu(mesh->r0, lane_index()), ir0 = ldu(mesh->ir0, lane_index());
                 bool ok = true;
 #pragma unroll
                 for (int i = 0; i < 3; ++i) {
-                    const uint32_t li = (uint32_t)(i * kSlots) + lane_index();
                     float tx, ty, tz;
-                    ok &= spring_rcp(stiffness, bl[i], ldu(mesh->R0, li), ldu(mesh->R0inv, li), bx[i], by[i], bz[i],
-                                     tx, ty, tz);
+                    ok &= spring_rcp(stiffness, bl[i], r0.f[i], ir0.f[i], bx[i], by[i], bz[i], tx, ty, tz);
                     FX += tx;
                     FY += ty;
                     FZ += tz;
@@ -1113,20 +1256,40 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
 #pragma unroll
                     for (int i = 0; i < 3; ++i) {
                         float tx, ty, tz;
-                        spring_div(stiffness, bl[i], ldu(mesh->R0, (uint32_t)(i * kSlots) + lane_index()), bx[i], by[i],
-                                   bz[i], tx, ty, tz);
+                        spring_div(stiffness, sqrt_cr(b2[i]), r0.f[i], bx[i], by[i], bz[i], tx, ty, tz);
                         FX += tx;
                         FY += ty;
                         FZ += tz;
                     }
                 }
+                if (angles) {  // each angle once (propagate.cu:26-60): (n0,n1), (n1,n2), (n0,n2)
+                    st |= node_angles(bx, by, bz, b2, bl, mt, P->angle_k, mesh, sx, sy, sz, lt, u.angF + lt * 18);
+                }
             }
-            if (angles) __syncthreads();  // the angle forces of every node are in LDS
+        }
+        const int nc = ncf & ((1 << kCandBits) - 1), first = ncf >> kCandBits;
+        float fdx = 0.f, fdy = 0.f, fdz = 0.f;
+        if (search) fill_owners(owner, lt, first, nc, 0);
+        if (fused && node) {
+            const float vix = svx[lt], viy = svy[lt], viz = svz[lt];
+            const float gint = P->internal_damping;
+            const uint32_t nnw = ldu(mesh->th, lane_index()).w;
+            const int nn3[3] = {mesh_nn(nnw, 0), mesh_nn(nnw, 1), mesh_nn(nnw, 2)};
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {  // bond damping, propagate.cu:547-554
+                const int N = nn3[i];
+                fdx = fdx - gint * (vix - svx[N]);
+                fdy = fdy - gint * (viy - svy[N]);
+                fdz = fdz - gint * (viz - svz[N]);
+            }
+        }
+        __syncthreads();  // the angle forces, normals and owners of every node are in LDS
+        if (forces) {
             if (node) {
-                const float X = lds_reread(sx, tid), Y = lds_reread(sy, tid), Z = lds_reread(sz, tid);
+                const float X = lds_reread(sx, lt), Y = lds_reread(sy, lt), Z = lds_reread(sz, lt);
                 // ---- pressure, propagate.cu:318-330 (centre of mass from the last CenterOfMass)
                 const float rx = X - cld(p.CMX + slot), ry = Y - cld(p.CMY + slot), rz = Z - cld(p.CMZ + slot);
-                const float inv = inv_rn(sqrt_cr(rx * rx + ry * ry + rz * rz));
+                const float inv = inv_sqrt_rn(rx * rx + ry * ry + rz * rz);
                 const float g = 3.0f * cld(p.P + slot);
                 FX += g * (inv * rx);
                 FY += g * (inv * ry);
@@ -1134,7 +1297,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
             }
             // ---- angle forces gathered in the summation order of CalculateAngleForce (propagate.cu:81-181)
             if (angles && node) {
-                const float* a = u.angF + tid * 18;
+                const float* a = u.angF + lt * 18;
                 float ax = 0.f, ay = 0.f, az = 0.f;
 #pragma unroll
                 for (int q = 0; q < 3; ++q) {
@@ -1142,10 +1305,11 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
                     ay = ay - (a[q * 6 + 1] + a[q * 6 + 4]);
                     az = az - (a[q * 6 + 2] + a[q * 6 + 5]);
                 }
-                const uint32_t lg = lane_index() * 6;
+                const uint32_t lg = lane_index();
+                const uint32_t gt[3] = {ldu(mesh->r0, lg).w, ldu(mesh->ir0, lg).w, ldu(mesh->gs, lg).w};
 #pragma unroll
                 for (int q = 0; q < 6; ++q) {
-                    const float* f = u.angF + ldu(mesh->gather, lg + q);
+                    const float* f = u.angF + ((gt[q >> 1] >> (16 * (q & 1))) & 0xffffu);
                     ax = ax + f[0];
                     ay = ay + f[1];
                     az = az + f[2];
@@ -1153,10 +1317,9 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
                 FX += ax; FY += ay; FZ += az;
             }
         }
-        if (search && node) {
-            const float X = lds_reread(sx, tid), Y = lds_reread(sy, tid), Z = lds_reread(sz, tid);
-            const int nc = nc_pre;
-            const int32_t* cand = p.CAND + (size_t)slot * kPMax * kSlots;  // the cell's lists (uniform)
+        float cfx = 0.f, cfy = 0.f, cfz = 0.f;
+        int np = 0;
+        if (total > 0) {
             const size_t sb = (size_t)sbase * kSlots;                      // the system's first node
             const RuleCtx R = rule_ctx(MC, P);
             PairConsts k;
@@ -1166,40 +1329,29 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
             k.ka = -P->attraction_strength * P->youngs_mod;
             k.kr = +P->repulsion_strength * P->youngs_mod;
             k.gext = P->viscotic_damping;
-            float cfx = 0.f, cfy = 0.f, cfz = 0.f;
-            float fdx = 0.f, fdy = 0.f, fdz = 0.f;
             int32_t* rec = p.PAIRS + (size_t)slot * kPMax * kSlots;
             const int32_t* sVR = p.VRANGE + (size_t)sbase * 6;
             const float* sBB = rBB + (size_t)sbase * 6;
-            int np;
+            if (fused)
+                np = pair_pass<true, true>(cand, key0, rec, lt, first, nc, total, u.pr, owner, R, k, sx, sy, sz, svx, svy, svz,
+                                           snx, sny, snz, sVR, sBB, rX + sb, rY + sb, rZ + sb, rVX + sb, rVY + sb,
+                                           rVZ + sb, cfx, cfy, cfz, fdx, fdy, fdz);
+            else if (forces)
+                np = pair_pass<true, false>(cand, key0, rec, lt, first, nc, total, u.pr, owner, R, k, sx, sy, sz, svx, svy,
+                                            svz, snx, sny, snz, sVR, sBB, rX + sb, rY + sb, rZ + sb, rVX + sb,
+                                            rVY + sb, rVZ + sb, cfx, cfy, cfz, fdx, fdy, fdz);
+            else
+                np = pair_pass<false, false>(cand, key0, rec, lt, first, nc, total, u.pr, owner, R, k, sx, sy, sz, svx, svy,
+                                             svz, snx, sny, snz, sVR, sBB, rX + sb, rY + sb, rZ + sb, rVX + sb,
+                                             rVY + sb, rVZ + sb, cfx, cfy, cfz, fdx, fdy, fdz);
+        }
+        if (search && node) {
+            const float X = lds_reread(sx, lt), Y = lds_reread(sy, lt), Z = lds_reread(sz, lt);
             if (fused) {
-                const float vix = svx[tid], viy = svy[tid], viz = svz[tid];
-                const float gint = P->internal_damping;
-                int nn3[3];
-#pragma unroll
-                for (int i = 0; i < 3; ++i) {  // bond damping, propagate.cu:547-554
-                    nn3[i] = ldu(mesh->nn, (uint32_t)(i * kSlots) + lane_index());
-                    const int N = nn3[i];
-                    fdx = fdx - gint * (vix - svx[N]);
-                    fdy = fdy - gint * (viy - svy[N]);
-                    fdz = fdz - gint * (viz - svz[N]);
-                }
-                float nx, ny, nz;
-                node_normal(sx, sy, sz, mesh, tid, nn3[0], nn3[1], nn3[2], nx, ny, nz);
-                np = accept_forces<true, true>(cand, (int)ln, nc, rec, X, Y, Z, R, sVR, sBB, vix, viy, viz, nx, ny, nz, k,
-                                               rX + sb, rY + sb, rZ + sb, rVX + sb, rVY + sb, rVZ + sb, cfx, cfy,
-                                               cfz, fdx, fdy, fdz);
+                const float vix = svx[lt], viy = svy[lt], viz = svz[lt];
                 fdx = fdx - P->gamma_visc * vix;  // drag, propagate.cu:658
                 fdy = fdy - P->gamma_visc * viy;
                 fdz = fdz - P->gamma_visc * viz;
-            } else if (forces) {
-                np = accept_forces<true, false>(cand, (int)ln, nc, rec, X, Y, Z, R, sVR, sBB, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, k,
-                                                rX + sb, rY + sb, rZ + sb, rVX + sb, rVY + sb, rVZ + sb, cfx, cfy,
-                                                cfz, fdx, fdy, fdz);
-            } else {
-                np = accept_forces<false, false>(cand, (int)ln, nc, rec, X, Y, Z, R, sVR, sBB, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f,
-                                                 k, rX + sb, rY + sb, rZ + sb, rVX + sb, rVY + sb, rVZ + sb, cfx, cfy,
-                                                 cfz, fdx, fdy, fdz);
             }
             stu(pool_late()->NPAIR + cb, ln, np);
             if (forces) {
@@ -1223,13 +1375,13 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
                 float frx = 0.f, fry = 0.f, frz = 0.f;
                 if (P->add_rands) {  // CalculateRanForce for this step (propagate.cu:667-676)
                     float zr[3];
-                    noise3(P->noise_seed, (uint32_t)(c * kSlots + tid), MC->step + 1, zr);
+                    noise3(P->noise_seed, (uint32_t)(c * kSlots + lt), MC->step + 1, zr);
                     const float sc = P->rand_scale_factor;
                     frx = sc * zr[0]; fry = sc * zr[1]; frz = sc * zr[2];
                     const CPool q = pool_late();
                     stu(q->FRX + cb, ln, frx); stu(q->FRY + cb, ln, fry); stu(q->FRZ + cb, ln, frz);
                 }
-                const float vix = svx[tid], viy = svy[tid], viz = svz[tid];
+                const float vix = svx[lt], viy = svy[lt], viz = svz[lt];
                 // VelocityUpdateA (propagate.cu:721-723) then VelocityUpdateB (:732-734)
                 float vx = (float)((double)vix + kick_a(dt * FX + rdt * frx, m, MC));
                 float vy = (float)((double)viy + kick_a(dt * FY + rdt * fry, m, MC));
@@ -1270,10 +1422,10 @@ __global__ __launch_bounds__(192) void k_bonded(Pool p, Range r) {
     if (node) {
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-            nb[i] = mesh->nn[i * kSlots + tid];
-            r0[i] = mesh->R0[i * kSlots + tid];
-            ir0[i] = mesh->R0inv[i * kSlots + tid];
-            if (ANGLES) th[i] = mesh->theta0[3 * tid + i];
+            nb[i] = mesh_nn(mesh->th[tid].w, i);
+            r0[i] = mesh->r0[tid].f[i];
+            ir0[i] = mesh->ir0[tid].f[i];
+            if (ANGLES) th[i] = mesh->th[tid].f[i];
         }
     }
     int slot = r.slot_lo + blockIdx.x;
@@ -1344,7 +1496,7 @@ __global__ __launch_bounds__(192) void k_bonded(Pool p, Range r) {
                     }
                 }
                 const float rx = X - p.CMX[slot], ry = Y - p.CMY[slot], rz = Z - p.CMZ[slot];
-                const float inv = inv_rn(sqrt_cr(rx * rx + ry * ry + rz * rz));
+                const float inv = inv_sqrt_rn(rx * rx + ry * ry + rz * rz);
                 const float g = 3.0f * p.P[slot];
                 FX += g * (inv * rx);
                 FY += g * (inv * ry);
@@ -1358,10 +1510,10 @@ __global__ __launch_bounds__(192) void k_bonded(Pool p, Range r) {
                         ay = ay - (a[q * 6 + 1] + a[q * 6 + 4]);
                         az = az - (a[q * 6 + 2] + a[q * 6 + 5]);
                     }
-                    const int32_t* gt = mesh->gather + tid * 6;
+                    const uint32_t gt[3] = {mesh->r0[tid].w, mesh->ir0[tid].w, mesh->gs[tid].w};
 #pragma unroll
                     for (int q = 0; q < 6; ++q) {
-                        const float* f = angF + gt[q];
+                        const float* f = angF + ((gt[q >> 1] >> (16 * (q & 1))) & 0xffffu);
                         ax = ax + f[0];
                         ay = ay + f[1];
                         az = az + f[2];
@@ -1413,6 +1565,8 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
         float vX = 0.f, vY = 0.f, vZ = 0.f;
         if (do_dis) { vX = ldu(rVX + cb, ln); vY = ldu(rVY + cb, ln); vZ = ldu(rVZ + cb, ln); }
         const int np = (do_dis && node) ? ldu(p.NPAIR + cb, ln) : 0;
+        const uint32_t nnw = do_dis ? ldu(mesh->th, ln).w : 0u;
+        const float sg = do_dis ? ldu(mesh->gs, ln).sign : 0.f;
         float fcX = 0.f, fcY = 0.f, fcZ = 0.f, xbX = 0.f, xbY = 0.f, xbZ = 0.f;
         if (fused && do_dis && node) {
             fcX = ldu(p.FCX + cb, ln); fcY = ldu(p.FCY + cb, ln); fcZ = ldu(p.FCZ + cb, ln);
@@ -1439,17 +1593,16 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
             float fx = 0.f, fy = 0.f, fz = 0.f;
             const float vix = svx[tid], viy = svy[tid], viz = svz[tid];
             const float gint = P->internal_damping;
-            int nn3[3];
+            const int nn3[3] = {mesh_nn(nnw, 0), mesh_nn(nnw, 1), mesh_nn(nnw, 2)};
 #pragma unroll
             for (int i = 0; i < 3; ++i) {  // bond damping, propagate.cu:547-554
-                const int N = mesh->nn[i * kSlots + tid];
-                nn3[i] = N;
+                const int N = nn3[i];
                 fx = fx - gint * (vix - svx[N]);
                 fy = fy - gint * (viy - svy[N]);
                 fz = fz - gint * (viz - svz[N]);
             }
             float nx, ny, nz;
-            node_normal(sx, sy, sz, mesh, tid, nn3[0], nn3[1], nn3[2], nx, ny, nz);
+            node_normal(sx, sy, sz, sg, nn3[0], nn3[1], nn3[2], nx, ny, nz);
             PairConsts k;
             k.ar = P->attraction_range;
             k.ar2 = k.ar * k.ar;
@@ -1570,13 +1723,18 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
             const bool sph = P->check_sphericity != 0;
             float totvol = 0.f, faceArea = 0.f;
             if (tid < CS3D_FACES) {  // volume.cu:37-119
-                const int32_t* rr = mesh->faces + 7 * tid;
+                const uint64_t fw = mesh->face[tid];
+                int rr[7];
+#pragma unroll
+                for (int i = 0; i < 7; ++i) rr[i] = (int)((fw >> (8 * i)) & 0xffu);
                 float avX = 0.0f, avY = 0.0f, avZ = 0.0f;
+#pragma unroll
                 for (int i = 0; i < 5; ++i) { avX += sx[rr[i]]; avY += sy[rr[i]]; avZ += sz[rr[i]]; }
                 float fac = 0.166666667f;
                 if (tid < 12) fac = 0.2f;
                 else { avX += sx[rr[5]]; avY += sy[rr[5]]; avZ += sz[rr[5]]; }
                 avX *= fac; avY *= fac; avZ *= fac;
+#pragma unroll
                 for (int i = 0; i < 6; ++i) {
                     const int a = rr[i], b = rr[i + 1];
                     const float n1 = (sy[b] * avZ - avY * sz[b]) * sx[a];
@@ -2493,12 +2651,13 @@ void launch_con(const Pool& p, const Range& r, int mode, bool use_va, hipStream_
     const float* vx = use_va ? p.VAX : p.VX;
     const float* vy = use_va ? p.VAY : p.VY;
     const float* vz = use_va ? p.VAZ : p.VZ;
-    if (r.live)
-        launch(k_con_dis<1>, dim3(grid_cells(r, p.wg_per_cu)), dim3(192), st, p, r, mode, p.X, p.Y, p.Z, vx, vy, vz,
-                               p.BBOX);
+    const dim3 grid(grid_cells(r, p.wg_per_cu)), block(192);
+    if (mode != M_STEP)  // one system
+        launch(k_con_dis<0, false>, grid, block, st, p, r, mode, p.X, p.Y, p.Z, vx, vy, vz, p.BBOX);
+    else if (r.live)
+        launch(k_con_dis<1, true>, grid, block, st, p, r, mode, p.X, p.Y, p.Z, vx, vy, vz, p.BBOX);
     else
-        launch(k_con_dis<0>, dim3(grid_cells(r, p.wg_per_cu)), dim3(192), st, p, r, mode, p.X, p.Y, p.Z, vx, vy, vz,
-                               p.BBOX);
+        launch(k_con_dis<0, true>, grid, block, st, p, r, mode, p.X, p.Y, p.Z, vx, vy, vz, p.BBOX);
 }
 // angles: 0 = systems without bending, 1 = with, -1 = both launches
 void launch_bonded(const Pool& p, const Range& r, int angles, hipStream_t st) {

@@ -1,0 +1,91 @@
+"""The contact pass of k_con_dis where its work lists can go wrong, bit for bit
+against the oracle through the C ABI: no candidates at all, one round (at most 192
+pairs per cell), several rounds, nodes whose candidates straddle a round or a
+64-lane word, and lists near the 40-entry limit; and the bonds and angles at the
+edges of the short arithmetic (rest shape, crushed, stretched, bonds at and below
+its range)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(oracle_mesh, X, Y, Z, n, skin, steps, seed, grow=0.0):
+    from cellsim3d_amd import abi as A
+    from cellsim3d_amd import configs, engine
+    from oracle import oracle as O
+    p = configs.base_params(seed)
+    p.growth_rate = grow
+    p.division_vol = 1e30
+    p.pair_skin = skin
+    p.voxel_capacity = 64
+    rng = np.random.default_rng(seed)
+    V = [np.zeros((n, 192), np.float32) for _ in range(3)]
+    for v in V:
+        v[:, :180] = rng.normal(0, 0.3, (n, 180)).astype(np.float32)
+    V = [v.reshape(-1) for v in V]
+    sim = O.Sim(p, oracle_mesh, X, Y, Z, n, max_cells=n, budget=1 << 14)
+    for f, v in zip((A.F_VX, A.F_VY, A.F_VZ), V):
+        sim.set(f, v)
+    sim.init()
+    with engine.Context(oracle_mesh, capacity_cells=n, voxel_budget=1 << 21) as ctx:
+        s = ctx.add_system(p, X, Y, Z, n, max_cells=n, voxels=1 << 14, V=V)
+        counts = s.get(A.F_CANDCOUNT).reshape(n, 192)
+        assert not counts[:, 180:].any()
+        fields = [A.F_FCX, A.F_FCY, A.F_FCZ, A.F_FDX, A.F_FDY, A.F_FDZ, A.F_X, A.F_Y, A.F_Z, A.F_VX, A.F_VY, A.F_VZ]
+        for k in range(2):
+            for f in fields:
+                a, b = s.get(f)[:n * 192], sim.get(f)[:n * 192]
+                assert np.array_equal(a, b, equal_nan=True), (k, f, int((a != b).sum()))
+            if k == 0:
+                # the partner lists: ascending keys of nodes within attraction_range
+                pc = s.get(A.F_PAIRCOUNT).reshape(n, 192)
+                keys = s.get(A.F_PAIRS).reshape(n, 40, 192)
+                P = np.stack([a.reshape(-1) for a in (X, Y, Z)]).astype(np.float64)
+                for c in range(n):
+                    for i in np.flatnonzero(pc[c]):
+                        g = keys[c, :pc[c, i], i]
+                        assert np.all(np.diff(g) > 0)
+                        d = np.sqrt(((P[:, g] - P[:, c * 192 + i][:, None]) ** 2).sum(0))
+                        assert np.all(d < p.attraction_range + 1e-5)
+                sim.step(steps)
+                s.step(steps)
+                ctx.sync()
+        status = s.info()[2]
+    return counts, status
+
+
+# spacing in x, cells, skin -> rounds of 192 pairs in the fullest cell
+@pytest.mark.parametrize("spacing,n,skin,rounds", [(4.0, 3, 0.05, (0, 0)), (2.1, 2, 0.05, (1, 1)), (1.9, 5, 0.15, (2, 4)),
+                                                   (1.8, 7, 0.2, (4, 9)), (1.75, 9, 0.22, (6, 38))])
+def test_pair_rounds_match_oracle(oracle_mesh, spacing, n, skin, rounds):
+    from cellsim3d_amd import abi as A
+    from cellsim3d_amd import configs
+    print("pairs: spacing %g, %d cells, skin %g" % (spacing, n, skin), flush=True)
+    centres = [(spacing * (i % 3), spacing * (i // 3), 0.3 * (i % 2)) for i in range(n)]
+    X, Y, Z = configs.place(configs.unit_mesh(), centres, 0.02, np.random.default_rng(n))
+    counts, status = _run(oracle_mesh, X, Y, Z, n, skin, 4, 3 + n)
+    assert not status & A.SYS_FATAL_MASK
+    full = -(-int(counts.sum(1).max()) // 192)
+    assert rounds[0] <= full <= rounds[1], full
+
+
+# a cell scaled per axis, then some nodes drawn to their first neighbour, to the given
+# distance (0: the shape as it is).  (Scaling a whole cell far down would put its 180
+# nodes into one search bin of 32 entries, which the engine refuses.)
+@pytest.mark.parametrize("scale,bond", [((1.0, 1.0, 1.0), 0.0), ((1.0, 1.0, 0.02), 0.0), ((1.0, 0.3, 3.0), 0.0),
+                                        ((1.0, 1.0, 1.0), 2e-3), ((1.0, 1.0, 1.0), 1e-4), ((1.0, 1.0, 1.0), 1e-6)])
+def test_deformed_cells_match_oracle(oracle_mesh, scale, bond):
+    from cellsim3d_amd import configs, mesh as M
+    print("bonds and angles: scale %s, bond %g" % (scale, bond), flush=True)
+    m = configs.unit_mesh()
+    base = M.centred(m).astype(np.float32)
+    A = [np.zeros((2, 192), np.float32) for _ in range(3)]
+    for k in range(3):
+        A[k][0, :180] = base[:, k] * np.float32(scale[k])
+        A[k][1, :180] = base[:, k] + np.float32(5.0 if k == 0 else 0.0)
+        if bond:
+            for i in range(0, 180, 20):
+                A[k][0, i] = A[k][0, m["nn"][i, 0]] + np.float32(bond)
+    # one step: the strongly deformed ones move far, and both sides with them
+    _run(oracle_mesh, A[0].reshape(-1), A[1].reshape(-1), A[2].reshape(-1), 2, 0.05, 1, 7)
