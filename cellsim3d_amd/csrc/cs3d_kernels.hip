@@ -696,17 +696,23 @@ struct RuleCtx {
     int xd, yd, zd;
 };
 
+struct CellBox {  // voxel range and box of a cell
+    int2 r01, r23, r45;
+    float2 c01, c23, c45;
+};
 // sVR, sBB: voxel ranges and boxes from the system's first cell (uniform); b: the
-// partner cell's local index
-__device__ __forceinline__ bool rule_ok(const int32_t* __restrict__ sVR, const float* __restrict__ sBB, uint32_t b,
-                                        int vx, int vy, int vz, float X, float Y, float Z, float ar2) {
-    // all twelve words are loaded before any test (8-byte aligned pairs)
+// cell's local index
+__device__ __forceinline__ CellBox load_cell_box(const int32_t* __restrict__ sVR, const float* __restrict__ sBB,
+                                                 uint32_t b) {
     const int2* vr = reinterpret_cast<const int2*>(sVR);
     const float2* bb = reinterpret_cast<const float2*>(sBB);
-    const int2 r01 = ldu(vr, 3 * b), r23 = ldu(vr, 3 * b + 1), r45 = ldu(vr, 3 * b + 2);
-    const float2 c01 = ldu(bb, 3 * b), c23 = ldu(bb, 3 * b + 1), c45 = ldu(bb, 3 * b + 2);
-    const bool inlist = (r01.x <= vx) & (vx <= r01.y) & (r23.x <= vy) & (vy <= r23.y) & (r45.x <= vz) & (vz <= r45.y);
-    const float b0 = c01.x, b1 = c01.y, b2 = c23.x, b3 = c23.y, b4 = c45.x, b5 = c45.y;
+    return CellBox{ldu(vr, 3 * b), ldu(vr, 3 * b + 1), ldu(vr, 3 * b + 2),
+                   ldu(bb, 3 * b), ldu(bb, 3 * b + 1), ldu(bb, 3 * b + 2)};
+}
+__device__ __forceinline__ bool rule_ok(const CellBox& k, int vx, int vy, int vz, float X, float Y, float Z, float ar2) {
+    const bool inlist = (k.r01.x <= vx) & (vx <= k.r01.y) & (k.r23.x <= vy) & (vy <= k.r23.y) & (k.r45.x <= vz) &
+                        (vz <= k.r45.y);
+    const float b0 = k.c01.x, b1 = k.c01.y, b2 = k.c23.x, b3 = k.c23.y, b4 = k.c45.x, b5 = k.c45.y;
     float qx = (float)(X - b1 > 0.0f) * (X - b1);
     qx += (float)(b0 - X > 0.0f) * (b0 - X);
     float qy = (float)(Y - b3 > 0.0f) * (Y - b3);
@@ -917,24 +923,45 @@ __device__ __forceinline__ void fill_owners(uint8_t* owner, int tid, int first, 
     for (int j = lo; j < hi; ++j) owner[j - c0] = (uint8_t)tid;
 }
 
+// What a pair needs of its partner, all of it known from the key: loaded together
+// (one memory round trip), before the lane needs any of it.
+struct PairIn {
+    float x, y, z, wx, wy, wz;  // position and velocity
+    CellBox box;                // voxel range and box of its cell
+};
+// sX .. sVZ, sVR, sBB: node arrays, voxel ranges and boxes from the system's first
+// slot (uniform)
+struct SysArrays {
+    const float *X, *Y, *Z, *VX, *VY, *VZ;
+    const int32_t* VR;
+    const float* BB;
+};
+template <bool DIS> __device__ __forceinline__ PairIn load_pair(int key, const SysArrays& a) {
+    const uint32_t g = (uint32_t)key;
+    PairIn in;
+    in.x = ldu(a.X, g); in.y = ldu(a.Y, g); in.z = ldu(a.Z, g);
+    if (DIS) { in.wx = ldu(a.VX, g); in.wy = ldu(a.VY, g); in.wz = ldu(a.VZ, g); }
+    in.box = load_cell_box(a.VR, a.BB, g / kSlots);
+    return in;
+}
+
 // The reference's tests and force terms for one pair (node at X with velocity
-// vi and normal n, partner at px with velocity w): distance (ConForce skips
+// vi and normal n, partner in): distance (ConForce skips
 // R^2 >= ar^2, DisForce R^2 > ar^2, propagate.cu:421,641), the candidate rule of
 // the partner's cell, the contact terms of propagate.cu:411-440 and the friction
 // term of 633-653.  A term that does not apply stays 0: the sums start at +0 and
 // never become -0, so adding it changes nothing.  Returns whether the pair is
 // accepted.
 template <bool CON, bool DIS>
-__device__ __forceinline__ bool pair_terms(int key, float X, float Y, float Z, float px, float py, float pz, float vix,
-                                           float viy, float viz, float wx, float wy, float wz, float nx, float ny,
-                                           float nz, const RuleCtx& R, const PairConsts& k,
-                                           const int32_t* __restrict__ sVR, const float* __restrict__ sBB, float* t) {
-    const float dX = X - px, dY = Y - py, dZ = Z - pz;
+__device__ __forceinline__ bool pair_terms(const PairIn& in, float X, float Y, float Z, float vix, float viy, float viz,
+                                           float nx, float ny, float nz, const RuleCtx& R, const PairConsts& k,
+                                           float* t) {
+    const float dX = X - in.x, dY = Y - in.y, dZ = Z - in.z;
     const float R2 = dX * dX + dY * dY + dZ * dZ;
     if (R2 > k.ar2) return false;
     // the node's voxel (propagate.cu:360-372)
     const int vx = vox1(X, R.gx, R.DL, R.xd), vy = vox1(Y, R.gy, R.DL, R.yd), vz = vox1(Z, R.gz, R.DL, R.zd);
-    if (!rule_ok(sVR, sBB, (uint32_t)(key / kSlots), vx, vy, vz, X, Y, Z, R.ar2)) return false;
+    if (!rule_ok(in.box, vx, vy, vz, X, Y, Z, R.ar2)) return false;
     if (CON && R2 < k.ar2) {
         const float Rl = sqrt_cr(R2);
         if (Rl < k.ar) {
@@ -949,7 +976,7 @@ __device__ __forceinline__ bool pair_terms(int key, float X, float Y, float Z, f
         }
     }
     if (DIS) {
-        const float ux = vix - wx, uy = viy - wy, uz = viz - wz;
+        const float ux = vix - in.wx, uy = viy - in.wy, uz = viz - in.wz;
         const float d = ux * nx + uy * ny + uz * nz;
         t[6] = k.gext * (ux - d * nx);
         t[7] = k.gext * (uy - d * ny);
@@ -960,37 +987,27 @@ __device__ __forceinline__ bool pair_terms(int key, float X, float Y, float Z, f
 
 // All pairs of a cell (every lane of the workgroup calls it).  cand, rec: the
 // cell's candidate list (flat) and accepted-partner lists (entries at i * 192 +
-// tid), uniform; key0: cand[tid]; first, nc: this lane's entries; total: entries of the cell;
-// owner: filled for the first round and visible; sX .. sVZ, sVR, sBB: node arrays,
-// voxel ranges and boxes from the system's first slot (uniform); sx .. snz: the
+// tid), uniform; key, in: the lane's pair of the first round (where tid < total);
+// first, nc: this lane's entries; total: entries of the cell;
+// owner: filled for the first round and visible; sx .. snz: the
 // cell's own positions, velocities and normals in LDS.  u is written only after a
 // barrier that ends its previous use.  Returns the number accepted.
 template <bool CON, bool DIS>
-__device__ __forceinline__ int pair_pass(const int32_t* cand, int key0, int32_t* rec, int tid, int first, int nc, int total,
-                                         PairLds& u, uint8_t* owner, const RuleCtx& R, const PairConsts& k,
-                                         const float* sx, const float* sy, const float* sz, const float* svx,
-                                         const float* svy, const float* svz, const float* snx, const float* sny,
-                                         const float* snz, const int32_t* __restrict__ sVR,
-                                         const float* __restrict__ sBB, const float* __restrict__ sX,
-                                         const float* __restrict__ sY, const float* __restrict__ sZ,
-                                         const float* __restrict__ sVX, const float* __restrict__ sVY,
-                                         const float* __restrict__ sVZ, float& cfx, float& cfy, float& cfz, float& fdx,
-                                         float& fdy, float& fdz) {
+__device__ __forceinline__ int pair_pass(const int32_t* cand, int key, PairIn in, int32_t* rec, int tid, int first,
+                                         int nc, int total, PairLds& u, uint8_t* owner, const RuleCtx& R,
+                                         const PairConsts& k, const float* sx, const float* sy, const float* sz,
+                                         const float* svx, const float* svy, const float* svz, const float* snx,
+                                         const float* sny, const float* snz, const SysArrays& arr, float& cfx,
+                                         float& cfy, float& cfz, float& fdx, float& fdy, float& fdz) {
     int np = 0;
     for (int c0 = 0; c0 < total; c0 += kSlots) {
-        const bool has = c0 + tid < total;
-        const int key = c0 == 0 ? key0 : (has ? ldu(cand, (uint32_t)(c0 + tid)) : 0);
         float t[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         bool ok = false;
-        if (has) {
-            const uint32_t g = (uint32_t)key;
-            const float px = ldu(sX, g), py = ldu(sY, g), pz = ldu(sZ, g);
-            float wx = 0.f, wy = 0.f, wz = 0.f;
-            if (DIS) { wx = ldu(sVX, g); wy = ldu(sVY, g); wz = ldu(sVZ, g); }
+        if (c0 + tid < total) {
             const int o = owner[tid];
-            ok = pair_terms<CON, DIS>(key, sx[o], sy[o], sz[o], px, py, pz, DIS ? svx[o] : 0.f, DIS ? svy[o] : 0.f,
-                                      DIS ? svz[o] : 0.f, wx, wy, wz, DIS ? snx[o] : 0.f, DIS ? sny[o] : 0.f,
-                                      DIS ? snz[o] : 0.f, R, k, sVR, sBB, t);
+            ok = pair_terms<CON, DIS>(in, sx[o], sy[o], sz[o], DIS ? svx[o] : 0.f, DIS ? svy[o] : 0.f,
+                                      DIS ? svz[o] : 0.f, DIS ? snx[o] : 0.f, DIS ? sny[o] : 0.f, DIS ? snz[o] : 0.f, R,
+                                      k, t);
         }
         __syncthreads();  // the previous use of u, and this round's owners, are done
         const uint64_t m = __ballot(ok);
@@ -1007,7 +1024,13 @@ __device__ __forceinline__ int pair_pass(const int32_t* cand, int key0, int32_t*
                 for (int a = 6; a < 9; ++a) u.t[a][tid] = t[a];
             }
         }
-        if (c0 + kSlots < total) fill_owners(owner, tid, first, nc, c0 + kSlots);
+        if (c0 + kSlots < total) {  // the next round's pair
+            fill_owners(owner, tid, first, nc, c0 + kSlots);
+            if (c0 + kSlots + tid < total) {
+                key = ldu(cand, (uint32_t)(c0 + kSlots + tid));
+                in = load_pair<DIS>(key, arr);
+            }
+        }
         __syncthreads();
         const int lo = max(first, c0), hi = min(first + nc, c0 + kSlots);
         if (lo < hi) {  // this node's accepted pairs of the round, in list order (at most kPMax < 64 bits)
@@ -1172,7 +1195,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
     const int tid = threadIdx.x;
     const bool node = tid < kNodes;
     const MeshDev* mesh = p.mesh;
-    const bool fused = kStep;
+    constexpr bool fused = kStep;
     const bool forces = kStep || mode != M_PAIRS;
     const bool search = kStep || mode != M_BONDED;
     // a multi-system step walks the compact list of live slots (k_live)
@@ -1196,6 +1219,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
         }
         const MeshRec mt = ldu(mesh->th, ln);
         const float sg = fused ? ldu(mesh->gs, ln).sign : 0.f;
+        const MeshRec r0 = ldu(mesh->r0, ln), ir0 = ldu(mesh->ir0, ln);
         const int s = __builtin_amdgcn_readfirstlane(sys_of(p, r, slot));
         if (s < 0) continue;
         SysMeta* M = p.meta + s;
@@ -1240,7 +1264,6 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
                 }
                 // ---- springs, propagate.cu:298-314
                 const float stiffness = cld(p.E + slot);
-                const MeshRec r0 = ldu(mesh->r0, lane_index()), ir0 = ldu(mesh->ir0, lane_index());
                 bool ok = true;
 #pragma unroll
                 for (int i = 0; i < 3; ++i) {
@@ -1283,6 +1306,18 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
                 fdz = fdz - gint * (viz - svz[N]);
             }
         }
+        // the lane's first pair and the gather table load while the barrier and the
+        // gather of the angle forces pass
+        const size_t sb = (size_t)sbase * kSlots;  // the system's first node
+        const SysArrays arr{rX + sb, rY + sb, rZ + sb, rVX + sb, rVY + sb, rVZ + sb, p.VRANGE + (size_t)sbase * 6,
+                            rBB + (size_t)sbase * 6};
+        // (lanes past the list load their own node)
+        const PairIn in = load_pair<fused>(lt < total ? key0 : c * kSlots + lt, arr);
+        uint32_t gt[3] = {0u, 0u, 0u};
+        if (angles) {
+            const uint32_t lg = lane_index();
+            gt[0] = ldu(mesh->r0, lg).w; gt[1] = ldu(mesh->ir0, lg).w; gt[2] = ldu(mesh->gs, lg).w;
+        }
         __syncthreads();  // the angle forces, normals and owners of every node are in LDS
         if (forces) {
             if (node) {
@@ -1305,8 +1340,6 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
                     ay = ay - (a[q * 6 + 1] + a[q * 6 + 4]);
                     az = az - (a[q * 6 + 2] + a[q * 6 + 5]);
                 }
-                const uint32_t lg = lane_index();
-                const uint32_t gt[3] = {ldu(mesh->r0, lg).w, ldu(mesh->ir0, lg).w, ldu(mesh->gs, lg).w};
 #pragma unroll
                 for (int q = 0; q < 6; ++q) {
                     const float* f = u.angF + ((gt[q >> 1] >> (16 * (q & 1))) & 0xffffu);
@@ -1320,7 +1353,6 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
         float cfx = 0.f, cfy = 0.f, cfz = 0.f;
         int np = 0;
         if (total > 0) {
-            const size_t sb = (size_t)sbase * kSlots;                      // the system's first node
             const RuleCtx R = rule_ctx(MC, P);
             PairConsts k;
             k.ar = P->attraction_range;
@@ -1330,20 +1362,15 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
             k.kr = +P->repulsion_strength * P->youngs_mod;
             k.gext = P->viscotic_damping;
             int32_t* rec = p.PAIRS + (size_t)slot * kPMax * kSlots;
-            const int32_t* sVR = p.VRANGE + (size_t)sbase * 6;
-            const float* sBB = rBB + (size_t)sbase * 6;
             if (fused)
-                np = pair_pass<true, true>(cand, key0, rec, lt, first, nc, total, u.pr, owner, R, k, sx, sy, sz, svx, svy, svz,
-                                           snx, sny, snz, sVR, sBB, rX + sb, rY + sb, rZ + sb, rVX + sb, rVY + sb,
-                                           rVZ + sb, cfx, cfy, cfz, fdx, fdy, fdz);
+                np = pair_pass<true, true>(cand, key0, in, rec, lt, first, nc, total, u.pr, owner, R, k, sx, sy, sz, svx,
+                                           svy, svz, snx, sny, snz, arr, cfx, cfy, cfz, fdx, fdy, fdz);
             else if (forces)
-                np = pair_pass<true, false>(cand, key0, rec, lt, first, nc, total, u.pr, owner, R, k, sx, sy, sz, svx, svy,
-                                            svz, snx, sny, snz, sVR, sBB, rX + sb, rY + sb, rZ + sb, rVX + sb,
-                                            rVY + sb, rVZ + sb, cfx, cfy, cfz, fdx, fdy, fdz);
+                np = pair_pass<true, false>(cand, key0, in, rec, lt, first, nc, total, u.pr, owner, R, k, sx, sy, sz, svx,
+                                            svy, svz, snx, sny, snz, arr, cfx, cfy, cfz, fdx, fdy, fdz);
             else
-                np = pair_pass<false, false>(cand, key0, rec, lt, first, nc, total, u.pr, owner, R, k, sx, sy, sz, svx, svy,
-                                             svz, snx, sny, snz, sVR, sBB, rX + sb, rY + sb, rZ + sb, rVX + sb,
-                                             rVY + sb, rVZ + sb, cfx, cfy, cfz, fdx, fdy, fdz);
+                np = pair_pass<false, false>(cand, key0, in, rec, lt, first, nc, total, u.pr, owner, R, k, sx, sy, sz,
+                                             svx, svy, svz, snx, sny, snz, arr, cfx, cfy, cfz, fdx, fdy, fdz);
         }
         if (search && node) {
             const float X = lds_reread(sx, lt), Y = lds_reread(sy, lt), Z = lds_reread(sz, lt);
