@@ -33,6 +33,7 @@ void launch_grid(const Pool& p, const Range& r, int vox_blocks, hipStream_t st);
 void launch_vox_lists(const Pool& p, const Range& r, int vox_blocks, hipStream_t st);
 void launch_vrange(const Pool& p, const Range& r, hipStream_t st);
 void launch_velocity_ab(const Pool& p, const Range& r, int which, hipStream_t st);
+void launch_pairs_list(const Pool& p, const Range& r, hipStream_t st);
 void launch_cellbox(const Pool& p, const Range& r, hipStream_t st);
 void launch_extent(const Pool& p, const Range& r, float* out, hipStream_t st);
 void launch_pressure_reset(const Pool& p, const Range& r, const int32_t* cells, int count, float value,
@@ -88,6 +89,7 @@ struct SysHost {
     int32_t vbudget = 0, vcap = 0;
     int64_t breg = 0;  // search-bin region offset
     int32_t bbudget = 0;
+    bool pairs_stale = false;  // a contact pass ran since the partner lists were made
     cs3d_params prm;
 };
 
@@ -237,8 +239,25 @@ void enqueue_step(cs3d_ctx* c, const Range& r, int /*vb*/) {
     for (int q = 0; q < CS3D_PHASES; ++q) enqueue_step_phase(c, r, q);
 }
 
+// The partner lists of a system (CS3D_F_PAIRS, CS3D_F_PAIRCOUNT) are made from the
+// candidates and their accept bits when a caller looks at them; a contact pass
+// makes them stale.
+void pairs_stale(cs3d_ctx* c, cs3d_sys s) {
+    if (s != CS3D_ALL) {
+        c->sys[s].pairs_stale = true;
+        return;
+    }
+    for (int i = 0; i < c->nsys_high; ++i) c->sys[i].pairs_stale = c->sys[i].used;
+}
+void make_pairs(cs3d_ctx* c, cs3d_sys s) {
+    if (!c->sys[s].pairs_stale) return;
+    launch_pairs_list(c->pool, range_of(c, s), c->stream);
+    c->sys[s].pairs_stale = false;
+}
+
 cs3d_status run_startup(cs3d_ctx* c, cs3d_sys s) {
     const Pool& p = c->pool;
+    pairs_stale(c, s);
     Range r = range_of(c, s);
     const int vb = vox_blocks_of(c, s);
     // CenterOfMass, bounding_boxes, minmaxpre/post, makeNNlist (GPUbounce.cu:739-763)
@@ -520,6 +539,7 @@ extern "C" cs3d_status cs3d_system_add_raw(cs3d_ctx* c, const cs3d_params* prm, 
     HIPCHK(hipMemsetAsync(p.BBOX + base * 6, 0, (size_t)max_cells * 24, c->stream));
     HIPCHK(hipMemsetAsync(p.BBOXN + base * 6, 0, (size_t)max_cells * 24, c->stream));
     HIPCHK(hipMemsetAsync(p.NPAIR + nb, 0, (size_t)max_cells * kSlots * 4, c->stream));
+    HIPCHK(hipMemsetAsync(p.NCAND + nb, 0, (size_t)max_cells * kSlots * 4, c->stream));
     HIPCHK(hipMemsetAsync(p.vox + vreg, 0, (size_t)vb * (1 + vcap) * 4, c->stream));
     HIPCHK(hipMemsetAsync(p.bins + breg, 0, (size_t)bb * 4, c->stream));
     std::vector<float> pv(max_cells, prm->min_pressure), ev(max_cells, prm->stiffness1), gv(max_cells, 1.0f);
@@ -697,6 +717,10 @@ extern "C" cs3d_status cs3d_get(cs3d_ctx* c, cs3d_sys s, cs3d_field f, void* hos
         }
         return CS3D_OK;
     }
+    if (f == CS3D_F_PAIRS || f == CS3D_F_PAIRCOUNT) {
+        make_pairs(c, s);
+        HIPCHK(hipGetLastError());
+    }
     if (f == CS3D_F_BBOX || f == CS3D_F_VOXCOUNT || f == CS3D_F_VOXLIST) {
         // the fused step keeps voxel counts only and leaves the per-cell part of a
         // grid rebuilt in the last step to the next step: complete it and fill the
@@ -773,6 +797,7 @@ extern "C" cs3d_status cs3d_set(cs3d_ctx* c, cs3d_sys s, cs3d_field f, const voi
         HIPCHK(hipStreamSynchronize(c->stream));
         return CS3D_OK;
     }
+    if (f == CS3D_F_PAIRS || f == CS3D_F_PAIRCOUNT) make_pairs(c, s);  // what the caller leaves as it is
     HIPCHK(hipMemcpyAsync(L.ptr, host, bytes, hipMemcpyHostToDevice, c->stream));
     if (f == CS3D_F_BBOX) launch_vrange(c->pool, range_of(c, s), c->stream);
     HIPCHK(hipGetLastError());
@@ -1145,6 +1170,7 @@ extern "C" cs3d_status cs3d_step_timed(cs3d_ctx* c, cs3d_sys s, int32_t n_steps,
     if (s != CS3D_ALL && !valid_sys(c, s)) return fail(CS3D_INVALID_ARG, "unknown system");
     const Range r = range_of(c, s);
     if (r.slot_hi <= r.slot_lo || r.sys_hi <= r.sys_lo) return CS3D_OK;
+    pairs_stale(c, s);
     cs3d_status st = CS3D_OK;
     for (int k = 0; k < n_steps && st == CS3D_OK; ++k)
         st = timed_groups(c, CS3D_PHASES, [&](int q) { enqueue_step_phase(c, r, q); }, phase_ms);
@@ -1197,6 +1223,7 @@ extern "C" cs3d_status cs3d_step(cs3d_ctx* c, cs3d_sys s, int32_t n_steps) {
     if (s == CS3D_ALL && c->nsys_high == 0) return CS3D_OK;
     const Range r = range_of(c, s);
     const int vb = vox_blocks_of(c, s);
+    pairs_stale(c, s);
     int done = 0;
     if (c->use_graph && n_steps >= c->graph_steps) {
         const cs3d_ctx::GraphRec* g = nullptr;
@@ -1261,6 +1288,7 @@ extern "C" cs3d_status cs3d_k_con_force(cs3d_ctx* c, cs3d_sys s) {
     launch_integrate(c->pool, r, I_BINS, 0, c->stream);
     launch_search(c->pool, r, 1, c->stream);
     launch_con(c->pool, r, M_CON, false, c->stream);
+    pairs_stale(c, s);
     launch_integrate(c->pool, r, I_CLEAR, 0, c->stream);
     launch_set_flags(c->pool, r, -1, 1, c->stream);
     return finish(c);
@@ -1278,6 +1306,7 @@ extern "C" cs3d_status cs3d_k_dis_force(cs3d_ctx* c, cs3d_sys s, int32_t which) 
     launch_integrate(c->pool, r, I_BINS, 0, c->stream);
     launch_search(c->pool, r, 1, c->stream);
     launch_con(c->pool, r, M_PAIRS, false, c->stream);
+    pairs_stale(c, s);
     launch_dis(c->pool, r, which ? M_DIS_VA : M_DIS_V, 0, 1, which != 0, c->stream);
     launch_set_flags(c->pool, r, -1, 1, c->stream);
     return finish(c);
@@ -1418,6 +1447,8 @@ extern "C" cs3d_status cs3d_time_kernel(cs3d_ctx* c, cs3d_sys s, int32_t which, 
         else if (which == 1) launch_dis(c->pool, r, M_COM, 0, 0, false, c->stream);
         else launch_search(c->pool, r, 1, c->stream);
     };
+    // the timed search replaces the candidates that the accept bits belong to
+    if (which == 2) make_pairs(c, s);
     // the full search reads the search bins: filled from the current positions here,
     // cleared after, and the next step searches again (as after cs3d_k_con_force)
     if (which == 2) launch_integrate(c->pool, r, I_BINS, 0, c->stream);

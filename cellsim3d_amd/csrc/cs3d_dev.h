@@ -8,11 +8,12 @@
 //                float[cap_cells * 6]    bbox of the positions at the end of the latest step
 //                int32[cap_cells * 6]    voxel range of the contact-rule bbox (kept with it)
 //   pair lists   int32[cap_cells * kPMax * 192]  contact partners of each node, (cell, node)
-//                ascending, k-major per cell so lanes access consecutive words
-//                int32[cap_cells * 192]  partner count per node
+//                ascending, k-major per cell, and int32[cap_cells * 192] their count: made
+//                from the candidates and their accept bits when a caller reads them
 //                int32[cap_cells * kPMax * 192]  contact candidates (within attraction_range + skin
 //                at the last search): per cell one flat list, node after node, + per node the
-//                count (low kCandBits bits) and the index of its first entry (above them)
+//                count (low kCandBits bits) and the index of its first entry (above them); behind the
+//                list one accept bit per entry
 //                float[cap_cells * 192] x3  node positions at the last search
 //   voxel pool   int32                   per system: counts[budget] then lists[budget * capacity]
 //                                        (the reference's 2.9-wide cell grid)
@@ -37,6 +38,12 @@ constexpr int kFacePad = 128;        // rows of the face table (CS3D_FACES, the 
 constexpr int kPMax = 40;            // contact candidates / partners stored per node
 constexpr int kCandBits = 8;         // low bits of an NCAND word that hold the count
 static_assert(kPMax < (1 << kCandBits), "a node's candidate count fits its bits");
+// The candidate room of a cell (kPMax * kSlots words) holds its flat list (at most
+// kPMax * kNodes words) and, behind it, one bit per entry: accepted by the contact
+// tests of the latest contact pass (entry j is bit j % 64 of word j / 64).
+constexpr int kMaskAt = kPMax * kNodes;
+constexpr int kMaskWords = (kMaskAt + kSlots - 1) / kSlots * (kSlots / 64);
+static_assert(kMaskAt % 2 == 0 && kMaskAt + 2 * kMaskWords <= kPMax * kSlots, "the mask fits behind the list");
 constexpr int kBCap = CS3D_BIN_CAP;  // nodes per search bin
 constexpr int kMaxSys = 4096;        // systems per context
 constexpr int kMaxPartial = 192;     // listed cells beyond which the next search is a full one (at most the
@@ -113,6 +120,10 @@ struct MeshDev {
     ThetaCoeffs theta;  // kTheta
 };
 __host__ __device__ inline int mesh_nn(uint32_t w, int k) { return (int)((w >> (8 * k)) & 0xffu); }
+
+__host__ __device__ inline uint64_t* pair_mask(int32_t* cand, int64_t slot) {
+    return reinterpret_cast<uint64_t*>(cand + slot * (kPMax * kSlots) + kMaskAt);
+}
 
 struct Pool {
     float *X, *Y, *Z;

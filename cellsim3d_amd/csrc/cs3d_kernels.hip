@@ -864,43 +864,6 @@ struct PairConsts {
 // Partner keys are local cell * 192 + node: the index of the node in a system's
 // arrays, read through the system's first slot (a uniform pointer).
 
-constexpr int kChunk = 4;  // partners whose loads are issued together
-
-// Friction (propagate.cu:633-653) over the node's stored partners, in stored
-// (reference) order.  The keys, then the partner velocities, of kChunk partners
-// are loaded before any of them is used.
-// lst: the cell's list (uniform), entries at i * 192 + tid; sVX/sVY/sVZ: the
-// velocity arrays from the system's first slot (uniform).
-__device__ __forceinline__ void pair_friction(const int32_t* lst, int tid, int np, float vix, float viy, float viz,
-                                              float nx, float ny, float nz, float gext,
-                                              const float* __restrict__ sVX, const float* __restrict__ sVY,
-                                              const float* __restrict__ sVZ, float& fdx, float& fdy, float& fdz) {
-    for (int i0 = 0; i0 < np; i0 += kChunk) {
-        uint32_t g[kChunk];
-#pragma unroll
-        for (int j = 0; j < kChunk; ++j) g[j] = i0 + j < np ? (uint32_t)ldu(lst, (uint32_t)((i0 + j) * kSlots + tid)) : 0u;
-        float wx[kChunk], wy[kChunk], wz[kChunk];
-#pragma unroll
-        for (int j = 0; j < kChunk; ++j) {
-            const bool in = i0 + j < np;
-            wx[j] = in ? ldu(sVX, g[j]) : 0.f;
-            wy[j] = in ? ldu(sVY, g[j]) : 0.f;
-            wz[j] = in ? ldu(sVZ, g[j]) : 0.f;
-        }
-#pragma unroll
-        for (int j = 0; j < kChunk; ++j) {
-            if (i0 + j < np) {
-                const float vx = vix - wx[j], vy = viy - wy[j], vz = viz - wz[j];
-                const float d = vx * nx + vy * ny + vz * nz;
-                const float tx = vx - d * nx, ty = vy - d * ny, tz = vz - d * nz;
-                fdx = fdx - gext * tx;
-                fdy = fdy - gext * ty;
-                fdz = fdz - gext * tz;
-            }
-        }
-    }
-}
-
 // The contact pass works on pairs, not on nodes: the candidates of a cell's nodes
 // lie one after another in the cell's list (node order, each node's keys ascending,
 // so reference order), and lane t of the workgroup takes entry c0 + t of the list,
@@ -910,16 +873,26 @@ __device__ __forceinline__ void pair_friction(const int32_t* lst, int tid, int n
 // and leaves the force terms in LDS; each node then adds the terms of its accepted
 // pairs in list order, so every sum has the reference's order.
 // NCAND holds a node's candidate count in its low kCandBits bits and the index of
-// its first entry above them.
+// its first entry above them.  Which entries are accepted is kept as one bit per
+// entry (pair_mask) for the second friction pass; the partner lists that callers
+// read (CS3D_F_PAIRS) are made from it when they are read (k_pairs_list).
 struct PairLds {
     float t[9][kSlots];    // attraction, repulsion and friction terms of the round's pairs
-    int32_t key[kSlots];   // their partner keys
     uint64_t ok[4];        // accepted pairs of the round, one bit each (the fourth word stays 0)
 };
 
-// owner[j] = node whose entry c0 + j is, for this lane's entries in the round
+// the n bits (1 to 63) from bit j of the words at m (one word past them is read)
+__device__ __forceinline__ uint64_t bit_range(const uint64_t* m, int j, int n) {
+    const int w = j >> 6, sh = j & 63;
+    uint64_t bits = m[w] >> sh;
+    if (sh) bits |= m[w + 1] << (64 - sh);
+    return bits & ((1ull << n) - 1);
+}
+
+// owner[j] = node whose entry c0 + j is, for this lane's entries in the round of kRound entries
+template <int kRound = kSlots>
 __device__ __forceinline__ void fill_owners(uint8_t* owner, int tid, int first, int nc, int c0) {
-    const int lo = max(first, c0), hi = min(first + nc, c0 + kSlots);
+    const int lo = max(first, c0), hi = min(first + nc, c0 + kRound);
     for (int j = lo; j < hi; ++j) owner[j - c0] = (uint8_t)tid;
 }
 
@@ -985,21 +958,20 @@ __device__ __forceinline__ bool pair_terms(const PairIn& in, float X, float Y, f
     return true;
 }
 
-// All pairs of a cell (every lane of the workgroup calls it).  cand, rec: the
-// cell's candidate list (flat) and accepted-partner lists (entries at i * 192 +
-// tid), uniform; key, in: the lane's pair of the first round (where tid < total);
-// first, nc: this lane's entries; total: entries of the cell;
+// All pairs of a cell (every lane of the workgroup calls it).  cand, mask: the
+// cell's candidate list (flat) and its accepted entries, uniform; in: the lane's
+// pair of the first round (where tid < total); first, nc: this lane's entries;
+// total: entries of the cell;
 // owner: filled for the first round and visible; sx .. snz: the
 // cell's own positions, velocities and normals in LDS.  u is written only after a
-// barrier that ends its previous use.  Returns the number accepted.
+// barrier that ends its previous use.
 template <bool CON, bool DIS>
-__device__ __forceinline__ int pair_pass(const int32_t* cand, int key, PairIn in, int32_t* rec, int tid, int first,
+__device__ __forceinline__ void pair_pass(const int32_t* cand, uint64_t* mask, PairIn in, int tid, int first,
                                          int nc, int total, PairLds& u, uint8_t* owner, const RuleCtx& R,
                                          const PairConsts& k, const float* sx, const float* sy, const float* sz,
                                          const float* svx, const float* svy, const float* svz, const float* snx,
                                          const float* sny, const float* snz, const SysArrays& arr, float& cfx,
                                          float& cfy, float& cfz, float& fdx, float& fdy, float& fdz) {
-    int np = 0;
     for (int c0 = 0; c0 < total; c0 += kSlots) {
         float t[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         bool ok = false;
@@ -1011,10 +983,12 @@ __device__ __forceinline__ int pair_pass(const int32_t* cand, int key, PairIn in
         }
         __syncthreads();  // the previous use of u, and this round's owners, are done
         const uint64_t m = __ballot(ok);
-        if ((tid & 63) == 0) u.ok[tid >> 6] = m;
+        if ((tid & 63) == 0) {
+            u.ok[tid >> 6] = m;
+            mask[(c0 + tid) >> 6] = m;
+        }
         if (tid == 0) u.ok[3] = 0;
         if (ok) {
-            u.key[tid] = key;
             if (CON) {
 #pragma unroll
                 for (int a = 0; a < 6; ++a) u.t[a][tid] = t[a];
@@ -1026,23 +1000,15 @@ __device__ __forceinline__ int pair_pass(const int32_t* cand, int key, PairIn in
         }
         if (c0 + kSlots < total) {  // the next round's pair
             fill_owners(owner, tid, first, nc, c0 + kSlots);
-            if (c0 + kSlots + tid < total) {
-                key = ldu(cand, (uint32_t)(c0 + kSlots + tid));
-                in = load_pair<DIS>(key, arr);
-            }
+            if (c0 + kSlots + tid < total) in = load_pair<DIS>(ldu(cand, (uint32_t)(c0 + kSlots + tid)), arr);
         }
         __syncthreads();
         const int lo = max(first, c0), hi = min(first + nc, c0 + kSlots);
-        if (lo < hi) {  // this node's accepted pairs of the round, in list order (at most kPMax < 64 bits)
-            const int j0 = lo - c0, w = j0 >> 6, sh = j0 & 63;
-            uint64_t bits = u.ok[w] >> sh;
-            if (sh) bits |= u.ok[w + 1] << (64 - sh);
-            bits &= (1ull << (hi - lo)) - 1;
+        if (lo < hi) {  // this node's accepted pairs of the round, in list order
+            uint64_t bits = bit_range(u.ok, lo - c0, hi - lo);
             while (bits) {
-                const int j = j0 + __ffsll((unsigned long long)bits) - 1;
+                const int j = lo - c0 + __ffsll((unsigned long long)bits) - 1;
                 bits &= bits - 1;
-                stu(rec, (uint32_t)(np * kSlots + tid), u.key[j]);
-                ++np;
                 if (CON) {
                     cfx += u.t[0][j]; cfy += u.t[1][j]; cfz += u.t[2][j];
                     cfx += u.t[3][j]; cfy += u.t[4][j]; cfz += u.t[5][j];
@@ -1051,7 +1017,6 @@ __device__ __forceinline__ int pair_pass(const int32_t* cand, int key, PairIn in
             }
         }
     }
-    return np;
 }
 
 // ------------------------------------------------------------------------------
@@ -1351,7 +1316,6 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
             }
         }
         float cfx = 0.f, cfy = 0.f, cfz = 0.f;
-        int np = 0;
         if (total > 0) {
             const RuleCtx R = rule_ctx(MC, P);
             PairConsts k;
@@ -1361,15 +1325,15 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
             k.ka = -P->attraction_strength * P->youngs_mod;
             k.kr = +P->repulsion_strength * P->youngs_mod;
             k.gext = P->viscotic_damping;
-            int32_t* rec = p.PAIRS + (size_t)slot * kPMax * kSlots;
+            uint64_t* mask = pair_mask(p.CAND, slot);
             if (fused)
-                np = pair_pass<true, true>(cand, key0, in, rec, lt, first, nc, total, u.pr, owner, R, k, sx, sy, sz, svx,
+                pair_pass<true, true>(cand, mask, in, lt, first, nc, total, u.pr, owner, R, k, sx, sy, sz, svx,
                                            svy, svz, snx, sny, snz, arr, cfx, cfy, cfz, fdx, fdy, fdz);
             else if (forces)
-                np = pair_pass<true, false>(cand, key0, in, rec, lt, first, nc, total, u.pr, owner, R, k, sx, sy, sz, svx,
+                pair_pass<true, false>(cand, mask, in, lt, first, nc, total, u.pr, owner, R, k, sx, sy, sz, svx,
                                             svy, svz, snx, sny, snz, arr, cfx, cfy, cfz, fdx, fdy, fdz);
             else
-                np = pair_pass<false, false>(cand, key0, in, rec, lt, first, nc, total, u.pr, owner, R, k, sx, sy, sz,
+                pair_pass<false, false>(cand, mask, in, lt, first, nc, total, u.pr, owner, R, k, sx, sy, sz,
                                              svx, svy, svz, snx, sny, snz, arr, cfx, cfy, cfz, fdx, fdy, fdz);
         }
         if (search && node) {
@@ -1380,7 +1344,6 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
                 fdy = fdy - P->gamma_visc * viy;
                 fdz = fdz - P->gamma_visc * viz;
             }
-            stu(pool_late()->NPAIR + cb, ln, np);
             if (forces) {
                 FX += cfx; FY += cfy; FZ += cfz;
                 if (P->use_rigid_box) {  // propagate.cu:473-510 (lower wall at 0)
@@ -1557,29 +1520,72 @@ __global__ __launch_bounds__(192) void k_bonded(Pool p, Range r) {
 }
 
 // ------------------------------------------------------------------------------
+// Reductions over a wave without LDS.  lane_down<o> gives a lane the value of the
+// lane o above it, for the lanes that a tree reduction to lane 0 still uses at that
+// level (lanes below o): the halves and rows of a wave are swapped by
+// v_permlane32_swap / v_permlane16_swap, within a row of 16 the DPP row shift reads
+// upwards.  The pairs are those of the shuffle tree (i, i + o), o = 32 .. 1.
+// ------------------------------------------------------------------------------
+template <int o> __device__ __forceinline__ float lane_down(float v) {
+    const uint32_t x = __float_as_uint(v);
+    if constexpr (o == 32) return __uint_as_float(__builtin_amdgcn_permlane32_swap(x, x, false, false)[1]);
+    else if constexpr (o == 16) return __uint_as_float(__builtin_amdgcn_permlane16_swap(x, x, false, false)[1]);
+    else return __int_as_float(__builtin_amdgcn_update_dpp(0, (int)x, 0x100 | o, 0xf, 0xf, true));
+}
+struct OpAdd { static __device__ __forceinline__ float f(float a, float b) { return a + b; } };
+struct OpMin { static __device__ __forceinline__ float f(float a, float b) { return fminf(a, b); } };
+struct OpMax { static __device__ __forceinline__ float f(float a, float b) { return fmaxf(a, b); } };
+template <class Op> __device__ __forceinline__ float wave_tree(float v) {  // the result is lane 0's
+    v = Op::f(v, lane_down<32>(v));
+    v = Op::f(v, lane_down<16>(v));
+    v = Op::f(v, lane_down<8>(v));
+    v = Op::f(v, lane_down<4>(v));
+    v = Op::f(v, lane_down<2>(v));
+    return Op::f(v, lane_down<1>(v));
+}
+// the value of the even lane of each lane pair
+__device__ __forceinline__ float even_lane(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xa0, 0xf, 0xf, true));  // quad_perm 0 0 2 2
+}
+
+// ------------------------------------------------------------------------------
 // Dissipative force (CalculateDisForce, propagate.cu:523-665) with the
 // end-of-step velocities, then CenterOfMass (centermass.cu:8-50) and, on growth
 // steps, volumes (volume.cu:5-163).  Modes: M_STEP, M_DIS_V, M_DIS_VA, M_COM,
 // M_VOLUMES.
 // ------------------------------------------------------------------------------
-// kLive: walk Pool::LIVE (a multi-system step) instead of the range's slots
-template <int kLive>
+// What bounds it: at a few hundred cells the latency of one cell's chain (loads,
+// barriers, dependent arithmetic), at 20,000 cells memory traffic.  Friction works
+// on pairs as in k_con_dis, two entries of the cell's candidate list per lane and
+// round (384 cover most cells in one round), gated by the accept bits that
+// k_con_dis left; the centre of mass is one wave's work straight from the positions
+// in LDS, beside the other waves' normals; the box and the trees use cross-lane
+// moves instead of LDS; each face is shared by two lanes, which split its edges.
+// kLive: walk Pool::LIVE (a multi-system step) instead of the range's slots; kStep:
+// mode is M_STEP
+template <int kLive, bool kStep>
 __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode, int64_t step_override,
                                                   int32_t clear_bins, const float* __restrict__ rX,
                                                   const float* __restrict__ rY, const float* __restrict__ rZ,
                                                   const float* __restrict__ rVX, const float* __restrict__ rVY,
                                                   const float* __restrict__ rVZ) {
+    constexpr int kRound = 2 * kSlots;
     __shared__ float sx[kSlots], sy[kSlots], sz[kSlots];
     __shared__ float svx[kSlots], svy[kSlots], svz[kSlots];
-    __shared__ float red[3][128];
+    __shared__ float snx[kSlots], sny[kSlots], snz[kSlots];  // friction normals
+    __shared__ float term[3][kRound];                        // friction terms of the round's pairs
+    __shared__ uint64_t okm[kRound / 64 + 1];                // their accept bits (the last word stays 0)
+    __shared__ uint8_t owner[kRound];
+    __shared__ float red[2][128];
     __shared__ float cm[3];
     __shared__ float bpart[3][6];
     __shared__ int32_t moved;
     const int tid = threadIdx.x;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool node = tid < kNodes;
     const MeshDev* mesh = p.mesh;
-    const bool do_dis = mode == M_STEP || mode == M_DIS_V || mode == M_DIS_VA;
-    const bool fused = mode == M_STEP;
+    const bool do_dis = kStep || mode == M_DIS_V || mode == M_DIS_VA;
+    constexpr bool fused = kStep;
     // a multi-system step walks the compact list of live slots (k_live)
     const int nit = kLive ? *p.n_live : r.slot_hi - r.slot_lo;
     for (int it = xcd_block(); it < nit; it += gridDim.x) {
@@ -1588,17 +1594,27 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
         // overlaps the metadata reads
         const size_t cb = (size_t)slot * kSlots;  // the cell's first node (uniform)
         const uint32_t ln = lane_index();
+        const int lt = (int)ln;
         const float X = ldu(rX + cb, ln), Y = ldu(rY + cb, ln), Z = ldu(rZ + cb, ln);
         float vX = 0.f, vY = 0.f, vZ = 0.f;
-        if (do_dis) { vX = ldu(rVX + cb, ln); vY = ldu(rVY + cb, ln); vZ = ldu(rVZ + cb, ln); }
-        const int np = (do_dis && node) ? ldu(p.NPAIR + cb, ln) : 0;
-        const uint32_t nnw = do_dis ? ldu(mesh->th, ln).w : 0u;
-        const float sg = do_dis ? ldu(mesh->gs, ln).sign : 0.f;
+        const int32_t* cand = p.CAND + (size_t)slot * kPMax * kSlots;
+        const uint64_t* mask = pair_mask(p.CAND, slot);
+        int ncf = 0, total = 0, key[2] = {0, 0};
+        uint64_t m[2] = {0, 0};  // this wave's words of the first round
+        if (do_dis) {
+            vX = ldu(rVX + cb, ln); vY = ldu(rVY + cb, ln); vZ = ldu(rVZ + cb, ln);
+            ncf = ldu(p.NCAND + cb, ln);
+            key[0] = ldu(cand, ln); key[1] = ldu(cand, ln + kSlots);
+            total = cld(p.NCAND + cb + kNodes) >> kCandBits;
+            m[0] = cld(mask + wv); m[1] = cld(mask + 3 + wv);
+        }
         float fcX = 0.f, fcY = 0.f, fcZ = 0.f, xbX = 0.f, xbY = 0.f, xbZ = 0.f;
-        if (fused && do_dis && node) {
+        if (fused && node) {
             fcX = ldu(p.FCX + cb, ln); fcY = ldu(p.FCY + cb, ln); fcZ = ldu(p.FCZ + cb, ln);
             xbX = ldu(p.XBX + cb, ln); xbY = ldu(p.XBY + cb, ln); xbZ = ldu(p.XBZ + cb, ln);
         }
+        const uint32_t nnw = do_dis ? ldu(mesh->th, ln).w : 0u;
+        const float sg = do_dis ? ldu(mesh->gs, ln).sign : 0.f;
         const int s = sys_of(p, r, slot);
         if (s < 0) continue;
         // metadata and parameters through scalar loads: the fields read here are not
@@ -1610,15 +1626,32 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
         if (!sys_live(MC)) continue;
         const int c = slot - MC->base;
         if (c >= MC->n) continue;
-        if (tid == 0) moved = 0;
-        sx[tid] = X; sy[tid] = Y; sz[tid] = Z;
-        if (do_dis) { svx[tid] = vX; svy[tid] = vY; svz[tid] = vZ; }
+        const int nc = ncf & ((1 << kCandBits) - 1), first = ncf >> kCandBits;
+        if (tid == 0) { moved = 0; okm[kRound / 64] = 0; }
+        sx[lt] = X; sy[lt] = Y; sz[lt] = Z;
+        if (do_dis) {
+            svx[lt] = vX; svy[lt] = vY; svz[lt] = vZ;
+            fill_owners<kRound>(owner, lt, first, nc, 0);
+        }
         __syncthreads();
         uint32_t st = 0;
-        bool far = false;
+        const size_t sb = (size_t)MC->base * kSlots;  // the system's first node
+        float fx = 0.f, fy = 0.f, fz = 0.f;
+        float wx[2], wy[2], wz[2];  // partner velocities of the lane's accepted pairs
+        bool acc[2];
+        auto load_partners = [&](int c0) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const bool in = c0 + h * kSlots + lt < total;
+                acc[h] = in && (m[h] >> (lt & 63) & 1);
+                const uint32_t g = acc[h] ? (uint32_t)key[h] : (uint32_t)(c * kSlots + lt);
+                wx[h] = ldu(rVX + sb, g); wy[h] = ldu(rVY + sb, g); wz[h] = ldu(rVZ + sb, g);
+                if ((lt & 63) == 0) okm[3 * h + (lt >> 6)] = c0 + h * kSlots < total ? m[h] : 0;
+            }
+        };
+        if (do_dis) load_partners(0);
         if (do_dis && node) {
-            float fx = 0.f, fy = 0.f, fz = 0.f;
-            const float vix = svx[tid], viy = svy[tid], viz = svz[tid];
+            const float vix = svx[lt], viy = svy[lt], viz = svz[lt];
             const float gint = P->internal_damping;
             const int nn3[3] = {mesh_nn(nnw, 0), mesh_nn(nnw, 1), mesh_nn(nnw, 2)};
 #pragma unroll
@@ -1630,16 +1663,86 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
             }
             float nx, ny, nz;
             node_normal(sx, sy, sz, sg, nn3[0], nn3[1], nn3[2], nx, ny, nz);
-            PairConsts k;
-            k.ar = P->attraction_range;
-            k.ar2 = k.ar * k.ar;
-            k.rr = P->repulsion_range;
-            k.ka = 0.f;
-            k.kr = 0.f;
-            k.gext = P->viscotic_damping;
-            const int32_t* lst = p.PAIRS + (size_t)slot * kPMax * kSlots;
-            const size_t sb = (size_t)MC->base * kSlots;  // the system's first node
-            pair_friction(lst, (int)ln, np, vix, viy, viz, nx, ny, nz, k.gext, rVX + sb, rVY + sb, rVZ + sb, fx, fy, fz);
+            snx[lt] = nx; sny[lt] = ny; snz[lt] = nz;
+        }
+        const bool do_com = kStep || mode == M_COM;
+        if (do_com && wv == 2) {
+            // 256-slot tree of centermass.cu:32-41: slots t and t+128 (180 and above hold 0),
+            // t and t+64, then 32..1 across the wave
+            const int t = lt & 63;
+            const bool hi = t + 128 < kNodes;
+            const float a = (sx[t] + (hi ? sx[t + 128] : 0.0f)) + (sx[t + 64] + 0.0f);
+            const float b = (sy[t] + (hi ? sy[t + 128] : 0.0f)) + (sy[t + 64] + 0.0f);
+            const float d = (sz[t] + (hi ? sz[t + 128] : 0.0f)) + (sz[t + 64] + 0.0f);
+            const float ra = wave_tree<OpAdd>(a), rb = wave_tree<OpAdd>(b), rd = wave_tree<OpAdd>(d);
+            if (t == 0) {
+                cm[0] = ra / 180.0f; cm[1] = rb / 180.0f; cm[2] = rd / 180.0f;
+                const CPool q = pool_late();
+                q->CMX[slot] = cm[0]; q->CMY[slot] = cm[1]; q->CMZ[slot] = cm[2];
+            }
+        } else if (!do_com && tid == 0) {
+            const CPool q = pool_late();
+            cm[0] = q->CMX[slot]; cm[1] = q->CMY[slot]; cm[2] = q->CMZ[slot];
+        }
+        if (fused) {  // this wave's part of the cell's bbox at the end of the step (bounding_boxes, propagatebound.cu:10-141)
+            const float b0 = wave_tree<OpMin>(node ? X : INFINITY), b1 = wave_tree<OpMax>(node ? X : -INFINITY);
+            const float b2 = wave_tree<OpMin>(node ? Y : INFINITY), b3 = wave_tree<OpMax>(node ? Y : -INFINITY);
+            const float b4 = wave_tree<OpMin>(node ? Z : INFINITY), b5 = wave_tree<OpMax>(node ? Z : -INFINITY);
+            if ((lt & 63) == 0) {
+                float* b = bpart[wv];
+                b[0] = b0; b[1] = b1; b[2] = b2; b[3] = b3; b[4] = b4; b[5] = b5;
+            }
+        }
+        __syncthreads();  // normals, owners, accept bits, centre and box parts are in LDS
+        if (fused && lt < 6) {
+            float b = bpart[0][lt];
+            b = (lt & 1) ? fmaxf(b, bpart[1][lt]) : fminf(b, bpart[1][lt]);
+            b = (lt & 1) ? fmaxf(b, bpart[2][lt]) : fminf(b, bpart[2][lt]);
+            stu(pool_late()->BBOXN + (size_t)slot * 6, ln, b);
+        }
+        if (do_dis) {
+            // ---- friction, propagate.cu:633-653: the pairs' terms, then each node's sum
+            const float gext = P->viscotic_damping;
+            for (int c0 = 0; c0 < total; c0 += kRound) {
+                if (c0 > 0) {
+                    __syncthreads();  // the sums of the round before are done
+                    fill_owners<kRound>(owner, lt, first, nc, c0);
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const int e = c0 + h * kSlots;
+                        key[h] = e + lt < total ? ldu(cand, (uint32_t)(e + lt)) : 0;
+                        m[h] = e < total ? cld(mask + e / 64 + wv) : 0;
+                    }
+                    load_partners(c0);
+                    __syncthreads();
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    if (acc[h]) {
+                        const int j = h * kSlots + lt, o = owner[j];
+                        const float nx = snx[o], ny = sny[o], nz = snz[o];
+                        const float vx = svx[o] - wx[h], vy = svy[o] - wy[h], vz = svz[o] - wz[h];
+                        const float d = vx * nx + vy * ny + vz * nz;
+                        term[0][j] = gext * (vx - d * nx);
+                        term[1][j] = gext * (vy - d * ny);
+                        term[2][j] = gext * (vz - d * nz);
+                    }
+                }
+                __syncthreads();
+                const int lo = max(first, c0), hi = min(first + nc, c0 + kRound);
+                if (lo < hi) {
+                    uint64_t bits = bit_range(okm, lo - c0, hi - lo);
+                    while (bits) {
+                        const int j = lo - c0 + __ffsll((unsigned long long)bits) - 1;
+                        bits &= bits - 1;
+                        fx = fx - term[0][j]; fy = fy - term[1][j]; fz = fz - term[2][j];
+                    }
+                }
+            }
+        }
+        bool far = false;
+        if (do_dis && node) {
+            const float vix = svx[lt], viy = svy[lt], viz = svz[lt];
             fx = fx - P->gamma_visc * vix;  // drag, propagate.cu:658
             fy = fy - P->gamma_visc * viy;
             fz = fz - P->gamma_visc * viz;
@@ -1649,30 +1752,32 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
                 // the next step's Integrate moves this node to X + v' dt with v' from the
                 // values now in V, F_con and F_dis (bit-identical to k_integrate): search
                 // again next step when that is pair_skin/2 or more from the last search
-                const float dt = P->dt, m = P->mass, rdt = sqrt_cr(dt);
+                const float dt = P->dt, m_ = P->mass, rdt = sqrt_cr(dt);
                 const bool rnd = P->add_rands != 0;
-                const float qx = X + half_kick(vix, fcX, fx, rnd ? ldu(q->FRX + cb, ln) : 0.f, dt, rdt, m, MC) * dt - xbX;
-                const float qy = Y + half_kick(viy, fcY, fy, rnd ? ldu(q->FRY + cb, ln) : 0.f, dt, rdt, m, MC) * dt - xbY;
-                const float qz = Z + half_kick(viz, fcZ, fz, rnd ? ldu(q->FRZ + cb, ln) : 0.f, dt, rdt, m, MC) * dt - xbZ;
+                const float x = lds_reread(sx, lt), y = lds_reread(sy, lt), z = lds_reread(sz, lt);
+                const float qx = x + half_kick(vix, fcX, fx, rnd ? ldu(q->FRX + cb, ln) : 0.f, dt, rdt, m_, MC) * dt - xbX;
+                const float qy = y + half_kick(viy, fcY, fy, rnd ? ldu(q->FRY + cb, ln) : 0.f, dt, rdt, m_, MC) * dt - xbY;
+                const float qz = z + half_kick(viz, fcZ, fz, rnd ? ldu(q->FRZ + cb, ln) : 0.f, dt, rdt, m_, MC) * dt - xbZ;
                 const float h = 0.5f * P->pair_skin;
                 far = !(qx * qx + qy * qy + qz * qz <= h * h);
             }
         }
         // a node of this cell leaves the skin next step: the cell is listed for the next
-        // (partial) search, up to the list size (one atomic per such cell); the flag
-        // atomic is skipped once it is visibly set
-        if (far) moved = 1;
-        __syncthreads();
-        if (fused && tid == 0 && moved) {
-            pool_late()->RESET[slot] = 1;
-            if (__hip_atomic_load(&M->search_next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
-                atomicOr(&M->search_next, 1);
-            if (__hip_atomic_load(&M->n_reset, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <= kMaxPartial) {
-                const int k = atomicAdd(&M->n_reset, 1);
-                if (k < kMaxPartial) pool_late()->RSL[MC->base + k] = c;
+        // (partial) search, up to the list size (by the first wave that finds one; one
+        // atomic per such cell); the flag atomic is skipped once it is visibly set
+        if (fused && __any(far)) {
+            const uint64_t fm = __ballot(far);
+            if ((lt & 63) == __ffsll((unsigned long long)fm) - 1 && atomicExch(&moved, 1) == 0) {
+                pool_late()->RESET[slot] = 1;
+                if (__hip_atomic_load(&M->search_next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+                    atomicOr(&M->search_next, 1);
+                if (__hip_atomic_load(&M->n_reset, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <= kMaxPartial) {
+                    const int k = atomicAdd(&M->n_reset, 1);
+                    if (k < kMaxPartial) pool_late()->RSL[MC->base + k] = c;
+                }
             }
         }
-        if (clear_bins && (mode != M_STEP || MC->need_search)) {
+        if (clear_bins && (!kStep || MC->need_search)) {
             // the search of this step is done: this cell's share of the system's
             // search-bin counters (those of the current bin grid, which every
             // insertion since the last clear used) is cleared in one coalesced run
@@ -1682,115 +1787,65 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
             int32_t* counts = pool_late()->bins + MC->bbase;
             for (int64_t b = lo + tid; b < hi; b += blockDim.x) counts[b] = 0;
         }
-        if (fused) {  // this cell's bbox at the end of the step (bounding_boxes, propagatebound.cu:10-141)
-            float b[6] = {node ? X : INFINITY, node ? X : -INFINITY, node ? Y : INFINITY,
-                          node ? Y : -INFINITY, node ? Z : INFINITY, node ? Z : -INFINITY};
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-#pragma unroll
-                for (int a = 0; a < 6; a += 2) {
-                    b[a] = fminf(b[a], __shfl_xor(b[a], o));
-                    b[a + 1] = fmaxf(b[a + 1], __shfl_xor(b[a + 1], o));
-                }
-            }
-            if ((tid & 63) == 0)
-#pragma unroll
-                for (int a = 0; a < 6; ++a) bpart[tid >> 6][a] = b[a];
-        }  // combined after the next barrier
-
-        const bool do_com = mode == M_STEP || mode == M_COM;
         const int64_t stepno = step_override >= 0 ? step_override : MC->step + 1;
-        const bool do_vol =
-            mode == M_VOLUMES || (mode == M_STEP && stepno <= P->div_time_steps && rgrowth(P, MC->n) > 0.0f);
-        if (do_com) {
-            // 256-slot tree of centermass.cu:32-41: levels 128 and 64 through LDS, 32..1 by shuffles
-            if (tid < 128) {
-                const bool hi = tid + 128 < kNodes;
-                red[0][tid] = sx[tid] + (hi ? sx[tid + 128] : 0.0f);
-                red[1][tid] = sy[tid] + (hi ? sy[tid + 128] : 0.0f);
-                red[2][tid] = sz[tid] + (hi ? sz[tid + 128] : 0.0f);
-            }
-            __syncthreads();
-            if (tid < 64) {
-                float a = red[0][tid] + red[0][tid + 64];
-                float b = red[1][tid] + red[1][tid + 64];
-                float d = red[2][tid] + red[2][tid + 64];
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) {
-                    a = a + __shfl_down(a, o);
-                    b = b + __shfl_down(b, o);
-                    d = d + __shfl_down(d, o);
-                }
-                if (tid == 0) {
-                    cm[0] = a / 180.0f; cm[1] = b / 180.0f; cm[2] = d / 180.0f;
-                    const CPool q = pool_late();
-                    q->CMX[slot] = cm[0]; q->CMY[slot] = cm[1]; q->CMZ[slot] = cm[2];
-                }
-            }
-            if (fused && tid < 6) {
-                float b = bpart[0][tid];
-                b = (tid & 1) ? fmaxf(b, bpart[1][tid]) : fminf(b, bpart[1][tid]);
-                b = (tid & 1) ? fmaxf(b, bpart[2][tid]) : fminf(b, bpart[2][tid]);
-                pool_late()->BBOXN[(int64_t)slot * 6 + tid] = b;
-            }
-            __syncthreads();
-        } else if (do_vol) {
-            if (tid == 0) {
-                const CPool q = pool_late();
-                cm[0] = q->CMX[slot]; cm[1] = q->CMY[slot]; cm[2] = q->CMZ[slot];
-            }
-            __syncthreads();
-        }
+        const bool do_vol = mode == M_VOLUMES || (kStep && stepno <= P->div_time_steps && rgrowth(P, MC->n) > 0.0f);
         if (do_vol) {
-            // volume.cu:22-26: local coordinates about the (fresh) centre of mass
-            const float qx = X - cm[0], qy = Y - cm[1], qz = Z - cm[2];
-            __syncthreads();
-            sx[tid] = qx; sy[tid] = qy; sz[tid] = qz;
-            __syncthreads();
             const bool sph = P->check_sphericity != 0;
-            float totvol = 0.f, faceArea = 0.f;
-            if (tid < CS3D_FACES) {  // volume.cu:37-119
-                const uint64_t fw = mesh->face[tid];
-                int rr[7];
-#pragma unroll
-                for (int i = 0; i < 7; ++i) rr[i] = (int)((fw >> (8 * i)) & 0xffu);
+            // volume.cu:22-26: local coordinates about the (fresh) centre of mass
+            const float cx = cm[0], cy = cm[1], cz = cm[2];
+            // volume.cu:37-119, lanes 2f and 2f + 1 on face f: its edges 0..2 and 3..5, the
+            // sums running through both in edge order
+            const int f = lt >> 1, h = lt & 1;
+            float vol[3] = {0.f, 0.f, 0.f}, sq[3] = {0.f, 0.f, 0.f};
+            if (f < CS3D_FACES) {
+                const uint64_t fw = ldu(mesh->face, (uint32_t)f);
                 float avX = 0.0f, avY = 0.0f, avZ = 0.0f;
 #pragma unroll
-                for (int i = 0; i < 5; ++i) { avX += sx[rr[i]]; avY += sy[rr[i]]; avZ += sz[rr[i]]; }
-                float fac = 0.166666667f;
-                if (tid < 12) fac = 0.2f;
-                else { avX += sx[rr[5]]; avY += sy[rr[5]]; avZ += sz[rr[5]]; }
-                avX *= fac; avY *= fac; avZ *= fac;
-#pragma unroll
                 for (int i = 0; i < 6; ++i) {
-                    const int a = rr[i], b = rr[i + 1];
-                    const float n1 = (sy[b] * avZ - avY * sz[b]) * sx[a];
-                    const float n2 = (sz[b] * avX - avZ * sx[b]) * sy[a];
-                    const float n3 = (sx[b] * avY - avX * sy[b]) * sz[a];
-                    totvol += fabsf(n1 + n2 + n3);
+                    const int n = (int)((fw >> (8 * i)) & 0xffu);
+                    if (i < 5 || f >= 12) { avX += sx[n] - cx; avY += sy[n] - cy; avZ += sz[n] - cz; }
+                }
+                const float fac = f < 12 ? 0.2f : 0.166666667f;
+                avX *= fac; avY *= fac; avZ *= fac;
+                const uint32_t ew = (uint32_t)(fw >> (24 * h));  // entries 3 h .. 3 h + 3
+                float ax, ay, az, bx, by, bz;
+                {
+                    const int n = (int)(ew & 0xffu);
+                    bx = sx[n] - cx; by = sy[n] - cy; bz = sz[n] - cz;
+                }
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    ax = bx; ay = by; az = bz;
+                    const int n = (int)((ew >> (8 * (i + 1))) & 0xffu);
+                    bx = sx[n] - cx; by = sy[n] - cy; bz = sz[n] - cz;
+                    const float n1 = (by * avZ - avY * bz) * ax;
+                    const float n2 = (bz * avX - avZ * bx) * ay;
+                    const float n3 = (bx * avY - avX * by) * az;
+                    vol[i] = fabsf(n1 + n2 + n3);
                     if (sph) {
-                        const float x1 = sx[a] - avX, y1 = sy[a] - avY, z1 = sz[a] - avZ;
-                        const float x2 = sx[b] - avX, y2 = sy[b] - avY, z2 = sz[b] - avZ;
+                        const float x1 = ax - avX, y1 = ay - avY, z1 = az - avZ;
+                        const float x2 = bx - avX, y2 = by - avY, z2 = bz - avZ;
                         const float xx = y1 * z2 - z1 * y2, yy = z1 * x2 - x1 * z2, zz = x1 * y2 - y1 * x2;
-                        faceArea = (float)((double)faceArea + 0.5 * (double)sqrt_cr(xx * xx + yy * yy + zz * zz));
+                        sq[i] = sqrt_cr(xx * xx + yy * yy + zz * zz);
                     }
                 }
             }
-            // canonical 128-slot tree over the faces (faces >= 92 contribute 0)
-            if (tid < 128) {
-                red[0][tid] = tid < CS3D_FACES ? totvol : 0.0f;
-                red[1][tid] = tid < CS3D_FACES ? faceArea : 0.0f;
-            }
-            __syncthreads();
-            if (tid < 64) {
-                float a = red[0][tid] + red[0][tid + 64];
-                float b = red[1][tid] + red[1][tid + 64];
+            auto sum3 = [](float v, const float* e) { return ((v + e[0]) + e[1]) + e[2]; };
+            auto area3 = [](float a, const float* e) {
 #pragma unroll
-                for (int o = 32; o > 0; o >>= 1) {
-                    a = a + __shfl_down(a, o);
-                    b = b + __shfl_down(b, o);
-                }
-                if (tid == 0) {  // volume.cu:129-161
+                for (int i = 0; i < 3; ++i) a = (float)((double)a + 0.5 * (double)e[i]);
+                return a;
+            };
+            const float totvol = sum3(even_lane(sum3(0.f, vol)), vol);  // the odd lane's is the face's
+            const float faceArea = area3(even_lane(area3(0.f, sq)), sq);
+            // canonical 128-slot tree over the faces (faces >= 92 contribute 0)
+            if (h == 1 && f < CS3D_FACES) { red[0][f] = totvol; red[1][f] = faceArea; }
+            if (lt < 128 - CS3D_FACES) { red[0][CS3D_FACES + lt] = 0.0f; red[1][CS3D_FACES + lt] = 0.0f; }
+            __syncthreads();
+            if (wv == 0) {
+                const float a = wave_tree<OpAdd>(red[0][lt] + red[0][lt + 64]);
+                const float b = wave_tree<OpAdd>(red[1][lt] + red[1][lt + 64]);
+                if (lt == 0) {  // volume.cu:129-161
                     const float volume = (float)((double)a / 6.0);
                     pool_late()->VOL[slot] = volume;
                     if (!isfinite(volume)) st |= CS3D_SYS_VOLUME_NONFINITE;
@@ -2433,6 +2488,26 @@ __global__ __launch_bounds__(192) void k_grid_adopt(Pool p, Range r) {
     }
 }
 
+// The partner lists that callers read (CS3D_F_PAIRS, CS3D_F_PAIRCOUNT): each live
+// node's accepted candidates, ascending, k-major per cell.
+__global__ __launch_bounds__(192) void k_pairs_list(Pool p, Range r) {
+    const int tid = threadIdx.x;
+    for (int slot = r.slot_lo + blockIdx.x; slot < r.slot_hi; slot += gridDim.x) {
+        const int s = sys_of(p, r, slot);
+        if (s < 0 || tid >= kNodes) continue;
+        const SysMeta* M = p.meta + s;
+        if (slot - M->base >= M->n) continue;
+        const int ncf = p.NCAND[(int64_t)slot * kSlots + tid];
+        const int nc = ncf & ((1 << kCandBits) - 1), first = ncf >> kCandBits;
+        const int32_t* cand = p.CAND + (int64_t)slot * kPMax * kSlots;
+        const uint64_t* mask = pair_mask(p.CAND, slot);
+        int np = 0;
+        for (int j = first; j < first + nc; ++j)
+            if (mask[j >> 6] >> (j & 63) & 1) p.PAIRS[((int64_t)slot * kPMax + np++) * kSlots + tid] = cand[j];
+        p.NPAIR[(int64_t)slot * kSlots + tid] = np;
+    }
+}
+
 // voxel ranges of the current bboxes (after a caller sets BBOX or the grid)
 __global__ void k_vrange(Pool p, Range r) {
     for (int slot = r.slot_lo + blockIdx.x * blockDim.x + threadIdx.x; slot < r.slot_hi;
@@ -2696,12 +2771,13 @@ void launch_dis(const Pool& p, const Range& r, int mode, int64_t step_override, 
     const float* vx = use_va ? p.VAX : p.VX;
     const float* vy = use_va ? p.VAY : p.VY;
     const float* vz = use_va ? p.VAZ : p.VZ;
-    if (r.live)
-        launch(k_dis_post<1>, dim3(grid_cells(r, p.wg_per_cu)), dim3(192), st, p, r, mode, step_override, clear_bins,
-                               p.X, p.Y, p.Z, vx, vy, vz);
+    const dim3 grid(grid_cells(r, p.wg_per_cu)), block(192);
+    if (mode != M_STEP)  // one system
+        launch(k_dis_post<0, false>, grid, block, st, p, r, mode, step_override, clear_bins, p.X, p.Y, p.Z, vx, vy, vz);
+    else if (r.live)
+        launch(k_dis_post<1, true>, grid, block, st, p, r, mode, step_override, clear_bins, p.X, p.Y, p.Z, vx, vy, vz);
     else
-        launch(k_dis_post<0>, dim3(grid_cells(r, p.wg_per_cu)), dim3(192), st, p, r, mode, step_override, clear_bins,
-                               p.X, p.Y, p.Z, vx, vy, vz);
+        launch(k_dis_post<0, true>, grid, block, st, p, r, mode, step_override, clear_bins, p.X, p.Y, p.Z, vx, vy, vz);
 }
 void launch_divide(const Pool& p, const Range& r, int mode, hipStream_t st) {
     const int ns = r.sys_hi - r.sys_lo;
@@ -2733,6 +2809,9 @@ void launch_vox_lists(const Pool& p, const Range& r, int vox_blocks, hipStream_t
     launch(k_vox_clear, dim3(vox_blocks, ns > 0 ? ns : 1), dim3(256), st, p, r);
     launch(k_insert, dim3(cb > 0 ? cb : 1), dim3(256), st, p, r, 1);
     launch(k_sort, dim3(vox_blocks, ns > 0 ? ns : 1), dim3(256), st, p, r, 1);
+}
+void launch_pairs_list(const Pool& p, const Range& r, hipStream_t st) {
+    launch(k_pairs_list, dim3(grid_cells(r, p.wg_per_cu)), dim3(192), st, p, r);
 }
 void launch_velocity_ab(const Pool& p, const Range& r, int which, hipStream_t st) {
     launch(k_velocity_ab, dim3(grid_cells(r, p.wg_per_cu)), dim3(192), st, p, r, which);
