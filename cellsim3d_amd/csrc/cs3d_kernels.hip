@@ -392,7 +392,14 @@ __device__ __forceinline__ void store_vrange(int32_t* vrange, int64_t slot, cons
 // pair_skin so that every pair within that range lies in adjacent bins, two bins
 // of margin, coarser when the extent outgrows the bin budget).  Returns the
 // number of voxel counters to clear.  Called by one thread.
-__device__ int64_t set_grid_geometry(SysMeta* M, const cs3d_params* P, const float* e) {
+struct GridConsts {  // what set_grid_geometry needs of the parameters and metadata
+    float DL, ar, skin;
+    int32_t vbudget, bbudget;
+};
+template <class MP, class PP> __device__ __forceinline__ GridConsts grid_consts(MP M, PP P) {
+    return GridConsts{P->grid_dl, P->attraction_range, P->pair_skin, M->vbudget, M->bbudget};
+}
+__device__ __forceinline__ int64_t set_grid_geometry(SysMeta* M, const GridConsts& k, const float* e) {
     if (!(e[1] >= e[0] && e[3] >= e[2] && e[5] >= e[4])) {
         // no cells (the extent kept its sentinels): a one-voxel grid, nothing to flag
         for (int a = 0; a < 3; ++a) {
@@ -401,18 +408,18 @@ __device__ int64_t set_grid_geometry(SysMeta* M, const cs3d_params* P, const flo
         }
         return 1;
     }
-    const float DL = P->grid_dl;
+    const float DL = k.DL;
     const int xd = (int)((e[1] - e[0]) / DL + 1.0f);
     const int yd = (int)((e[3] - e[2]) / DL + 1.0f);
     const int zd = (int)((e[5] - e[4]) / DL + 1.0f);
     const int64_t nv = (int64_t)xd * yd * zd;
-    const bool ok = xd > 0 && yd > 0 && zd > 0 && nv <= M->vbudget;
+    const bool ok = xd > 0 && yd > 0 && zd > 0 && nv <= k.vbudget;
     M->gmin[0] = e[0]; M->gmin[1] = e[2]; M->gmin[2] = e[4];
     M->dims[0] = ok ? xd : 1; M->dims[1] = ok ? yd : 1; M->dims[2] = ok ? zd : 1;
     if (!ok) atomicOr(&M->status, (uint32_t)CS3D_SYS_GRID_TOO_LARGE);
     // search bins of edge attraction_range + pair_skin covering the extent, or
     // fewer along the longest axes when the budget is short (periodic bins)
-    float h = (P->attraction_range + P->pair_skin) * 1.001f;
+    float h = (k.ar + k.skin) * 1.001f;
     if (!(h > 0.f)) h = 1.0f;
     const float sz[3] = {e[1] - e[0], e[3] - e[2], e[5] - e[4]};
     int bd[3];
@@ -421,7 +428,7 @@ __device__ int64_t set_grid_geometry(SysMeta* M, const cs3d_params* P, const flo
         bd[a] = (q >= 0.f && q < 1.0e6f) ? (int)q + 5 : 1000000;
     }
     for (int it = 0; it < 200; ++it) {
-        if ((int64_t)bd[0] * bd[1] * bd[2] <= M->bbudget) break;
+        if ((int64_t)bd[0] * bd[1] * bd[2] <= k.bbudget) break;
         const int a = bd[0] >= bd[1] && bd[0] >= bd[2] ? 0 : (bd[1] >= bd[2] ? 1 : 2);
         bd[a] = max(3, (int)(bd[a] * 0.9f));
     }
@@ -430,7 +437,7 @@ __device__ int64_t set_grid_geometry(SysMeta* M, const cs3d_params* P, const flo
         M->bdims[a] = bd[a];
     }
     M->bh = h;
-    return ok ? nv : (int64_t)M->vbudget;
+    return ok ? nv : (int64_t)k.vbudget;
 }
 
 // {minx, maxx, miny, maxy, minz, maxz} of the node positions of one cell
@@ -514,6 +521,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
         const int c = slot - MC->base;
         if (c >= MC->n) continue;
         const CPool q = pool_late();  // pointers read again where used (see pool_late)
+        bool over = false;  // a voxel count beyond its capacity: looked at after the kick, which need not wait for it
         if ((flags & I_GRIDCOUNT) && MC->rebuild && !(MC->status & CS3D_SYS_GRID_TOO_LARGE)) {
             // the grid was rebuilt at the end of the last step: this cell's new bbox
             // becomes the one the contact rule uses, and its voxels are counted
@@ -529,13 +537,10 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
             const int total = (nx > 0 && ny > 0 && nz > 0) ? nx * ny * nz : 0;
             int32_t* counts = q->vox + MC->vbase;
             const int xd = MC->dims[0], yd = MC->dims[1], cap = MC->vcap;
-            bool over = false;
             for (int t = tid; t < total; t += blockDim.x) {
                 const int j3 = v.sz + t % nz, j2 = v.sy + (t / nz) % ny, j1 = v.sx + t / (nz * ny);
                 if (atomicAdd(&counts[j3 * xd * yd + j2 * xd + j1], 1) >= cap) over = true;
             }
-            if (__any(over) && (tid & 63) == __ffsll((unsigned long long)__ballot(over)) - 1)
-                atomicOr(&M->status, (uint32_t)CS3D_SYS_VOXEL_OVERFLOW);
         }
         if (node && kick) {
             const float dt = P->dt, m = P->mass;
@@ -594,6 +599,8 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
             }
             q->P[slot] = pr;
         }
+        if (__any(over) && (tid & 63) == __ffsll((unsigned long long)__ballot(over)) - 1)
+            atomicOr(&M->status, (uint32_t)CS3D_SYS_VOXEL_OVERFLOW);
         if (kick && (flags & I_IFSEARCH) && MC->need_search == 2 && q->RESET[slot]) {
             // a cell that divided or left the skin in the last step publishes the box of
             // its new positions: the partial search re-searches the cells within reach
@@ -1982,6 +1989,8 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
     const int64_t div_time = PC->div_time_steps;
     const int32_t m_gint = PC->grid_interval, m_ccom = PC->correct_com;
     const float m_rgrowth = rgrowth(PC, n0);
+    const GridConsts m_grid = grid_consts(MC, PC);
+    const int64_t m_vbase = MC->vbase;
     const bool live = m_active && (m_horizon < 0 || m_step < m_horizon) && !(m_status & CS3D_SYS_FATAL_MASK);
     // a stopped system keeps a pending grid adoption: its bboxes are adopted when it
     // resumes or when a caller reads the grid
@@ -1994,8 +2003,45 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
     bool growth = true;
     if (step_mode) growth = stepno <= div_time && m_rgrowth > 0.0f;
     if (tid == 0) { nev = 0; ncur = n0; stop = 0; bad = 0; }
-    __syncthreads();
+    // whether any cell divides: most steps of a growing tissue have no event, and need
+    // none of the list's scans and barriers.  The boxes that a rebuild without events
+    // needs are loaded beside the flags.
+    constexpr int kUnroll = 8;  // boxes per thread and pass of the extent
+    float bb[kUnroll][6];
+    const int gint = m_gint > 0 ? m_gint : 1;
+    const bool due = step_mode && stepno % gint == 0;
+    auto load_boxes = [&](int c0, int n) {
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            const float2* b = reinterpret_cast<const float2*>(p.BBOXN + (int64_t)(base + min(c0 + u * 256 + tid, n - 1)) * 6);
+            const float2 b0 = b[0], b1 = b[1], b2 = b[2];
+            bb[u][0] = b0.x; bb[u][1] = b0.y; bb[u][2] = b1.x; bb[u][3] = b1.y; bb[u][4] = b2.x; bb[u][5] = b2.y;
+        }
+    };
+    if (due && n0 > 0) load_boxes(0, n0);
+    bool any = false;
     if (growth) {
+        // 16 flags per load between the 16-byte boundaries, the rest one by one
+        const int8_t* F = p.FLAG + base;
+        const int head = min(n0, (int)(-(uint32_t)base & 15u)), vecs = (n0 - head) >> 4, tail = head + 16 * vecs;
+        const uint4* v = reinterpret_cast<const uint4*>(F + head);
+        auto one = [](uint32_t w) {  // whether a byte of w is 1 (the zero-byte test on w ^ 0x01010101)
+            const uint32_t x = w ^ 0x01010101u;
+            return ((x - 0x01010101u) & ~x & 0x80808080u) != 0;
+        };
+        constexpr int kVec = 4;  // loads in flight per thread
+        for (int i = tid; i < vecs; i += kVec * 256) {
+            uint4 w[kVec];
+#pragma unroll
+            for (int u = 0; u < kVec; ++u) w[u] = i + u * 256 < vecs ? v[i + u * 256] : make_uint4(0, 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < kVec; ++u) any |= one(w[u].x) | one(w[u].y) | one(w[u].z) | one(w[u].w);
+        }
+        if (tid < head) any |= F[tid] == 1;
+        if (tail + tid < n0) any |= F[tail + tid] == 1;
+    }
+    any = __syncthreads_or(any);
+    if (any) {
         // ascending event list in EVL[base .. base + nev), 4096 cells per pass: each
         // thread loads the flags of 16 consecutive cells at once and counts them, a scan
         // of the counts (shuffles within a wave, then the four wave totals) gives the
@@ -2131,30 +2177,21 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
             }
         }
     }
-    __syncthreads();
+    if (any) __syncthreads();
     const int events = ncur - n0;
-    const int gint = m_gint > 0 ? m_gint : 1;
-    const bool rebuild = step_mode && (events > 0 || stepno % gint == 0);
+    const bool rebuild = step_mode && (events > 0 || due);
     if (rebuild) {
         // grid rebuild from the end-of-step bboxes: minmaxpre/minmaxpost
         // (propagatebound.cu:145-204, 266-323, sentinels +-1e8) and the grid
         // geometry; the per-cell part (bbox adoption, voxel counts) is done by the
         // next step's Integrate
-        float e[12];
+        float e[6];
 #pragma unroll
-        for (int a = 0; a < 12; a += 2) { e[a] = 1.0E8f; e[a + 1] = -1.0E8f; }
+        for (int a = 0; a < 6; a += 2) { e[a] = 1.0E8f; e[a + 1] = -1.0E8f; }
         // the boxes of 8 cells per thread are loaded before any is reduced (min and max
         // are exact in any order)
-        constexpr int kUnroll = 8;
         for (int c0 = 0; c0 < ncur; c0 += kUnroll * 256) {
-            float bb[kUnroll][6];
-#pragma unroll
-            for (int u = 0; u < kUnroll; ++u) {
-                const int c = c0 + u * 256 + tid;
-                const float* b = p.BBOXN + (int64_t)(base + min(c, ncur - 1)) * 6;
-#pragma unroll
-                for (int a = 0; a < 6; ++a) bb[u][a] = b[a];
-            }
+            if (c0 > 0 || events > 0 || !due) load_boxes(c0, ncur);
 #pragma unroll
             for (int u = 0; u < kUnroll; ++u) {
                 if (c0 + u * 256 + tid < ncur) {
@@ -2166,10 +2203,23 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
                 }
             }
         }
-        block_minmax12(e, mpart, mres);
-        if (tid == 0) nclear = set_grid_geometry(M, P, mres);
+#pragma unroll
+        for (int a = 0; a < 6; a += 2) {
+            const float lo = wave_tree<OpMin>(e[a]), hi = wave_tree<OpMax>(e[a + 1]);
+            if ((tid & 63) == 0) { mpart[tid >> 6][a] = lo; mpart[tid >> 6][a + 1] = hi; }
+        }
         __syncthreads();
-        int32_t* counts = p.vox + M->vbase;
+        if (tid == 0) {
+            float x[6];
+#pragma unroll
+            for (int a = 0; a < 6; a += 2) {
+                x[a] = fminf(fminf(mpart[0][a], mpart[1][a]), fminf(mpart[2][a], mpart[3][a]));
+                x[a + 1] = fmaxf(fmaxf(mpart[0][a + 1], mpart[1][a + 1]), fmaxf(mpart[2][a + 1], mpart[3][a + 1]));
+            }
+            nclear = set_grid_geometry(M, m_grid, x);
+        }
+        __syncthreads();
+        int32_t* counts = p.vox + m_vbase;
         for (int64_t v = tid; v < nclear; v += blockDim.x) counts[v] = 0;
     }
     const bool shift = step_mode && m_ccom;
@@ -2177,7 +2227,7 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
         // calc_sys_CM (GPUbounce.cu:2504-2520): float sums of the cell centres in
         // cell order (daughters of this step still hold 0), divided by the count;
         // the nodes are shifted by k_com_shift (CorrectCoMMotion, propagate.cu:766-776)
-        float acc[3] = {0.f, 0.f, 0.f};
+        float acc = 0.f;  // lanes 0..2: one component each
         for (int c0 = 0; c0 < ncur; c0 += 128) {
             if (tid < 128 && c0 + tid < ncur) {
                 redc[0][tid] = p.CMX[base + c0 + tid];
@@ -2186,12 +2236,21 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
             }
             __syncthreads();
             if (tid < 3) {
+                // (the reads of 16 centres ahead of their sequential sum)
                 const int m = min(128, ncur - c0);
-                for (int k = 0; k < m; ++k) acc[tid] = acc[tid] + redc[tid][k];
+                int k = 0;
+                for (; k + 16 <= m; k += 16) {
+                    float v[16];
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) v[j] = redc[tid][k + j];
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) acc = acc + v[j];
+                }
+                for (; k < m; ++k) acc = acc + redc[tid][k];
             }
             __syncthreads();
         }
-        if (tid < 3) M->sys_cm[tid] = acc[tid] / (float)ncur;
+        if (tid < 3) M->sys_cm[tid] = acc / (float)ncur;
     }
     if (tid == 0) {
         M->shift_pending = shift ? 1 : 0;
@@ -2411,7 +2470,7 @@ __global__ __launch_bounds__(256) void k_grid_dims(Pool p, Range r) {
     int32_t* counts = p.vox + M->vbase;
     for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nclear; v += (int64_t)gridDim.x * blockDim.x)
         counts[v] = 0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) (void)set_grid_geometry(M, P, e);
+    if (blockIdx.x == 0 && threadIdx.x == 0) (void)set_grid_geometry(M, grid_consts(M, P), e);
 }
 
 // force = 1: fill the lists of the current grid whatever the rebuild flag says

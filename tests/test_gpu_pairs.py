@@ -89,3 +89,34 @@ def test_deformed_cells_match_oracle(oracle_mesh, scale, bond):
                 A[k][0, i] = A[k][0, m["nn"][i, 0]] + np.float32(bond)
     # one step: the strongly deformed ones move far, and both sides with them
     _run(oracle_mesh, A[0].reshape(-1), A[1].reshape(-1), A[2].reshape(-1), 2, 0.05, 1, 7)
+
+
+# the flag test of the division phase reads 16 flags at a time between 16-byte
+# boundaries: rooms that start at any of them, counts around them, and flag values
+# other than 1, which are no event (d_cell_div, GPUbounce.cu:2489-2500)
+@pytest.mark.parametrize("offset", [0, 1, 7, 15])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 33, 70])
+def test_every_flagged_cell_divides(oracle_mesh, n, offset):
+    from cellsim3d_amd import abi as A
+    from cellsim3d_amd import configs, engine
+    print("flags: %d cells from slot %d" % (n, offset), flush=True)
+    _, X, Y, Z, _ = configs.lattice_tissue(n, 0.2, seed=n)
+    p = configs.base_params(2)
+    p.voxel_capacity = 64
+    with engine.Context(oracle_mesh, capacity_cells=offset + 2 * n, voxel_budget=1 << 21, bin_budget=1 << 23) as ctx:
+        if offset:
+            ctx.add_system_raw(p, 0, max_cells=offset, voxels=1)
+        for cells in ([], [0], [n - 1], [n // 2], sorted({0, n // 3, n - 1})):
+            s = ctx.add_system(p, X, Y, Z, n, max_cells=2 * n, voxels=1 << 12)
+            flags = np.zeros(2 * n, np.int8)
+            flags[:n:2] = 2
+            flags[1:n:2] = -1
+            flags[n:] = 1  # past the live cells
+            for c in cells:
+                flags[c] = 1
+            s.set(A.F_DIVFLAG, flags)
+            assert s.k_divide() == len(cells)
+            assert s.info()[0] == n + len(cells)
+            moved = np.flatnonzero((s.get(A.F_X)[:n * 192].reshape(n, 192) != X.reshape(n, 192)).any(1))
+            assert moved.tolist() == cells
+            s.remove()
