@@ -170,6 +170,15 @@ struct Range {
     int32_t live;     // 1: the cell kernels walk Pool::LIVE (built by k_live) instead of the slots
 };
 
+// Pieces of device memory that one launch copies into a buffer (k_gather).
+constexpr int kMaxGather = 16;
+struct GatherList {
+    const uint32_t* src[kMaxGather];
+    uint32_t dst[kMaxGather];    // first word in the buffer, a multiple of 4
+    uint32_t words[kMaxGather];
+    int32_t n;
+};
+
 // kernel modes
 enum : int32_t {
     M_STEP = 0,        // fused step path (state flags decided on the device)

@@ -2035,7 +2035,7 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
 #pragma unroll
             for (int u = 0; u < kVec; ++u) w[u] = i + u * 256 < vecs ? v[i + u * 256] : make_uint4(0, 0, 0, 0);
 #pragma unroll
-            for (int u = 0; u < kVec; ++u) any |= one(w[u].x) | one(w[u].y) | one(w[u].z) | one(w[u].w);
+            for (int u = 0; u < kVec; ++u) any = any || one(w[u].x) || one(w[u].y) || one(w[u].z) || one(w[u].w);
         }
         if (tid < head) any |= F[tid] == 1;
         if (tail + tid < n0) any |= F[tail + tid] == 1;
@@ -2746,6 +2746,19 @@ __global__ __launch_bounds__(256) void k_copy_calibrate(const float4* __restrict
         dst[i] = src[i];
 }
 
+// Copies the pieces of a list into dst (pinned host memory): 16 bytes per lane where
+// the source allows, the host link's width is reached with 64 workgroups.
+__global__ __launch_bounds__(256) void k_gather(GatherList g, uint32_t* __restrict__ dst) {
+    const uint32_t t0 = blockIdx.x * blockDim.x + threadIdx.x, nt = gridDim.x * blockDim.x;
+    for (int k = 0; k < g.n; ++k) {
+        const uint32_t* s = g.src[k];
+        uint32_t* d = dst + g.dst[k];
+        const uint32_t n = g.words[k], n4 = (reinterpret_cast<uintptr_t>(s) & 15) ? 0 : n / 4;
+        for (uint32_t i = t0; i < n4; i += nt) reinterpret_cast<uint4*>(d)[i] = reinterpret_cast<const uint4*>(s)[i];
+        for (uint32_t i = 4 * n4 + t0; i < n; i += nt) d[i] = s[i];
+    }
+}
+
 // sets the grid-rebuild and candidate-search flags of systems (-1 = unchanged)
 __global__ void k_set_flags(Pool p, Range r, int32_t rebuild, int32_t search) {
     const int s = r.sys_lo + blockIdx.x * blockDim.x + threadIdx.x;
@@ -2871,6 +2884,12 @@ void launch_vox_lists(const Pool& p, const Range& r, int vox_blocks, hipStream_t
 }
 void launch_pairs_list(const Pool& p, const Range& r, hipStream_t st) {
     launch(k_pairs_list, dim3(grid_cells(r, p.wg_per_cu)), dim3(192), st, p, r);
+}
+void launch_gather(const GatherList& g, void* dst, hipStream_t st) {
+    uint64_t words = 0;
+    for (int k = 0; k < g.n; ++k) words += g.words[k];
+    const uint64_t b = (words + 1023) / 1024;  // one 16-byte store per thread up to 512 workgroups
+    launch(k_gather, dim3(b < 1 ? 1 : (b < 512 ? (uint32_t)b : 512)), dim3(256), st, g, (uint32_t*)dst);
 }
 void launch_velocity_ab(const Pool& p, const Range& r, int which, hipStream_t st) {
     launch(k_velocity_ab, dim3(grid_cells(r, p.wg_per_cu)), dim3(192), st, p, r, which);

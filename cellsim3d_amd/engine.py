@@ -345,7 +345,7 @@ class System:
             return st
         nbytes = lib().cs3d_field_bytes(self.ctx.h, self.id, f)
         dt = np.dtype(self._dtype(f))
-        out = np.zeros(nbytes // dt.itemsize, dtype=dt)
+        out = np.empty(nbytes // dt.itemsize, dtype=dt)  # filled whole
         check(lib().cs3d_get(self.ctx.h, self.id, f, out.ctypes.data_as(vp), out.nbytes), "cs3d_get")
         return out
 
@@ -408,10 +408,10 @@ class System:
     def get_state(self):
         """Positions, velocities (each (3, n*192)), pressure, centres (3, n), volumes, n and status."""
         n = self.info()[0]
-        xyz = np.zeros((3, n * 192), np.float32)
-        v = np.zeros((3, n * 192), np.float32)
-        P, V = np.zeros(n, np.float32), np.zeros(n, np.float32)
-        CM = np.zeros((3, n), np.float32)
+        xyz = np.empty((3, n * 192), np.float32)  # filled whole
+        v = np.empty((3, n * 192), np.float32)
+        P, V = np.empty(n, np.float32), np.empty(n, np.float32)
+        CM = np.empty((3, n), np.float32)
         nc, st = C.c_int32(), C.c_uint32()
         check(lib().cs3d_get_state(self.ctx.h, self.id, xyz.ctypes.data_as(vp), v.ctypes.data_as(vp),
                                    P.ctypes.data_as(vp), CM.ctypes.data_as(vp), V.ctypes.data_as(vp),

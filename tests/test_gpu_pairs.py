@@ -1,9 +1,11 @@
-"""The contact pass of k_con_dis where its work lists can go wrong, bit for bit
-against the oracle through the C ABI: no candidates at all, one round (at most 192
+"""Paths whose form depends on sizes, through the C ABI.
+
+The contact pass of k_con_dis where its work lists can go wrong, bit for bit
+against the oracle: no candidates at all, one round (at most 192
 pairs per cell), several rounds, nodes whose candidates straddle a round or a
 64-lane word, and lists near the 40-entry limit; and the bonds and angles at the
 edges of the short arithmetic (rest shape, crushed, stretched, bonds at and below
-its range)."""
+its range); the division phase's flag test; reads of device memory."""
 import numpy as np
 import pytest
 
@@ -120,3 +122,47 @@ def test_every_flagged_cell_divides(oracle_mesh, n, offset):
             moved = np.flatnonzero((s.get(A.F_X)[:n * 192].reshape(n, 192) != X.reshape(n, 192)).any(1))
             assert moved.tolist() == cells
             s.remove()
+
+
+# reads below, between and above the sizes where the way back changes (56 KB, 1 MB,
+# the 2 MB slots and the ring of four), odd lengths among them
+@pytest.mark.parametrize("n", [1, 3, 70, 73, 76, 700, 1400, 3001])
+def test_reads_return_what_was_written(oracle_mesh, n):
+    from cellsim3d_amd import abi as A
+    from cellsim3d_amd import configs, engine
+    print("reads of %d cells" % n, flush=True)
+    L = engine.lib()
+    p = configs.base_params(2)
+    rng = np.random.default_rng(n)
+    with engine.Context(oracle_mesh, capacity_cells=n + 3, voxel_budget=1 << 20, bin_budget=1 << 23) as ctx:
+        ctx.add_system_raw(p, 0, max_cells=2, voxels=1)
+        s = ctx.add_system_raw(p, n, max_cells=n + 1, voxels=16)
+        want = {}
+        for f in (A.F_X, A.F_Y, A.F_Z, A.F_VX, A.F_VY, A.F_VZ):
+            want[f] = rng.random((n + 1) * 192).astype(np.float32)
+            s.set(f, want[f])
+        for f in (A.F_PRESSURE, A.F_CMX, A.F_CMY, A.F_CMZ, A.F_VOLUME):
+            want[f] = rng.random(n + 1).astype(np.float32)
+            s.set(f, want[f])
+        flags = rng.integers(-3, 3, n + 1).astype(np.int8)
+        s.set(A.F_DIVFLAG, flags)
+        for f, w in want.items():
+            assert np.array_equal(s.get(f), w), f
+        assert np.array_equal(s.get(A.F_DIVFLAG), flags)
+        for nb in (1, 4, 7, 4 * (n * 96 + 1)):  # parts of a field
+            part = np.full(4 * (n + 1) * 192, 77, np.uint8)
+            engine.check(L.cs3d_get(ctx.h, s.id, A.F_Y, part.ctypes.data, nb), "cs3d_get")
+            assert np.array_equal(part[:nb], want[A.F_Y].view(np.uint8)[:nb]) and np.all(part[nb:] == 77)
+        st = s.get_state()
+        assert st["n"] == n and st["status"] == 0
+        for k, f in enumerate((A.F_X, A.F_Y, A.F_Z)):
+            assert np.array_equal(st["xyz"][k], want[f][:n * 192])
+        for k, f in enumerate((A.F_VX, A.F_VY, A.F_VZ)):
+            assert np.array_equal(st["v"][k], want[f][:n * 192])
+        for k, f in enumerate((A.F_CMX, A.F_CMY, A.F_CMZ)):
+            assert np.array_equal(st["CM"][k], want[f][:n])
+        assert np.array_equal(st["P"], want[A.F_PRESSURE][:n]) and np.array_equal(st["V"], want[A.F_VOLUME][:n])
+        # without some of the outputs
+        P = np.zeros(n, np.float32)
+        engine.check(L.cs3d_get_state(ctx.h, s.id, None, None, P.ctypes.data, None, None, None, None), "cs3d_get_state")
+        assert np.array_equal(P, want[A.F_PRESSURE][:n])
