@@ -148,8 +148,9 @@ struct Pool {
     int8_t* RESET;   // int8[cap_cells]: 1 = the cell takes its current positions as search positions at
                      // the next partial search (a node left the skin, or the cell divided)
     int32_t* RSL;    // int32[cap_cells]: per system, the local indices of its RESET cells (n_reset)
-    int32_t* LIVE;   // int32[cap_cells]: live cell slots of the stepped systems (k_live)
-    int32_t* n_live; // int32[1]: entries of LIVE
+    int2* LIVE;      // {slot, system}[cap_cells]: live cells of the stepped systems (k_live)
+    int2* SRCH;      // {slot, system}[cap_cells]: those of them whose system searches in this step
+    int32_t* n_live; // int32[2]: entries of LIVE and SRCH
     int32_t* EVL;
     int32_t* slot_sys;
     int32_t* nsys;   // int32[1]: system ids in use are below this (kernels over all systems read it, so a

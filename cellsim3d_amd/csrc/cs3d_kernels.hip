@@ -200,12 +200,16 @@ __device__ __forceinline__ CPool pool_late() {
     return q;
 }
 
-// The cell slot of loop iteration `it` of a cell kernel, made wave-uniform with
-// readfirstlane: the per-cell base pointers derived from it stay in scalar
-// registers instead of becoming per-lane 64-bit induction variables.
+// The cell slot and system of loop iteration `it` of a cell kernel: an entry of a
+// list made by k_live (a multi-system step), read with one scalar load, or the
+// it-th slot of the range.  Wave-uniform: the per-cell base pointers derived from
+// the slot stay in scalar registers instead of becoming per-lane 64-bit induction
+// variables.
 template <int kLive>
-__device__ __forceinline__ int cell_slot(const Pool& p, const Range& r, int it) {
-    return __builtin_amdgcn_readfirstlane(kLive ? p.LIVE[it] : r.slot_lo + it);
+__device__ __forceinline__ int2 cell_at(const Pool& p, const Range& r, const int2* list, int it) {
+    if (kLive) return int2{cld(&list[it].x), cld(&list[it].y)};
+    const int slot = __builtin_amdgcn_readfirstlane(r.slot_lo + it);
+    return int2{slot, __builtin_amdgcn_readfirstlane(sys_of(p, r, slot))};
 }
 
 // The lane's node index as a value the compiler cannot see through (an empty asm
@@ -494,9 +498,10 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
     const int tid = threadIdx.x;
     const bool node = tid < kNodes;
     // a multi-system step walks the compact list of live slots (k_live)
-    const int nit = kLive ? *p.n_live : r.slot_hi - r.slot_lo;
+    const int nit = kLive ? cld(p.n_live) : r.slot_hi - r.slot_lo;
     for (int it = xcd_block(); it < nit; it += gridDim.x) {
-        const int slot = kLive ? p.LIVE[it] : r.slot_lo + it;
+        const int2 at = cell_at<kLive>(p, r, p.LIVE, it);
+        const int slot = at.x, s = at.y;
         // the cell's node data are loaded before the system checks (every slot of the
         // range is allocated), so their latency overlaps the metadata reads
         // (plain 64-bit node indices here: measured faster for this short kernel than
@@ -510,7 +515,6 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
             fcx = p.FCX[gi]; fcy = p.FCY[gi]; fcz = p.FCZ[gi];
             fdx = p.FDX[gi]; fdy = p.FDY[gi]; fdz = p.FDZ[gi];
         }
-        const int s = sys_of(p, r, slot);
         if (s < 0) continue;
         // metadata and parameters through scalar loads: this kernel writes no field it
         // reads (only status bits, by atomics)
@@ -1031,7 +1035,8 @@ __device__ __forceinline__ void pair_pass(const int32_t* cand, uint64_t* mask, P
 // moved pair_skin/2 since the last search (or always, outside the fused step),
 // rebuild each node's sorted candidate list and remember the positions.
 // ------------------------------------------------------------------------------
-// kLive: walk Pool::LIVE (a multi-system step) instead of the range's slots
+// kLive: walk Pool::SRCH (a multi-system step: the cells of the systems that search)
+// instead of the range's slots
 template <int kLive>
 __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always) {
     __shared__ int32_t lst[kPMax][kSlots];
@@ -1044,11 +1049,11 @@ __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always)
         const CMeta M0 = cmeta(p.meta + r.sys_lo);
         if (!M0->need_search || !sys_live(M0)) return;
     }
-    // a multi-system step walks the compact list of live slots (k_live)
-    const int nit = kLive ? *p.n_live : r.slot_hi - r.slot_lo;
+    // a multi-system step walks the cells of the systems that search (k_live)
+    const int nit = kLive ? cld(p.n_live + 1) : r.slot_hi - r.slot_lo;
     for (int it = xcd_block(); it < nit; it += gridDim.x) {
-        const int slot = cell_slot<kLive>(p, r, it);
-        const int s = sys_of(p, r, slot);
+        const int2 at = cell_at<kLive>(p, r, p.SRCH, it);
+        const int slot = at.x, s = at.y;
         if (s < 0) continue;
         // metadata and parameters through scalar loads: this kernel writes none of
         // the fields it reads (only status bits, by atomics)
@@ -1171,9 +1176,10 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
     const bool forces = kStep || mode != M_PAIRS;
     const bool search = kStep || mode != M_BONDED;
     // a multi-system step walks the compact list of live slots (k_live)
-    const int nit = kLive ? *p.n_live : r.slot_hi - r.slot_lo;
+    const int nit = kLive ? cld(p.n_live) : r.slot_hi - r.slot_lo;
     for (int it = xcd_block(); it < nit; it += gridDim.x) {
-        const int slot = cell_slot<kLive>(p, r, it);
+        const int2 at = cell_at<kLive>(p, r, p.LIVE, it);
+        const int slot = at.x, s = at.y;
         // node data first (every slot of the range is allocated): their latency
         // overlaps the metadata reads
         const size_t cb = (size_t)slot * kSlots;  // the cell's first node (uniform)
@@ -1192,7 +1198,6 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
         const MeshRec mt = ldu(mesh->th, ln);
         const float sg = fused ? ldu(mesh->gs, ln).sign : 0.f;
         const MeshRec r0 = ldu(mesh->r0, ln), ir0 = ldu(mesh->ir0, ln);
-        const int s = __builtin_amdgcn_readfirstlane(sys_of(p, r, slot));
         if (s < 0) continue;
         SysMeta* M = p.meta + s;
         if (!sys_live(M)) continue;
@@ -1594,9 +1599,10 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
     const bool do_dis = kStep || mode == M_DIS_V || mode == M_DIS_VA;
     constexpr bool fused = kStep;
     // a multi-system step walks the compact list of live slots (k_live)
-    const int nit = kLive ? *p.n_live : r.slot_hi - r.slot_lo;
+    const int nit = kLive ? cld(p.n_live) : r.slot_hi - r.slot_lo;
     for (int it = xcd_block(); it < nit; it += gridDim.x) {
-        const int slot = cell_slot<kLive>(p, r, it);
+        const int2 at = cell_at<kLive>(p, r, p.LIVE, it);
+        const int slot = at.x, s = at.y;
         // node data first (every slot of the range is allocated): their latency
         // overlaps the metadata reads
         const size_t cb = (size_t)slot * kSlots;  // the cell's first node (uniform)
@@ -1622,7 +1628,6 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
         }
         const uint32_t nnw = do_dis ? ldu(mesh->th, ln).w : 0u;
         const float sg = do_dis ? ldu(mesh->gs, ln).sign : 0.f;
-        const int s = sys_of(p, r, slot);
         if (s < 0) continue;
         // metadata and parameters through scalar loads: the fields read here are not
         // written by this kernel (search_next and n_reset, which it updates by atomics,
@@ -2299,60 +2304,67 @@ __global__ __launch_bounds__(256) void k_sys_divide(Pool p, Range r, int32_t mod
     for (int s = r.sys_lo + blockIdx.x; s < hi; s += gridDim.x) divide_system(p, s, mode);
 }
 
-// Compact list of the live cell slots of a multi-system range (cells c < n of the
-// systems that step), rebuilt at the start of every step: the step's cell kernels
-// walk it instead of every slot of each system's room.  Every workgroup computes
-// the offsets of all systems in use (an exclusive scan of their live counts, 1024
-// at a time) and writes the slots of the systems s with s mod gridDim.x =
-// blockIdx.x, all lanes on one system at a time; workgroup 0 writes the count.
-__device__ __forceinline__ int live_cells(const SysMeta* m) { return sys_live(m) ? m->n : 0; }
-
+// Lists of the cells of a multi-system step, made at its start: LIVE, the live cells
+// (c < n) of the systems that step, and SRCH, those of them whose system searches
+// this step; n_live holds both counts.  The step's cell kernels walk them instead of
+// every slot of each system's room; each entry is {slot, system}.  Every workgroup
+// scans the counts of all systems in use, 1024 at a time, then finds the system of
+// each of its entries by bisection of the offsets in LDS, so the lists' 20,000
+// entries are written side by side (one system after another per workgroup took
+// 36.9 us for 256 systems; the search over all live cells 38 us where none
+// searched).
 constexpr int kLiveThreads = 1024;
 
 __global__ __launch_bounds__(kLiveThreads) void k_live(Pool p, Range r) {
-    __shared__ int32_t wsum[kLiveThreads / 64];
-    __shared__ int32_t offs[kLiveThreads];
-    __shared__ int32_t carry;
+    __shared__ int2 wsum[kLiveThreads / 64];
+    __shared__ int32_t offl[kLiveThreads + 1], offs[kLiveThreads + 1], base[kLiveThreads];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int lo = r.sys_lo, hi = min(r.sys_hi, *p.nsys);
-    if (tid == 0) carry = 0;
-    __syncthreads();
+    int2 carry{0, 0};
     for (int c0 = lo; c0 < hi; c0 += kLiveThreads) {
         const int s = c0 + tid;
-        const int n = s < hi ? live_cells(p.meta + s) : 0;
+        int2 n{0, 0};
+        if (s < hi) {
+            const SysMeta* M = p.meta + s;
+            const int live = sys_live(M) ? M->n : 0;
+            n = int2{live, M->need_search ? live : 0};
+            base[tid] = M->base;
+        }
         // inclusive scan within the wave, then over the wave totals
-        int v = n;
+        int2 v = n;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
-            const int t = __shfl_up(v, o);
-            if (lane >= o) v += t;
+            const int tx = __shfl_up(v.x, o), ty = __shfl_up(v.y, o);
+            if (lane >= o) { v.x += tx; v.y += ty; }
         }
         if (lane == 63) wsum[wv] = v;
         __syncthreads();
-        if (tid == 0) {
-            int acc = carry;
-            for (int w = 0; w < kLiveThreads / 64; ++w) {
-                const int t = wsum[w];
-                wsum[w] = acc;
-                acc += t;
+        int2 before = carry;
+        for (int w = 0; w < kLiveThreads / 64; ++w) {
+            const int2 t = wsum[w];
+            if (w < wv) { before.x += t.x; before.y += t.y; }
+            carry.x += t.x;
+            carry.y += t.y;
+        }
+        offl[tid] = before.x + v.x - n.x;  // the system's first entry
+        offs[tid] = before.y + v.y - n.y;
+        if (tid == 0) { offl[kLiveThreads] = carry.x; offs[kLiveThreads] = carry.y; }
+        __syncthreads();
+        auto write = [&](const int32_t* off, int2* list) {
+            const int end = off[kLiveThreads];
+            for (int e = off[0] + blockIdx.x * kLiveThreads + tid; e < end; e += gridDim.x * kLiveThreads) {
+                int k = 0;  // the last system whose first entry is at or before e
+#pragma unroll
+                for (int step = kLiveThreads / 2; step > 0; step >>= 1)
+                    if (off[k + step] <= e) k += step;
+                list[e] = int2{base[k] + e - off[k], c0 + k};
             }
-            carry = acc;
-        }
-        __syncthreads();
-        offs[tid] = wsum[wv] + v - n;  // exclusive offset of system s
-        __syncthreads();
-        const int m = min(kLiveThreads, hi - c0);
-        for (int k = 0; k < m; ++k) {
-            const int sk = c0 + k;
-            if (sk % (int)gridDim.x != (int)blockIdx.x) continue;
-            const SysMeta* M = p.meta + sk;
-            const int nk = live_cells(M);
-            const int off = offs[k], base = M->base;
-            for (int c = tid; c < nk; c += kLiveThreads) p.LIVE[off + c] = base + c;
-        }
+        };
+        write(offl, p.LIVE);
+        write(offs, p.SRCH);
         __syncthreads();
     }
-    if (blockIdx.x == 0 && tid == 0) *p.n_live = carry;
+    if (blockIdx.x == 0 && tid < 2) p.n_live[tid] = tid == 0 ? carry.x : carry.y;
 }
 
 // Sets the count of system ids in use (stream-ordered with the steps).
@@ -2801,11 +2813,11 @@ static int grid_cells(const Range& r, int per_cu) {
     return n < 1 ? 1 : (n < cap ? n : cap);
 }
 
-// workgroups of k_live and of the division phase over several systems
-constexpr int kSysBlocks = 256;
+constexpr int kSysBlocks = 256;  // workgroups of the division phase over several systems
+constexpr int kLiveBlocks = 32;  // workgroups of k_live: 32,768 entries side by side
 
 void launch_live(const Pool& p, const Range& r, hipStream_t st) {
-    launch(k_live, dim3(kSysBlocks / 4), dim3(kLiveThreads), st, p, r);
+    launch(k_live, dim3(kLiveBlocks), dim3(kLiveThreads), st, p, r);
 }
 void launch_set_nsys(const Pool& p, int n, hipStream_t st) { launch(k_set_nsys, dim3(1), dim3(64), st, p, n); }
 

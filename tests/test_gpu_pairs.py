@@ -166,3 +166,52 @@ def test_reads_return_what_was_written(oracle_mesh, n):
         P = np.zeros(n, np.float32)
         engine.check(L.cs3d_get_state(ctx.h, s.id, None, None, P.ctypes.data, None, None, None, None), "cs3d_get_state")
         assert np.array_equal(P, want[A.F_PRESSURE][:n])
+
+
+def test_more_systems_than_one_scan_of_the_live_list(oracle_mesh):
+    """1030 systems in one batch (the live list scans 1024 at a time) of 0 to 3 cells, some
+    stopped at a horizon and some removed: each ends where it ends alone."""
+    from cellsim3d_amd import abi as A
+    from cellsim3d_amd import configs, engine
+    print("1030 systems", flush=True)
+    kinds = []
+    for n in range(4):
+        p = configs.base_params(3 + n)
+        p.grid_interval = 2
+        p.division_vol = 1e30  # (the default is the reference mesh's, below this mesh's rest volume)
+        X, Y, Z = configs.place(configs.unit_mesh(), [(2.1 * i, 0.1 * i, 0) for i in range(n)], 0.02,
+                                np.random.default_rng(n)) if n else (np.zeros(0, np.float32),) * 3
+        kinds.append((p, X, Y, Z, n))
+    nsys = 1030
+    with engine.Context(oracle_mesh, capacity_cells=4 * nsys, voxel_budget=nsys * 33 * 64,
+                        bin_budget=nsys * (16384 * A.BIN_WORDS + 16)) as ctx:
+        alone = {}
+        for n, k in enumerate(kinds):
+            for steps in (3, 12):
+                s = ctx.add_system(*k, max_cells=max(n, 1), voxels=32)
+                s.step(steps)
+                ctx.sync()
+                alone[n, steps] = [s.get(f)[:n * 192] for f in (A.F_X, A.F_VZ, A.F_FDY)]
+                s.remove()
+        systems = []
+        for i in range(nsys):
+            n = (i * 7 + i // 5) % 4
+            s = ctx.add_system(*kinds[n], max_cells=max(n, 1), voxels=32)
+            if i % 11 == 3:
+                s.set_horizon(3)
+            systems.append((i, n, s))
+        for i, n, s in systems:
+            if i % 50 == 7:
+                s.remove()
+        ctx.step(12)  # a captured ten and two eager steps
+        ctx.sync()
+        cells, steps, status = ctx.poll(0, nsys)
+        for i, n, s in systems:
+            if i % 50 == 7:
+                assert cells[s.id] == -1
+                continue
+            k = 3 if i % 11 == 3 else 12
+            assert (cells[s.id], steps[s.id], status[s.id]) == (n, k, 0), i
+            if i < 40 or i > 1015 or i % 37 == 0:
+                for f, want in zip((A.F_X, A.F_VZ, A.F_FDY), alone[n, k]):
+                    assert np.array_equal(s.get(f)[:n * 192], want), (i, f)
