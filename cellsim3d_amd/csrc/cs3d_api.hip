@@ -31,7 +31,8 @@ void launch_divide(const Pool& p, const Range& r, int mode, hipStream_t st);
 extern thread_local std::vector<std::pair<hipEvent_t, hipEvent_t>>* kernel_timer;
 void launch_com_shift(const Pool& p, const Range& r, hipStream_t st);
 void launch_live(const Pool& p, const Range& r, hipStream_t st);
-void launch_set_nsys(const Pool& p, int n, hipStream_t st);
+void launch_room_init(const Pool& p, const RoomInit& a, hipStream_t st);
+void launch_room_free(const Pool& p, int base, int cap, int sys, int nsys, hipStream_t st);
 void launch_grid(const Pool& p, const Range& r, int vox_blocks, hipStream_t st);
 void launch_vox_lists(const Pool& p, const Range& r, int vox_blocks, hipStream_t st);
 void launch_vrange(const Pool& p, const Range& r, hipStream_t st);
@@ -631,8 +632,10 @@ extern "C" cs3d_status cs3d_sync(cs3d_ctx* c) {
     return CS3D_OK;
 }
 
-extern "C" cs3d_status cs3d_system_add_raw(cs3d_ctx* c, const cs3d_params* prm, int32_t n_cells, int32_t max_cells,
-                                           int64_t voxels, cs3d_sys* out) {
+namespace {
+// cs3d_system_add_raw, enqueued on the context's stream
+cs3d_status room_add(cs3d_ctx* c, const cs3d_params* prm, int32_t n_cells, int32_t max_cells, int64_t voxels,
+                     cs3d_sys* out) {
     if (!c || !prm || !out) return fail(CS3D_INVALID_ARG, "NULL argument");
     cs3d_status st = cs3d_params_check(prm);
     if (st != CS3D_OK) return st;
@@ -674,27 +677,6 @@ extern "C" cs3d_status cs3d_system_add_raw(cs3d_ctx* c, const cs3d_params* prm, 
     h.prm = *prm;
     c->nsys_high = std::max(c->nsys_high, sid + 1);
     HIPCHK(hipSetDevice(c->device));
-    const Pool& p = c->pool;
-    const int64_t nb = base * kSlots, nbytes = (int64_t)max_cells * kSlots * 4;
-    float* node[] = {p.X,   p.Y,   p.Z,   p.VX,  p.VY,  p.VZ,  p.VAX, p.VAY, p.VAZ,
-                     p.FCX, p.FCY, p.FCZ, p.FDX, p.FDY, p.FDZ, p.FRX, p.FRY, p.FRZ};
-    for (float* a : node) HIPCHK(hipMemsetAsync(a + nb, 0, nbytes, c->stream));
-    float* cellz[] = {p.CMX, p.CMY, p.CMZ, p.VOL, p.AREA};
-    for (float* a : cellz) HIPCHK(hipMemsetAsync(a + base, 0, (size_t)max_cells * 4, c->stream));
-    HIPCHK(hipMemsetAsync(p.FLAG + base, 0, max_cells, c->stream));
-    HIPCHK(hipMemsetAsync(p.BBOX + base * 6, 0, (size_t)max_cells * 24, c->stream));
-    HIPCHK(hipMemsetAsync(p.BBOXN + base * 6, 0, (size_t)max_cells * 24, c->stream));
-    HIPCHK(hipMemsetAsync(p.NPAIR + nb, 0, (size_t)max_cells * kSlots * 4, c->stream));
-    HIPCHK(hipMemsetAsync(p.NCAND + nb, 0, (size_t)max_cells * kSlots * 4, c->stream));
-    HIPCHK(hipMemsetAsync(p.vox + vreg, 0, (size_t)vb * (1 + vcap) * 4, c->stream));
-    HIPCHK(hipMemsetAsync(p.bins + breg, 0, (size_t)bb * 4, c->stream));
-    std::vector<float> pv(max_cells, prm->min_pressure), ev(max_cells, prm->stiffness1), gv(max_cells, 1.0f);
-    std::vector<int32_t> owner(max_cells, sid);
-    HIPCHK(hipMemcpyAsync(p.P + base, pv.data(), max_cells * 4, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(p.E + base, ev.data(), max_cells * 4, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(p.GS + base, gv.data(), max_cells * 4, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(p.slot_sys + base, owner.data(), max_cells * 4, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync((void*)(p.prm + sid), prm, sizeof(cs3d_params), hipMemcpyHostToDevice, c->stream));
     SysMeta m;
     std::memset(&m, 0, sizeof(m));
     m.n = n_cells;
@@ -724,13 +706,20 @@ extern "C" cs3d_status cs3d_system_add_raw(cs3d_ctx* c, const cs3d_params* prm, 
     }
     cs3d_ranmar_init(&m.rng, prm->ranmar_ij, prm->ranmar_kl);
     kick_consts(prm->mass, prm->dt, m);
-    launch_set_nsys(c->pool, c->nsys_high, c->stream);
-    st = write_meta(c, sid, m);
-    if (st != CS3D_OK) return st;
+    launch_room_init(c->pool, RoomInit{m, *prm, sid, c->nsys_high}, c->stream);
+    HIPCHK(hipGetLastError());
     // a captured all-systems step without CorrectCoMMotion cannot serve this system
     auto g = c->graphs.find(CS3D_ALL);
     if (prm->correct_com && g != c->graphs.end() && !g->second.shift) drop_graphs(c, CS3D_ALL);
     *out = sid;
+    return CS3D_OK;
+}
+}  // namespace
+
+extern "C" cs3d_status cs3d_system_add_raw(cs3d_ctx* c, const cs3d_params* prm, int32_t n_cells, int32_t max_cells,
+                                           int64_t voxels, cs3d_sys* out) {
+    if (const cs3d_status st = room_add(c, prm, n_cells, max_cells, voxels, out); st != CS3D_OK) return st;
+    HIPCHK(hipStreamSynchronize(c->stream));
     return CS3D_OK;
 }
 
@@ -739,7 +728,7 @@ extern "C" cs3d_status cs3d_system_add(cs3d_ctx* c, const cs3d_params* prm, int3
                                        const float* vx, const float* vy, const float* vz, cs3d_sys* out) {
     if (!x || !y || !z) return fail(CS3D_INVALID_ARG, "positions are required");
     cs3d_sys s;
-    cs3d_status st = cs3d_system_add_raw(c, prm, n_cells, max_cells, voxels, &s);
+    cs3d_status st = room_add(c, prm, n_cells, max_cells, voxels, &s);
     if (st != CS3D_OK) return st;
     const size_t bytes = (size_t)n_cells * kSlots * 4;
     const int64_t nb = (int64_t)c->sys[s].base * kSlots;
@@ -771,11 +760,7 @@ extern "C" cs3d_status cs3d_system_remove(cs3d_ctx* c, cs3d_sys s) {
     if (!valid_sys(c, s)) return fail(CS3D_INVALID_ARG, "unknown system");
     HIPCHK(hipStreamSynchronize(c->stream));
     SysHost& h = c->sys[s];
-    std::vector<int32_t> owner(h.cap, -1);
-    HIPCHK(hipMemcpy(c->pool.slot_sys + h.base, owner.data(), h.cap * 4, hipMemcpyHostToDevice));
-    SysMeta m;
-    std::memset(&m, 0, sizeof(m));
-    HIPCHK(hipMemcpy(c->pool.meta + s, &m, sizeof(m), hipMemcpyHostToDevice));
+    const int32_t base = h.base, cap = h.cap;
     c->cells.release(h.base);
     c->voxels.release(h.vreg);
     c->bins.release(h.breg);
@@ -785,7 +770,7 @@ extern "C" cs3d_status cs3d_system_remove(cs3d_ctx* c, cs3d_sys s) {
     for (int i = 0; i < (int)c->sys.size(); ++i)
         if (c->sys[i].used) hi = i + 1;
     c->nsys_high = hi;
-    launch_set_nsys(c->pool, hi, c->stream);
+    launch_room_free(c->pool, base, cap, s, hi, c->stream);
     HIPCHK(hipGetLastError());
     return CS3D_OK;
 }

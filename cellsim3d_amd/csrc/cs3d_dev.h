@@ -156,7 +156,7 @@ struct Pool {
     int32_t* nsys;   // int32[1]: system ids in use are below this (kernels over all systems read it, so a
                      // captured all-systems step stays valid when systems are added or removed)
     SysMeta* meta;
-    const cs3d_params* prm;
+    cs3d_params* prm;
     int32_t* vox;
     int32_t* bins;
     const MeshDev* mesh;
@@ -169,6 +169,14 @@ struct Range {
     int32_t sys_lo, sys_hi;
     int32_t one_sys;  // 1: the range is exactly the slot range of system sys_lo
     int32_t live;     // 1: the cell kernels walk Pool::LIVE (built by k_live) instead of the slots
+};
+
+// A system entering its room (k_room_init): its metadata (room, voxel and bin
+// regions, geometry), parameters, id, and the count of system ids in use.
+struct RoomInit {
+    SysMeta meta;
+    cs3d_params prm;
+    int32_t sys, nsys;
 };
 
 // Pieces of device memory that one launch copies into a buffer (k_gather).
