@@ -90,6 +90,7 @@ struct RangeAlloc {
 struct SysHost {
     bool used = false;
     int32_t base = 0, cap = 0;
+    int32_t n_seen = 0;  // live cells when the host last looked
     int64_t vreg = 0;  // voxel region offset
     int32_t vbudget = 0, vcap = 0;
     int64_t breg = 0;  // search-bin region offset
@@ -117,6 +118,7 @@ struct cs3d_ctx {
         hipGraphExec_t exec;
         int steps;
         bool shift;  // the captured steps include CorrectCoMMotion
+        int32_t live;  // Range::live_hint at the capture
     };
     std::map<int, GraphRec> graphs;  // target -> captured steps
     cs3d_mesh mesh_host;  // the tables the context was created with (checkpoint check)
@@ -168,6 +170,10 @@ Range range_of(cs3d_ctx* c, cs3d_sys s) {
         r.sys_hi = kMaxSys;
         r.one_sys = 0;
         r.live = 0;
+        int64_t n = 0;
+        for (int i = 0; i < c->nsys_high; ++i)
+            if (c->sys[i].used) n += c->sys[i].n_seen;
+        r.live_hint = (int32_t)n;
     } else {
         r.slot_lo = c->sys[s].base;
         r.slot_hi = c->sys[s].base + c->sys[s].cap;
@@ -175,6 +181,7 @@ Range range_of(cs3d_ctx* c, cs3d_sys s) {
         r.sys_hi = s + 1;
         r.one_sys = 1;
         r.live = 0;
+        r.live_hint = c->sys[s].n_seen;
     }
     return r;
 }
@@ -329,12 +336,15 @@ cs3d_status read_back(cs3d_ctx* c, const ReadSeg* segs, int n_segs) {
 
 cs3d_status read_meta(cs3d_ctx* c, cs3d_sys s, SysMeta& m) {
     const ReadSeg seg{c->pool.meta + s, &m, sizeof(SysMeta)};
-    return read_back(c, &seg, 1);
+    const cs3d_status st = read_back(c, &seg, 1);
+    if (st == CS3D_OK) c->sys[s].n_seen = m.n;
+    return st;
 }
 
 cs3d_status write_meta(cs3d_ctx* c, cs3d_sys s, const SysMeta& m) {
     HIPCHK(hipMemcpyAsync(c->pool.meta + s, &m, sizeof(SysMeta), hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    c->sys[s].n_seen = m.n;
     return CS3D_OK;
 }
 
@@ -564,7 +574,7 @@ extern "C" cs3d_status cs3d_ctx_create(int device, const cs3d_mesh* mesh, int64_
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess)
         return cleanup(fail(CS3D_HIP_ERROR, "hipStreamCreate failed"));
     Pool& p = c->pool;
-    p.wg_per_cu = 16;
+    p.wg_per_cu = 0;
     const int64_t ns = capacity_cells * kSlots;
     cs3d_status st = CS3D_OK;
     float** nodes[] = {&p.X, &p.Y, &p.Z, &p.VX, &p.VY, &p.VZ, &p.VAX, &p.VAY, &p.VAZ,
@@ -669,6 +679,7 @@ cs3d_status room_add(cs3d_ctx* c, const cs3d_params* prm, int32_t n_cells, int32
     h.used = true;
     h.base = (int32_t)base;
     h.cap = max_cells;
+    h.n_seen = n_cells;
     h.vreg = vreg;
     h.vbudget = (int32_t)vb;
     h.vcap = vcap;
@@ -900,6 +911,7 @@ extern "C" cs3d_status cs3d_get_state(cs3d_ctx* c, cs3d_sys s, float* xyz, float
             if (cell_to(k, 0)) segs.push_back(ReadSeg{cell[k] + h.base, at, (size_t)h.cap * 4});
         const cs3d_status st = read_back(c, segs.data(), (int)segs.size());
         if (st != CS3D_OK) return st;
+        c->sys[s].n_seen = m.n;
         const size_t n = (size_t)m.n;
         for (int k = 0; k < 6; ++k)
             if (float* q = node_to(k, n)) std::memcpy(q, buf.data() + (size_t)k * h.cap * kSlots, n * kSlots * 4);
@@ -1164,6 +1176,7 @@ extern "C" cs3d_status cs3d_systems_poll(cs3d_ctx* c, int32_t first, int32_t cou
     if (const cs3d_status st = read_back(c, &seg, 1); st != CS3D_OK) return st;
     for (int32_t i = 0; i < count; ++i) {
         const bool used = c->sys[first + i].used;
+        if (used) c->sys[first + i].n_seen = m[i].n;
         if (n_cells) n_cells[i] = used ? m[i].n : -1;
         if (steps) steps[i] = used ? m[i].step : -1;
         if (status) status[i] = used ? m[i].status : 0u;
@@ -1334,9 +1347,15 @@ namespace {
 // The captured graph_steps steps of a target, captured, instantiated and
 // uploaded on first use.
 cs3d_status graph_of(cs3d_ctx* c, cs3d_sys s, const cs3d_ctx::GraphRec** out) {
+    const Range r = range_of(c, s);
     auto it = c->graphs.find(s);
+    // a tissue that has outgrown the grids of its capture (they would stride) is captured
+    // again; the factor keeps that rare
+    if (it != c->graphs.end() && r.live_hint > it->second.live + it->second.live / 2 + 64) {
+        drop_graphs(c, s);
+        it = c->graphs.end();
+    }
     if (it == c->graphs.end()) {
-        const Range r = range_of(c, s);
         const int vb = vox_blocks_of(c, s);
         hipGraph_t g = nullptr;
         HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
@@ -1351,7 +1370,7 @@ cs3d_status graph_of(cs3d_ctx* c, cs3d_sys s, const cs3d_ctx::GraphRec** out) {
             (void)hipGraphExecDestroy(ex);
             return fail(CS3D_HIP_ERROR, std::string("hipGraphUpload: ") + hipGetErrorString(e));
         }
-        it = c->graphs.emplace(s, cs3d_ctx::GraphRec{ex, c->graph_steps, any_correct_com(c, r)}).first;
+        it = c->graphs.emplace(s, cs3d_ctx::GraphRec{ex, c->graph_steps, any_correct_com(c, r), r.live_hint}).first;
     }
     *out = &it->second;
     return CS3D_OK;

@@ -160,7 +160,7 @@ struct Pool {
     int32_t* vox;
     int32_t* bins;
     const MeshDev* mesh;
-    int32_t wg_per_cu;  // host side: cap of the grid of the cell kernels, workgroups per CU
+    int32_t wg_per_cu;  // host side: the caller's cap of the grid of the cell kernels, workgroups per CU (0: none)
 };
 
 // What a launch works on: cell slots [slot_lo, slot_hi) and systems [sys_lo, sys_hi).
@@ -169,6 +169,7 @@ struct Range {
     int32_t sys_lo, sys_hi;
     int32_t one_sys;  // 1: the range is exactly the slot range of system sys_lo
     int32_t live;     // 1: the cell kernels walk Pool::LIVE (built by k_live) instead of the slots
+    int32_t live_hint;  // host side: live cells as of the host's last look (sizes grids, nothing else)
 };
 
 // A system entering its room (k_room_init): its metadata (room, voxel and bin

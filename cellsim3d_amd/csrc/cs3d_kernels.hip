@@ -2849,13 +2849,28 @@ static void launch(F kernel, dim3 grid, dim3 block, hipStream_t st, A... args) {
     hipLaunchKernelGGL(kernel, grid, block, 0, st, args...);
 }
 
-// Grid of a cell kernel: one workgroup per cell slot up to 256 CUs x wg_per_cu
-// workgroups; beyond that each workgroup strides over several cells.
+// Grid of a step's cell kernel: a workgroup for each live cell that the host knows of
+// and a quarter more (cells that divide before it looks again; beyond the grid the
+// workgroups stride), at most 256 CUs x wg_per_cu if the caller set that.  One cell per
+// workgroup lets the dispatcher even out the load: at 20,000 cells k_con_dis takes
+// 156 us, with 4096 workgroups of 4 or 5 cells 183 us, with 2048 172 us, with 6144
+// 197 us (k_dis_post 94, 109, 103, 118).  A workgroup without a cell still costs its
+// dispatch, 2 to 3 ns, so rooms far larger than their tissue are not launched whole.
+static int grid_step(const Range& r, int per_cu) {
+    const int64_t slots = r.slot_hi - r.slot_lo, live = (int64_t)r.live_hint + r.live_hint / 4 + 8;
+    const int64_t n = live < slots ? live : slots, cap = per_cu > 0 ? 256 * (int64_t)per_cu : n;
+    return (int)(n < 1 ? 1 : (n < cap ? n : cap));
+}
+// Grid of the other cell kernels: one workgroup per slot up to 4096, then they stride.
 static int grid_cells(const Range& r, int per_cu) {
     const int n = r.slot_hi - r.slot_lo;
     const int cap = 256 * (per_cu > 0 ? per_cu : 16);
     return n < 1 ? 1 : (n < cap ? n : cap);
 }
+// k_search in a multi-system step: few cells search, and which is not known here; the
+// 1280 workgroups that fit the chip (31 KB of LDS each) take 45 us of a step of 256
+// tissues, 4096 take 90, 20,480 110
+constexpr int kSearchLive = 1280;
 
 constexpr int kSysBlocks = 256;  // workgroups of the division phase over several systems
 constexpr int kLiveBlocks = 32;  // workgroups of k_live: 32,768 entries side by side
@@ -2875,21 +2890,22 @@ void launch_room_free(const Pool& p, int base, int cap, int sys, int nsys, hipSt
 
 void launch_integrate(const Pool& p, const Range& r, int flags, int64_t step_override, hipStream_t st) {
     if (r.live)
-        launch(k_integrate<1>, dim3(grid_cells(r, p.wg_per_cu)), dim3(192), st, p, r, flags, step_override);
+        launch(k_integrate<1>, dim3(grid_step(r, p.wg_per_cu)), dim3(192), st, p, r, flags, step_override);
     else
-        launch(k_integrate<0>, dim3(grid_cells(r, p.wg_per_cu)), dim3(192), st, p, r, flags, step_override);
+        launch(k_integrate<0>, dim3(grid_step(r, p.wg_per_cu)), dim3(192), st, p, r, flags, step_override);
 }
 void launch_search(const Pool& p, const Range& r, int always, hipStream_t st) {
+    const int g = grid_step(r, p.wg_per_cu);
     if (r.live)
-        launch(k_search<1>, dim3(grid_cells(r, p.wg_per_cu)), dim3(192), st, p, r, always);
+        launch(k_search<1>, dim3(g < kSearchLive ? g : kSearchLive), dim3(192), st, p, r, always);
     else
-        launch(k_search<0>, dim3(grid_cells(r, p.wg_per_cu)), dim3(192), st, p, r, always);
+        launch(k_search<0>, dim3(g), dim3(192), st, p, r, always);
 }
 void launch_con(const Pool& p, const Range& r, int mode, bool use_va, hipStream_t st) {
     const float* vx = use_va ? p.VAX : p.VX;
     const float* vy = use_va ? p.VAY : p.VY;
     const float* vz = use_va ? p.VAZ : p.VZ;
-    const dim3 grid(grid_cells(r, p.wg_per_cu)), block(192);
+    const dim3 grid(grid_step(r, p.wg_per_cu)), block(192);
     if (mode != M_STEP)  // one system
         launch(k_con_dis<0, false>, grid, block, st, p, r, mode, p.X, p.Y, p.Z, vx, vy, vz, p.BBOX);
     else if (r.live)
@@ -2907,7 +2923,7 @@ void launch_dis(const Pool& p, const Range& r, int mode, int64_t step_override, 
     const float* vx = use_va ? p.VAX : p.VX;
     const float* vy = use_va ? p.VAY : p.VY;
     const float* vz = use_va ? p.VAZ : p.VZ;
-    const dim3 grid(grid_cells(r, p.wg_per_cu)), block(192);
+    const dim3 grid(grid_step(r, p.wg_per_cu)), block(192);
     if (mode != M_STEP)  // one system
         launch(k_dis_post<0, false>, grid, block, st, p, r, mode, step_override, clear_bins, p.X, p.Y, p.Z, vx, vy, vz);
     else if (r.live)
@@ -2920,7 +2936,7 @@ void launch_divide(const Pool& p, const Range& r, int mode, hipStream_t st) {
     launch(k_sys_divide, dim3(ns < 1 ? 1 : (ns < kSysBlocks ? ns : kSysBlocks)), dim3(256), st, p, r, mode);
 }
 void launch_com_shift(const Pool& p, const Range& r, hipStream_t st) {
-    launch(k_com_shift, dim3(grid_cells(r, p.wg_per_cu)), dim3(kSlots), st, p, r);
+    launch(k_com_shift, dim3(grid_step(r, p.wg_per_cu)), dim3(kSlots), st, p, r);
 }
 void launch_grid(const Pool& p, const Range& r, int vox_blocks, hipStream_t st) {
     const int n = r.slot_hi - r.slot_lo;

@@ -284,7 +284,8 @@ cs3d_status cs3d_set_graph(cs3d_ctx* ctx, int32_t enable);
 /* Number of steps captured per HIP graph (default 10). */
 cs3d_status cs3d_set_graph_steps(cs3d_ctx* ctx, int32_t steps);
 /* Launch shape of the cell kernels: at most 256 x wg_per_cu workgroups (one
- * cell each; beyond that a workgroup strides over several cells).  Default 16.
+ * cell each; beyond that a workgroup strides over several cells).  Without a call
+ * the step's kernels launch one workgroup per live cell, the others as with 16.
  * No counterpart in the reference (one block per cell, GPUbounce.cu:1059-1164);
  * set by the ensemble autotuner. */
 cs3d_status cs3d_set_launch(cs3d_ctx* ctx, int32_t wg_per_cu);

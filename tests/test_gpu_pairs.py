@@ -5,7 +5,8 @@ against the oracle: no candidates at all, one round (at most 192
 pairs per cell), several rounds, nodes whose candidates straddle a round or a
 64-lane word, and lists near the 40-entry limit; and the bonds and angles at the
 edges of the short arithmetic (rest shape, crushed, stretched, bonds at and below
-its range); the division phase's flag test; reads of device memory."""
+its range); the division phase's flag test; reads of device memory; batches past one
+scan of the live list; grids smaller than their tissue."""
 import numpy as np
 import pytest
 
@@ -215,3 +216,37 @@ def test_more_systems_than_one_scan_of_the_live_list(oracle_mesh):
             if i < 40 or i > 1015 or i % 37 == 0:
                 for f, want in zip((A.F_X, A.F_VZ, A.F_FDY), alone[n, k]):
                     assert np.array_equal(s.get(f)[:n * 192], want), (i, f)
+
+
+# cells, workgroups per CU that the caller allows (0: no call), systems stepped together
+@pytest.mark.parametrize("n,cap,both", [(1, 0, False), (9, 0, False), (70, 0, False), (70, 0, True), (150, 0, True), (300, 1, True)])
+def test_grids_smaller_than_the_tissue(oracle_mesh, n, cap, both):
+    """Every cell divides in the first step, while the host still knows of half of them:
+    the grids of the following steps cover a part and stride, and the graph captured
+    with them gives way to a wider one at 300.  As with a host that looks after each step."""
+    from cellsim3d_amd import abi as A
+    from cellsim3d_amd import configs, engine
+    print("grids: %d cells, cap %d, both %d" % (n, cap, both), flush=True)
+    _, X, Y, Z, _ = configs.lattice_tissue(n, 0.2, seed=n)
+    p = configs.base_params(2)
+    p.voxel_capacity = 64
+    p.division_vol = 0.8 * configs.mesh_volume(configs.unit_mesh())  # the cells are above it, their daughters below
+    p.div_time_steps = 100
+    fields = (A.F_X, A.F_VY, A.F_FCZ, A.F_FDX, A.F_VOLUME, A.F_CANDCOUNT)
+    got = []
+    for look in (True, False):
+        with engine.Context(oracle_mesh, capacity_cells=6 * n + 2, voxel_budget=1 << 21, bin_budget=1 << 26) as ctx:
+            if cap:
+                ctx.set_launch(cap)
+            systems = [ctx.add_system(p, X, Y, Z, n, max_cells=2 * n + 1, voxels=1 << 12) for _ in range(2 if both else 1)]
+            for _ in range(24 if look else 2):
+                (ctx if both else systems[0]).step(1 if look else 12)
+                for s in systems:
+                    s.info()
+            ctx.sync()
+            assert all(s.info()[0] == 2 * n for s in systems)
+            got.append([[s.get(f) for f in fields] for s in systems])
+    for a, b in zip(*got):
+        for f, u, v in zip(fields, a, b):
+            k = 2 * n * (1 if f == A.F_VOLUME else 192)
+            assert np.array_equal(u[:k], v[:k], equal_nan=True), f
