@@ -294,26 +294,28 @@ cs3d_status read_back(cs3d_ctx* c, const ReadSeg* segs, int n_segs) {
     std::vector<std::atomic<int>> done(n);  // readers that have copied slot k
     for (auto& d : done) d.store(0, std::memory_order_relaxed);
     std::vector<std::thread> readers;
-    int want = total < kSerialRead ? 0 : kReaders;
-    try {
-        readers.reserve(want);
-        for (int t = 0; t < want; ++t)
-            readers.emplace_back([&, t] {
-                for (int k = 0; k < n; ++k) {
-                    while (ready.load(std::memory_order_acquire) <= k) {
-                        if (stop.load(std::memory_order_relaxed)) return;
-                        std::this_thread::yield();
+    int want = 0;
+    auto start_readers = [&] {  // once data is there: the stream may hold steps still to run, and readers spin
+        try {
+            readers.reserve(kReaders);
+            for (int t = 0; t < kReaders; ++t)
+                readers.emplace_back([&, t] {
+                    for (int k = 0; k < n; ++k) {
+                        while (ready.load(std::memory_order_acquire) <= k) {
+                            if (stop.load(std::memory_order_relaxed)) return;
+                            std::this_thread::yield();
+                        }
+                        copy_share(pieces[k], slot(k), t, kReaders);
+                        done[k].fetch_add(1, std::memory_order_release);
                     }
-                    copy_share(pieces[k], slot(k), t, kReaders);
-                    done[k].fetch_add(1, std::memory_order_release);
-                }
-            });
-    } catch (const std::exception&) {  // no threads to be had: those that run end, this one copies alone
-        stop.store(true);
-        for (auto& t : readers) t.join();
-        readers.clear();
-        want = 0;
-    }
+                });
+            want = kReaders;
+        } catch (const std::exception&) {  // no threads to be had: those that run end, this one copies alone
+            stop.store(true);
+            for (auto& t : readers) t.join();
+            readers.clear();
+        }
+    };
     hipError_t e = hipSuccess;
     for (int issued = 0, k = 0; k < n && e == hipSuccess; ++k) {
         for (; issued < n && issued < k + kSlotsInRing && e == hipSuccess; ++issued) {
@@ -325,6 +327,7 @@ cs3d_status read_back(cs3d_ctx* c, const ReadSeg* segs, int n_segs) {
         }
         if (e == hipSuccess) e = hipEventSynchronize(c->stage_ev[k % kSlotsInRing]);
         if (e != hipSuccess) break;
+        if (k == 0 && total >= kSerialRead) start_readers();
         if (want) ready.store(k + 1, std::memory_order_release);
         else copy_share(pieces[k], slot(k), 0, 1);
     }
