@@ -42,8 +42,26 @@ __device__ __forceinline__ int sys_of(const Pool& p, const Range& r, int slot) {
     return r.one_sys ? r.sys_lo : p.slot_sys[slot];
 }
 
+// The entry of a cell kernel is a chain of memory round trips that nothing else
+// overlaps in a small tissue: kernel arguments, then the cell's node data beside the
+// system's metadata (one scalar round trip), then what depends on them.  Read field by
+// field, with a branch on each, it was 7 trips in k_con_dis, 6 in k_dis_post and 5 in
+// k_integrate.  With it in three, and the division kernel's arguments and metadata read
+// in one batch each, a step took 24.4 instead of 25.6 us at 8 cells, 29.6 instead of
+// 30.9 at 403 and 40.5 instead of 42.3 at 2000.
 template <class MP> __device__ __forceinline__ bool sys_live(MP m) {
-    return m->active && (m->horizon < 0 || m->step < m->horizon) && !(m->status & CS3D_SYS_FATAL_MASK);
+    // every field read at once, no short-circuit branches: one memory round trip
+    const int32_t active = m->active;
+    const int64_t horizon = m->horizon, step = m->step;
+    const uint32_t status = m->status;
+    return (active != 0) & ((horizon < 0) | (step < horizon)) & !(status & CS3D_SYS_FATAL_MASK);
+}
+
+// Whether cell slot `slot` of the system is stepped; c: its local index.
+template <class MP> __device__ __forceinline__ bool cell_live(MP m, int slot, int& c) {
+    const int32_t base = m->base, n = m->n;
+    c = slot - base;
+    return sys_live(m) & (c < n);
 }
 
 __device__ __forceinline__ void flag(SysMeta* m, uint32_t bits) {
@@ -59,6 +77,15 @@ __device__ __forceinline__ void flag(SysMeta* m, uint32_t bits) {
 // key * 4 < 2^32).
 template <class T> __device__ __forceinline__ T ldu(const T* base, uint32_t i) {
     return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + i * (uint32_t)sizeof(T));
+}
+// ldu of a word whose load is issued here: as a relaxed atomic (a plain load
+// instruction at this scope) it is not moved behind a branch that follows.
+template <class T> __device__ __forceinline__ T load_now(const T* q) {
+    static_assert(sizeof(T) == 4, "one word");
+    return __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+template <class T> __device__ __forceinline__ T ldu_now(const T* base, uint32_t i) {
+    return load_now(reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + i * 4u));
 }
 template <class T> __device__ __forceinline__ void stu(T* base, uint32_t i, T v) {
     *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + i * (uint32_t)sizeof(T)) = v;
@@ -107,13 +134,14 @@ __device__ __forceinline__ float rcp_rn(float b) {
 // a short division otherwise).
 __device__ __forceinline__ void slow_path() { asm volatile(""); }
 
+// CS3D_SELDOM (cs3d_theta.h) marks branches hardly ever taken.  What one guards is
+// done for every lane of the wave that takes it: the general forms give the same
+// bits where the short ones are in range.
+
 // 1.0f / b: from rcp_rn where quot_ok(b), by division otherwise (the same bits)
 __device__ __forceinline__ float inv_rn(float b) {
     float y = rcp_rn(b);
-    if (!quot_ok(b)) {
-        slow_path();
-        y = 1.0f / b;
-    }
+    if (CS3D_SELDOM(!quot_ok(b))) y = 1.0f / b;
     return y;
 }
 
@@ -121,10 +149,7 @@ __device__ __forceinline__ float inv_rn(float b) {
 __device__ __forceinline__ float inv_sqrt_rn(float x2) {
     const float r = sqrt_normal(x2);
     float y = rcp_rn(r);
-    if (!quot_ok(r)) {
-        slow_path();
-        y = 1.0f / sqrt_cr(x2);
-    }
+    if (CS3D_SELDOM(!quot_ok(r))) y = 1.0f / sqrt_cr(x2);
     return y;
 }
 
@@ -160,7 +185,7 @@ __device__ __forceinline__ void spring_div(float stiffness, float R, float R0, f
 
 // rGrowth of the population model, GPUbounce.cu:1077-1088
 template <class PP> __device__ __forceinline__ float rgrowth(PP P, int n) {
-    if (P->do_pop_model == 1) {
+    if (__builtin_expect(P->do_pop_model == 1, 0)) {
         float r = (float)((double)P->growth_rate * (1 - (n * 1.0 / (double)P->max_pop)));
         if (r < 0) r = 0;
         return r;
@@ -208,8 +233,7 @@ __device__ __forceinline__ CPool pool_late() {
 template <int kLive>
 __device__ __forceinline__ int2 cell_at(const Pool& p, const Range& r, const int2* list, int it) {
     if (kLive) return int2{cld(&list[it].x), cld(&list[it].y)};
-    const int slot = __builtin_amdgcn_readfirstlane(r.slot_lo + it);
-    return int2{slot, __builtin_amdgcn_readfirstlane(sys_of(p, r, slot))};
+    return int2{__builtin_amdgcn_readfirstlane(r.slot_lo + it), r.sys_lo};
 }
 
 // The lane's node index as a value the compiler cannot see through (an empty asm
@@ -243,6 +267,14 @@ __device__ __forceinline__ int xcd_block() {
     const int q = G / kXcds, rem = G % kXcds;
     const int k = v % kXcds, j = v / kXcds;
     return k * q + min(k, rem) + j;
+}
+
+// The first iteration of a cell kernel's loop over nit cells.  The grid over a range of
+// slots has at most one workgroup per slot, so its loop need not be entered by a test.
+template <int kLive> __device__ __forceinline__ int first_cell(int nit) {
+    const int it = xcd_block();
+    if (!kLive) __builtin_assume(it < nit);
+    return it;
 }
 
 // Search bins are periodic: bin coordinate floor((x - origin) / h) modulo the bin
@@ -489,17 +521,20 @@ __device__ __forceinline__ void box_of_cell(float x, float y, float z, bool node
 // search bins.
 // ------------------------------------------------------------------------------
 // 6 waves per SIMD (at most 80 VGPRs): 8 workgroups per CU, one round for 2048 cells
-// kLive: walk Pool::LIVE (a multi-system step) instead of the range's slots
-template <int kLive>
+// kLive: walk Pool::LIVE (a multi-system step) instead of the range's slots; kStep: the
+// flags are those of the fused step (kStepFlags)
+constexpr int32_t kStepFlags = I_KICK | I_PRESSURE | I_BINS | I_IFSEARCH | I_GRIDCOUNT;
+template <int kLive, bool kStep>
 __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_integrate(Pool p, Range r,
-                                                                                              int32_t flags,
+                                                                                              int32_t run_flags,
                                                                                               int64_t step_override) {
+    const int32_t flags = kStep ? kStepFlags : run_flags;
     __shared__ float ibox[3][6];
     const int tid = threadIdx.x;
     const bool node = tid < kNodes;
     // a multi-system step walks the compact list of live slots (k_live)
     const int nit = kLive ? cld(p.n_live) : r.slot_hi - r.slot_lo;
-    for (int it = xcd_block(); it < nit; it += gridDim.x) {
+    for (int it = first_cell<kLive>(nit); it < nit; it += gridDim.x) {
         const int2 at = cell_at<kLive>(p, r, p.LIVE, it);
         const int slot = at.x, s = at.y;
         // the cell's node data are loaded before the system checks (every slot of the
@@ -507,34 +542,37 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
         // (plain 64-bit node indices here: measured faster for this short kernel than
         // the uniform-base form of the other cell kernels)
         const int64_t gi = (int64_t)slot * kSlots + tid;
-        float x = p.X[gi], y = p.Y[gi], z = p.Z[gi];
+        float x = load_now(p.X + gi), y = load_now(p.Y + gi), z = load_now(p.Z + gi);
         const bool kick = flags & I_KICK;
         float vx = 0.f, vy = 0.f, vz = 0.f, fcx = 0.f, fcy = 0.f, fcz = 0.f, fdx = 0.f, fdy = 0.f, fdz = 0.f;
         if (kick) {
-            vx = p.VX[gi]; vy = p.VY[gi]; vz = p.VZ[gi];
-            fcx = p.FCX[gi]; fcy = p.FCY[gi]; fcz = p.FCZ[gi];
-            fdx = p.FDX[gi]; fdy = p.FDY[gi]; fdz = p.FDZ[gi];
+            vx = load_now(p.VX + gi); vy = load_now(p.VY + gi); vz = load_now(p.VZ + gi);
+            fcx = load_now(p.FCX + gi); fcy = load_now(p.FCY + gi); fcz = load_now(p.FCZ + gi);
+            fdx = load_now(p.FDX + gi); fdy = load_now(p.FDY + gi); fdz = load_now(p.FDZ + gi);
         }
-        if (s < 0) continue;
         // metadata and parameters through scalar loads: this kernel writes no field it
         // reads (only status bits, by atomics)
         SysMeta* M = p.meta + s;
+        asm volatile("" : "+s"(M));  // read in the loop: ahead of it the node loads would wait
         const CMeta MC = cmeta(M);
         const CParams P = cparams(p.prm + s);
-        if (!sys_live(MC)) continue;
-        const int c = slot - MC->base;
-        if (c >= MC->n) continue;
+        // the cell's new box, which a grid rebuild needs, with the same round trip
+        const float* bn = p.BBOXN + (int64_t)slot * 6;
+        const float b[6] = {cld(bn), cld(bn + 1), cld(bn + 2), cld(bn + 3), cld(bn + 4), cld(bn + 5)};
+        const int32_t rebuild = MC->rebuild;
+        asm volatile("" ::"s"(b[0]), "s"(b[1]), "s"(b[2]), "s"(b[3]), "s"(b[4]), "s"(b[5]), "s"(rebuild));
+        int c;
+        if (!cell_live(MC, slot, c)) continue;
         const CPool q = pool_late();  // pointers read again where used (see pool_late)
         bool over = false;  // a voxel count beyond its capacity: looked at after the kick, which need not wait for it
-        if ((flags & I_GRIDCOUNT) && MC->rebuild && !(MC->status & CS3D_SYS_GRID_TOO_LARGE)) {
+        if ((flags & I_GRIDCOUNT) && rebuild && !(MC->status & CS3D_SYS_GRID_TOO_LARGE)) {
             // the grid was rebuilt at the end of the last step: this cell's new bbox
             // becomes the one the contact rule uses, and its voxels are counted
             // (makeNNlist's atomicAdd, propagatebound.cu:246-250) to catch overflow
-            const float* bn = q->BBOXN + (int64_t)slot * 6;
-            float b[6];
+            float mine = b[0];
 #pragma unroll
-            for (int a = 0; a < 6; ++a) b[a] = bn[a];
-            if (tid < 6) q->BBOX[(int64_t)slot * 6 + tid] = b[tid];
+            for (int a = 1; a < 6; ++a) mine = tid == a ? b[a] : mine;
+            if (tid < 6) q->BBOX[(int64_t)slot * 6 + tid] = mine;
             const VoxRange v = vox_range(b, MC, P);
             store_vrange(q->VRANGE, slot, v, tid);
             const int nx = v.ex - v.sx + 1, ny = v.ey - v.sy + 1, nz = v.ez - v.sz + 1;
@@ -754,8 +792,7 @@ __device__ __forceinline__ void angle_quotients(float idk, float ra2, float ya2,
     bool ok = quot_num_ok(idk);
     ok &= quot_ok(ra2);
     ok &= quot_ok(rb2);
-    if (!ok) {
-        slow_path();
+    if (CS3D_SELDOM(!ok)) {
         ca = idk / ra2;
         cb = idk / rb2;
     }
@@ -819,9 +856,9 @@ __device__ __forceinline__ bool angle_pair_fast(float ax, float ay, float az, fl
 
 // The three angles of node tid, (n0,n1), (n1,n2), (n0,n2) (propagate.cu:26-60), to
 // out[18] from its bond vectors, squared lengths b2 and lengths bl: by
-// angle_pair_fast, and where an operand is out of its range again by angle_pair
-// (a loop that is not unrolled, on vectors read again from the positions in LDS:
-// it adds nothing to the registers live in the common path).
+// angle_pair_fast, and in a wave where an operand is out of its range again by
+// angle_pair (a loop that is not unrolled, on vectors read again from the positions in
+// LDS: it adds nothing to the registers live in the common path).
 __device__ __forceinline__ uint32_t node_angles(const float* bx, const float* by, const float* bz, const float* b2,
                                                 const float* bl, const MeshRec& mt, float k, const MeshDev* mesh,
                                                 const float* sx, const float* sy, const float* sz, int tid,
@@ -1051,18 +1088,16 @@ __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always)
     }
     // a multi-system step walks the cells of the systems that search (k_live)
     const int nit = kLive ? cld(p.n_live + 1) : r.slot_hi - r.slot_lo;
-    for (int it = xcd_block(); it < nit; it += gridDim.x) {
+    for (int it = first_cell<kLive>(nit); it < nit; it += gridDim.x) {
         const int2 at = cell_at<kLive>(p, r, p.SRCH, it);
         const int slot = at.x, s = at.y;
-        if (s < 0) continue;
         // metadata and parameters through scalar loads: this kernel writes none of
         // the fields it reads (only status bits, by atomics)
         SysMeta* M = p.meta + s;
         const CMeta MC = cmeta(M);
         const CParams P = cparams(p.prm + s);
-        if (!sys_live(MC) || !(always || MC->need_search)) continue;
-        const int c = slot - MC->base;
-        if (c >= MC->n) continue;
+        int c;
+        if (!cell_live(MC, slot, c) || !(always || MC->need_search)) continue;
         const size_t cb = (size_t)slot * kSlots;  // the cell's first node (uniform)
         const uint32_t ln = lane_index();
         float X = ldu(p.X + cb, ln), Y = ldu(p.Y + cb, ln), Z = ldu(p.Z + cb, ln);
@@ -1177,7 +1212,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
     const bool search = kStep || mode != M_BONDED;
     // a multi-system step walks the compact list of live slots (k_live)
     const int nit = kLive ? cld(p.n_live) : r.slot_hi - r.slot_lo;
-    for (int it = xcd_block(); it < nit; it += gridDim.x) {
+    for (int it = first_cell<kLive>(nit); it < nit; it += gridDim.x) {
         const int2 at = cell_at<kLive>(p, r, p.LIVE, it);
         const int slot = at.x, s = at.y;
         // node data first (every slot of the range is allocated): their latency
@@ -1185,28 +1220,26 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
         const size_t cb = (size_t)slot * kSlots;  // the cell's first node (uniform)
         const uint32_t ln = lane_index();
         const int lt = (int)ln;  // for LDS indices as well: nothing per lane is kept across cells
-        const float X = ldu(rX + cb, ln), Y = ldu(rY + cb, ln), Z = ldu(rZ + cb, ln);
+        const float X = ldu_now(rX + cb, ln), Y = ldu_now(rY + cb, ln), Z = ldu_now(rZ + cb, ln);
         float vX = 0.f, vY = 0.f, vZ = 0.f;
-        if (fused) { vX = ldu(rVX + cb, ln); vY = ldu(rVY + cb, ln); vZ = ldu(rVZ + cb, ln); }
+        if (fused) { vX = ldu_now(rVX + cb, ln); vY = ldu_now(rVY + cb, ln); vZ = ldu_now(rVZ + cb, ln); }
         const int32_t* cand = p.CAND + (size_t)slot * kPMax * kSlots;  // the cell's candidate list (uniform)
         int ncf = 0, key0 = 0, total = 0;
         if (search) {
-            ncf = ldu(p.NCAND + cb, ln);
-            key0 = ldu(cand, ln);  // the first round's keys (in the list's room also where it is shorter)
+            ncf = ldu_now(p.NCAND + cb, ln);
+            key0 = ldu_now(cand, ln);  // the first round's keys (in the list's room also where it is shorter)
             total = cld(p.NCAND + cb + kNodes) >> kCandBits;  // entries of the list, from a padding lane
         }
         const MeshRec mt = ldu(mesh->th, ln);
         const float sg = fused ? ldu(mesh->gs, ln).sign : 0.f;
         const MeshRec r0 = ldu(mesh->r0, ln), ir0 = ldu(mesh->ir0, ln);
-        if (s < 0) continue;
         SysMeta* M = p.meta + s;
-        if (!sys_live(M)) continue;
-        // parameters and the fields of the metadata that this kernel does not write,
-        // through scalar loads
+        // parameters and the fields of the metadata that this kernel does not write
+        // (but for status bits, by atomics), through scalar loads
         const CMeta MC = cmeta(M);
-        const int sbase = MC->base;
-        const int c = slot - sbase;
-        if (c >= MC->n) continue;
+        int c;
+        if (!cell_live(MC, slot, c)) continue;
+        const int sbase = slot - c;
         const CParams P = cparams(p.prm + s);
         sx[lt] = X; sy[lt] = Y; sz[lt] = Z;
         if (fused) { svx[lt] = vX; svy[lt] = vY; svz[lt] = vZ; }
@@ -1250,8 +1283,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
                     FY += ty;
                     FZ += tz;
                 }
-                if (!ok) {  // an operand out of range: the three springs by division
-                    slow_path();
+                if (CS3D_SELDOM(!ok)) {  // an operand out of range: the three springs by division
                     FX = 0.f; FY = 0.f; FZ = 0.f;
 #pragma unroll
                     for (int i = 0; i < 3; ++i) {
@@ -1485,8 +1517,7 @@ __global__ __launch_bounds__(192) void k_bonded(Pool p, Range r) {
                     FY += ty;
                     FZ += tz;
                 }
-                if (!ok) {  // an operand out of range: the three springs by division
-                    slow_path();
+                if (CS3D_SELDOM(!ok)) {  // an operand out of range: the three springs by division
                     FX = 0.f; FY = 0.f; FZ = 0.f;
 #pragma unroll
                     for (int i = 0; i < 3; ++i) {
@@ -1600,7 +1631,7 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
     constexpr bool fused = kStep;
     // a multi-system step walks the compact list of live slots (k_live)
     const int nit = kLive ? cld(p.n_live) : r.slot_hi - r.slot_lo;
-    for (int it = xcd_block(); it < nit; it += gridDim.x) {
+    for (int it = first_cell<kLive>(nit); it < nit; it += gridDim.x) {
         const int2 at = cell_at<kLive>(p, r, p.LIVE, it);
         const int slot = at.x, s = at.y;
         // node data first (every slot of the range is allocated): their latency
@@ -1608,36 +1639,34 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
         const size_t cb = (size_t)slot * kSlots;  // the cell's first node (uniform)
         const uint32_t ln = lane_index();
         const int lt = (int)ln;
-        const float X = ldu(rX + cb, ln), Y = ldu(rY + cb, ln), Z = ldu(rZ + cb, ln);
+        const float X = ldu_now(rX + cb, ln), Y = ldu_now(rY + cb, ln), Z = ldu_now(rZ + cb, ln);
         float vX = 0.f, vY = 0.f, vZ = 0.f;
         const int32_t* cand = p.CAND + (size_t)slot * kPMax * kSlots;
         const uint64_t* mask = pair_mask(p.CAND, slot);
         int ncf = 0, total = 0, key[2] = {0, 0};
         uint64_t m[2] = {0, 0};  // this wave's words of the first round
         if (do_dis) {
-            vX = ldu(rVX + cb, ln); vY = ldu(rVY + cb, ln); vZ = ldu(rVZ + cb, ln);
-            ncf = ldu(p.NCAND + cb, ln);
-            key[0] = ldu(cand, ln); key[1] = ldu(cand, ln + kSlots);
+            vX = ldu_now(rVX + cb, ln); vY = ldu_now(rVY + cb, ln); vZ = ldu_now(rVZ + cb, ln);
+            ncf = ldu_now(p.NCAND + cb, ln);
+            key[0] = ldu_now(cand, ln); key[1] = ldu_now(cand, ln + kSlots);
             total = cld(p.NCAND + cb + kNodes) >> kCandBits;
             m[0] = cld(mask + wv); m[1] = cld(mask + 3 + wv);
         }
         float fcX = 0.f, fcY = 0.f, fcZ = 0.f, xbX = 0.f, xbY = 0.f, xbZ = 0.f;
-        if (fused && node) {
-            fcX = ldu(p.FCX + cb, ln); fcY = ldu(p.FCY + cb, ln); fcZ = ldu(p.FCZ + cb, ln);
-            xbX = ldu(p.XBX + cb, ln); xbY = ldu(p.XBY + cb, ln); xbZ = ldu(p.XBZ + cb, ln);
+        if (fused) {  // (padding lanes load their padding)
+            fcX = ldu_now(p.FCX + cb, ln); fcY = ldu_now(p.FCY + cb, ln); fcZ = ldu_now(p.FCZ + cb, ln);
+            xbX = ldu_now(p.XBX + cb, ln); xbY = ldu_now(p.XBY + cb, ln); xbZ = ldu_now(p.XBZ + cb, ln);
         }
         const uint32_t nnw = do_dis ? ldu(mesh->th, ln).w : 0u;
         const float sg = do_dis ? ldu(mesh->gs, ln).sign : 0.f;
-        if (s < 0) continue;
         // metadata and parameters through scalar loads: the fields read here are not
         // written by this kernel (search_next and n_reset, which it updates by atomics,
         // are read by atomic loads)
         SysMeta* M = p.meta + s;
         const CMeta MC = cmeta(M);
         const CParams P = cparams(p.prm + s);
-        if (!sys_live(MC)) continue;
-        const int c = slot - MC->base;
-        if (c >= MC->n) continue;
+        int c;
+        if (!cell_live(MC, slot, c)) continue;
         const int nc = ncf & ((1 << kCandBits) - 1), first = ncf >> kCandBits;
         if (tid == 0) { moved = 0; okm[kRound / 64] = 0; }
         sx[lt] = X; sy[lt] = Y; sz[lt] = Z;
@@ -1993,9 +2022,14 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
     const int32_t m_nreset = MC->n_reset, m_search_next = MC->search_next;
     const int64_t div_time = PC->div_time_steps;
     const int32_t m_gint = PC->grid_interval, m_ccom = PC->correct_com;
-    const float m_rgrowth = rgrowth(PC, n0);
     const GridConsts m_grid = grid_consts(MC, PC);
     const int64_t m_vbase = MC->vbase;
+    // (read here, not behind the branches that use them)
+    asm volatile("" ::"s"(m_active), "s"(n0), "s"(base), "s"(cap), "s"(m_step), "s"(m_horizon), "s"(m_status),
+                 "s"(m_nreset), "s"(m_search_next), "s"(m_cell_steps));
+    asm volatile("" ::"s"(div_time), "s"(m_gint), "s"(m_ccom), "s"(PC->do_pop_model), "s"(PC->growth_rate),
+                 "s"(m_grid.DL), "s"(m_grid.ar), "s"(m_grid.skin), "s"(m_grid.vbudget), "s"(m_grid.bbudget), "s"(m_vbase));
+    const float m_rgrowth = rgrowth(PC, n0);
     const bool live = m_active && (m_horizon < 0 || m_step < m_horizon) && !(m_status & CS3D_SYS_FATAL_MASK);
     // a stopped system keeps a pending grid adoption: its bboxes are adopted when it
     // resumes or when a caller reads the grid
@@ -2034,19 +2068,20 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
             const uint32_t x = w ^ 0x01010101u;
             return ((x - 0x01010101u) & ~x & 0x80808080u) != 0;
         };
-        constexpr int kVec = 4;  // loads in flight per thread
+        constexpr int kVec = 4;  // loads in flight per thread (past the end: the last again)
         for (int i = tid; i < vecs; i += kVec * 256) {
             uint4 w[kVec];
 #pragma unroll
-            for (int u = 0; u < kVec; ++u) w[u] = i + u * 256 < vecs ? v[i + u * 256] : make_uint4(0, 0, 0, 0);
+            for (int u = 0; u < kVec; ++u) w[u] = v[min(i + u * 256, vecs - 1)];
 #pragma unroll
-            for (int u = 0; u < kVec; ++u) any = any || one(w[u].x) || one(w[u].y) || one(w[u].z) || one(w[u].w);
+            for (int u = 0; u < kVec; ++u) any |= one(w[u].x) | one(w[u].y) | one(w[u].z) | one(w[u].w);
         }
         if (tid < head) any |= F[tid] == 1;
         if (tail + tid < n0) any |= F[tail + tid] == 1;
     }
     any = __syncthreads_or(any);
-    if (any) {
+    if (__builtin_expect(any, 0)) {
+        const CPool late = pool_late();  // its dozen pointers are read here only
         // ascending event list in EVL[base .. base + nev), 4096 cells per pass: each
         // thread loads the flags of 16 consecutive cells at once and counts them, a scan
         // of the counts (shuffles within a wave, then the four wave totals) gives the
@@ -2057,7 +2092,7 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
             const int cr = c0 + kRun * tid;
             int8_t f[kRun];
 #pragma unroll
-            for (int j = 0; j < kRun; ++j) f[j] = cr + j < n0 ? p.FLAG[base + cr + j] : (int8_t)0;
+            for (int j = 0; j < kRun; ++j) f[j] = cr + j < n0 ? late->FLAG[base + cr + j] : (int8_t)0;
             int cnt = 0;
 #pragma unroll
             for (int j = 0; j < kRun; ++j) cnt += f[j] == 1 ? 1 : 0;
@@ -2076,8 +2111,8 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
 #pragma unroll
                 for (int j = 0; j < kRun; ++j)
                     if (f[j] == 1) {
-                        p.EVL[base + e++] = cr + j;
-                        p.FLAG[base + cr + j] = 0;
+                        late->EVL[base + e++] = cr + j;
+                        late->FLAG[base + cr + j] = 0;
                     }
             }
             listed += wsum[0] + wsum[1] + wsum[2] + wsum[3];
@@ -2097,18 +2132,18 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
             }
             __syncthreads();
             if (stop) break;
-            const int rank = p.EVL[base + e];
+            const int rank = late->EVL[base + e];
             const int d = ncur;
             const int64_t pi = (int64_t)(base + rank) * kSlots + tid;
             const int64_t di = (int64_t)(base + d) * kSlots + tid;
-            const float cmx = p.CMX[base + rank], cmy = p.CMY[base + rank], cmz = p.CMZ[base + rank];
+            const float cmx = late->CMX[base + rank], cmy = late->CMY[base + rank], cmz = late->CMZ[base + rank];
             // bboxes of parent and daughter after the split (min/max pairs: parent x, y,
             // z, then daughter x, y, z)
             float bx[12];
 #pragma unroll
             for (int a = 0; a < 12; a += 2) { bx[a] = INFINITY; bx[a + 1] = -INFINITY; }
             if (tid < kNodes) {
-                const float x0 = p.X[pi], y0 = p.Y[pi], z0 = p.Z[pi];
+                const float x0 = late->X[pi], y0 = late->Y[pi], z0 = late->Z[pi];
 #pragma unroll
                 for (int side = 0; side < 2; ++side) {  // CalcAndUpdateDaughtPos, postscriptinit.cu:148-182
                     const float Nx = side ? -1 * nrm[0] : nrm[0];
@@ -2119,31 +2154,31 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
                     if (pd < 0.0f || pd == 0) { x = x - pd * Nx; y = y - pd * Ny; z = z - pd * Nz; }
                     x = x + (cmx + half * Nx); y = y + (cmy + half * Ny); z = z + (cmz + half * Nz);
                     const int64_t o = side ? di : pi;
-                    p.X[o] = x; p.Y[o] = y; p.Z[o] = z;
+                    late->X[o] = x; late->Y[o] = y; late->Z[o] = z;
                     bx[6 * side + 0] = x; bx[6 * side + 1] = x;
                     bx[6 * side + 2] = y; bx[6 * side + 3] = y;
                     bx[6 * side + 4] = z; bx[6 * side + 5] = z;
                 }
-                p.VX[di] = p.VX[pi]; p.VY[di] = p.VY[pi]; p.VZ[di] = p.VZ[pi];
+                late->VX[di] = late->VX[pi]; late->VY[di] = late->VY[pi]; late->VZ[di] = late->VZ[pi];
             } else if (tid < kSlots) {
-                p.X[di] = 0.f; p.Y[di] = 0.f; p.Z[di] = 0.f;
-                p.VX[di] = 0.f; p.VY[di] = 0.f; p.VZ[di] = 0.f;
+                late->X[di] = 0.f; late->Y[di] = 0.f; late->Z[di] = 0.f;
+                late->VX[di] = 0.f; late->VY[di] = 0.f; late->VZ[di] = 0.f;
             }
             if (tid < kSlots) {  // a new cell's forces start at zero (never-written slots in the reference)
-                p.FCX[di] = 0.f; p.FCY[di] = 0.f; p.FCZ[di] = 0.f;
-                p.FDX[di] = 0.f; p.FDY[di] = 0.f; p.FDZ[di] = 0.f;
+                late->FCX[di] = 0.f; late->FCY[di] = 0.f; late->FCZ[di] = 0.f;
+                late->FDX[di] = 0.f; late->FDY[di] = 0.f; late->FDZ[di] = 0.f;
             }
             if (step_mode) {
                 block_minmax12(bx, mpart, mres);
-                if (tid < 12) p.BBOXN[(int64_t)(base + (tid < 6 ? rank : d)) * 6 + tid % 6] = mres[tid];
+                if (tid < 12) late->BBOXN[(int64_t)(base + (tid < 6 ? rank : d)) * 6 + tid % 6] = mres[tid];
             }
             if (tid == 0) {
                 const int gd = base + d, gp = base + rank;
-                p.E[gd] = P->daught_same_stiffness ? p.E[gp] : P->stiffness1;
-                p.GS[gd] = p.GS[gp];
-                p.CMX[gd] = 0.f; p.CMY[gd] = 0.f; p.CMZ[gd] = 0.f;
-                p.P[gp] = P->min_pressure;
-                p.P[gd] = P->min_pressure;
+                late->E[gd] = P->daught_same_stiffness ? late->E[gp] : P->stiffness1;
+                late->GS[gd] = late->GS[gp];
+                late->CMX[gd] = 0.f; late->CMY[gd] = 0.f; late->CMZ[gd] = 0.f;
+                late->P[gp] = P->min_pressure;
+                late->P[gd] = P->min_pressure;
                 ncur = d + 1;
             }
             __syncthreads();
@@ -2152,13 +2187,13 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
             const int done = ncur - n0;
             for (int e = 0; e < done; ++e) {
                 for (int q = 0; q < 2; ++q) {
-                    const int cell = q ? n0 + e : p.EVL[base + e];
+                    const int cell = q ? n0 + e : late->EVL[base + e];
                     const int64_t o = (int64_t)(base + cell) * kSlots;
                     if (tid < 128) {  // same 256-slot tree as CenterOfMass
                         const bool hi = tid + 128 < kNodes;
-                        redc[0][tid] = p.X[o + tid] + (hi ? p.X[o + tid + 128] : 0.0f);
-                        redc[1][tid] = p.Y[o + tid] + (hi ? p.Y[o + tid + 128] : 0.0f);
-                        redc[2][tid] = p.Z[o + tid] + (hi ? p.Z[o + tid + 128] : 0.0f);
+                        redc[0][tid] = late->X[o + tid] + (hi ? late->X[o + tid + 128] : 0.0f);
+                        redc[1][tid] = late->Y[o + tid] + (hi ? late->Y[o + tid + 128] : 0.0f);
+                        redc[2][tid] = late->Z[o + tid] + (hi ? late->Z[o + tid + 128] : 0.0f);
                     }
                     __syncthreads();
                     if (tid < 64) {
@@ -2172,17 +2207,17 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
                             d = d + __shfl_down(d, k);
                         }
                         if (tid == 0) {
-                            p.CMX[base + cell] = a / 180.0f;
-                            p.CMY[base + cell] = b / 180.0f;
-                            p.CMZ[base + cell] = d / 180.0f;
+                            late->CMX[base + cell] = a / 180.0f;
+                            late->CMY[base + cell] = b / 180.0f;
+                            late->CMZ[base + cell] = d / 180.0f;
                         }
                     }
                     __syncthreads();
                 }
             }
         }
+        __syncthreads();
     }
-    if (any) __syncthreads();
     const int events = ncur - n0;
     const bool rebuild = step_mode && (events > 0 || due);
     if (rebuild) {
@@ -2196,15 +2231,13 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
         // the boxes of 8 cells per thread are loaded before any is reduced (min and max
         // are exact in any order)
         for (int c0 = 0; c0 < ncur; c0 += kUnroll * 256) {
-            if (c0 > 0 || events > 0 || !due) load_boxes(c0, ncur);
+            if (__builtin_expect(c0 > 0 || events > 0 || !due, 0)) load_boxes(c0, ncur);
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) {
-                if (c0 + u * 256 + tid < ncur) {
+            for (int u = 0; u < kUnroll; ++u) {  // (past the end: the last cell's box again)
 #pragma unroll
-                    for (int a = 0; a < 6; a += 2) {
-                        e[a] = fminf(e[a], bb[u][a]);
-                        e[a + 1] = fmaxf(e[a + 1], bb[u][a + 1]);
-                    }
+                for (int a = 0; a < 6; a += 2) {
+                    e[a] = fminf(e[a], bb[u][a]);
+                    e[a + 1] = fmaxf(e[a + 1], bb[u][a + 1]);
                 }
             }
         }
@@ -2224,20 +2257,21 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
             nclear = set_grid_geometry(M, m_grid, x);
         }
         __syncthreads();
-        int32_t* counts = p.vox + m_vbase;
+        int32_t* counts = pool_late()->vox + m_vbase;
         for (int64_t v = tid; v < nclear; v += blockDim.x) counts[v] = 0;
     }
     const bool shift = step_mode && m_ccom;
-    if (shift) {
+    if (__builtin_expect(shift, 0)) {
         // calc_sys_CM (GPUbounce.cu:2504-2520): float sums of the cell centres in
         // cell order (daughters of this step still hold 0), divided by the count;
         // the nodes are shifted by k_com_shift (CorrectCoMMotion, propagate.cu:766-776)
+        const CPool q = pool_late();
         float acc = 0.f;  // lanes 0..2: one component each
         for (int c0 = 0; c0 < ncur; c0 += 128) {
             if (tid < 128 && c0 + tid < ncur) {
-                redc[0][tid] = p.CMX[base + c0 + tid];
-                redc[1][tid] = p.CMY[base + c0 + tid];
-                redc[2][tid] = p.CMZ[base + c0 + tid];
+                redc[0][tid] = q->CMX[base + c0 + tid];
+                redc[1][tid] = q->CMY[base + c0 + tid];
+                redc[2][tid] = q->CMZ[base + c0 + tid];
             }
             __syncthreads();
             if (tid < 3) {
@@ -2280,14 +2314,16 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
             const int lim = min(kMaxPartial, cap);
             bool full = (events == 0 && m_search_next) || nr > lim || nr + 2 * events > lim ||
                         (shift && (events > 0 || m_search_next));
-            if (!full)
+            if (!full && events > 0) {
+                const CPool q = pool_late();
                 for (int e = 0; e < events; ++e) {
-                    const int pc = p.EVL[base + e], dc = n0 + e;
-                    p.RSL[base + nr++] = pc;
-                    p.RSL[base + nr++] = dc;
-                    p.RESET[base + pc] = 1;
-                    p.RESET[base + dc] = 1;
+                    const int pc = q->EVL[base + e], dc = n0 + e;
+                    q->RSL[base + nr++] = pc;
+                    q->RSL[base + nr++] = dc;
+                    q->RESET[base + pc] = 1;
+                    q->RESET[base + dc] = 1;
                 }
+            }
             M->need_search = full ? 1 : (nr > 0 ? 2 : 0);
             M->n_reset = full ? 0 : nr;
             M->search_next = 0;
@@ -2889,10 +2925,10 @@ void launch_room_free(const Pool& p, int base, int cap, int sys, int nsys, hipSt
 }
 
 void launch_integrate(const Pool& p, const Range& r, int flags, int64_t step_override, hipStream_t st) {
-    if (r.live)
-        launch(k_integrate<1>, dim3(grid_step(r, p.wg_per_cu)), dim3(192), st, p, r, flags, step_override);
-    else
-        launch(k_integrate<0>, dim3(grid_step(r, p.wg_per_cu)), dim3(192), st, p, r, flags, step_override);
+    const dim3 grid(grid_step(r, p.wg_per_cu)), block(192);
+    if (flags != kStepFlags) launch(k_integrate<0, false>, grid, block, st, p, r, flags, step_override);  // one system
+    else if (r.live) launch(k_integrate<1, true>, grid, block, st, p, r, flags, step_override);
+    else launch(k_integrate<0, true>, grid, block, st, p, r, flags, step_override);
 }
 void launch_search(const Pool& p, const Range& r, int always, hipStream_t st) {
     const int g = grid_step(r, p.wg_per_cu);
