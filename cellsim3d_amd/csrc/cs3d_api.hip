@@ -23,7 +23,7 @@
 namespace cs3d {
 void launch_integrate(const Pool& p, const Range& r, int flags, int64_t step_override, hipStream_t st);
 void launch_search(const Pool& p, const Range& r, int always, hipStream_t st);
-void launch_con(const Pool& p, const Range& r, int mode, bool use_va, hipStream_t st);
+void launch_con(const Pool& p, const Range& r, int mode, hipStream_t st);
 void launch_dis(const Pool& p, const Range& r, int mode, int64_t step_override, int clear_bins, bool use_va,
                 hipStream_t st);
 void launch_bonded(const Pool& p, const Range& r, int angles, hipStream_t st);
@@ -381,7 +381,7 @@ void enqueue_step_phase(cs3d_ctx* c, const Range& r, int phase) {
             launch_integrate(p, rl, I_KICK | I_PRESSURE | I_BINS | I_IFSEARCH | I_GRIDCOUNT, -1, c->stream);
             break;
         case CS3D_PH_SEARCH: launch_search(p, rl, 0, c->stream); break;
-        case CS3D_PH_CON_DIS: launch_con(p, rl, M_STEP, true, c->stream); break;
+        case CS3D_PH_CON_DIS: launch_con(p, rl, M_STEP, c->stream); break;
         case CS3D_PH_DIS_POST: launch_dis(p, rl, M_STEP, -1, 1, false, c->stream); break;
         case CS3D_PH_DIVIDE:
             launch_divide(p, r, M_STEP, c->stream);
@@ -424,7 +424,7 @@ cs3d_status run_startup(cs3d_ctx* c, cs3d_sys s) {
     // initial CalculateConForce and CalculateDisForce (GPUbounce.cu:978-1004)
     launch_integrate(p, r, I_BINS, 0, c->stream);
     launch_search(p, r, 1, c->stream);
-    launch_con(p, r, M_INIT, false, c->stream);
+    launch_con(p, r, M_INIT, c->stream);
     launch_dis(p, r, M_DIS_V, 0, 1, false, c->stream);
     launch_set_flags(p, r, -1, 0, c->stream);  // candidate lists are current
     HIPCHK(hipGetLastError());
@@ -1462,7 +1462,7 @@ extern "C" cs3d_status cs3d_k_con_force(cs3d_ctx* c, cs3d_sys s) {
     const Range r = range_of(c, s);
     launch_integrate(c->pool, r, I_BINS, 0, c->stream);
     launch_search(c->pool, r, 1, c->stream);
-    launch_con(c->pool, r, M_CON, false, c->stream);
+    launch_con(c->pool, r, M_CON, c->stream);
     pairs_stale(c, s);
     launch_integrate(c->pool, r, I_CLEAR, 0, c->stream);
     launch_set_flags(c->pool, r, -1, 1, c->stream);
@@ -1480,7 +1480,7 @@ extern "C" cs3d_status cs3d_k_dis_force(cs3d_ctx* c, cs3d_sys s, int32_t which) 
     const Range r = range_of(c, s);
     launch_integrate(c->pool, r, I_BINS, 0, c->stream);
     launch_search(c->pool, r, 1, c->stream);
-    launch_con(c->pool, r, M_PAIRS, false, c->stream);
+    launch_con(c->pool, r, M_PAIRS, c->stream);
     pairs_stale(c, s);
     launch_dis(c->pool, r, which ? M_DIS_VA : M_DIS_V, 0, 1, which != 0, c->stream);
     launch_set_flags(c->pool, r, -1, 1, c->stream);

@@ -225,13 +225,20 @@ __device__ __forceinline__ CPool pool_late() {
     return q;
 }
 
+// The kernel's Pool argument as a cell kernel's loop body sees it: read again in every
+// iteration (most workgroups have one).  With the argument itself the compiler computes
+// every address that does not change between iterations ahead of the loop, and spills
+// most of them there: k_con_dis took 8.9 instead of 8.2 us at 8 cells, 144 instead of
+// 137 at 20,000.  (The shorter kernels, which do not spill, are slower with it.)
+#define CS3D_LOOP_POOL(name) const auto& name = *pool_late()
+
 // The cell slot and system of loop iteration `it` of a cell kernel: an entry of a
 // list made by k_live (a multi-system step), read with one scalar load, or the
 // it-th slot of the range.  Wave-uniform: the per-cell base pointers derived from
 // the slot stay in scalar registers instead of becoming per-lane 64-bit induction
 // variables.
 template <int kLive>
-__device__ __forceinline__ int2 cell_at(const Pool& p, const Range& r, const int2* list, int it) {
+__device__ __forceinline__ int2 cell_at(const Range& r, const int2* list, int it) {
     if (kLive) return int2{cld(&list[it].x), cld(&list[it].y)};
     return int2{__builtin_amdgcn_readfirstlane(r.slot_lo + it), r.sys_lo};
 }
@@ -535,7 +542,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
     // a multi-system step walks the compact list of live slots (k_live)
     const int nit = kLive ? cld(p.n_live) : r.slot_hi - r.slot_lo;
     for (int it = first_cell<kLive>(nit); it < nit; it += gridDim.x) {
-        const int2 at = cell_at<kLive>(p, r, p.LIVE, it);
+        const int2 at = cell_at<kLive>(r, p.LIVE, it);
         const int slot = at.x, s = at.y;
         // the cell's node data are loaded before the system checks (every slot of the
         // range is allocated), so their latency overlaps the metadata reads
@@ -1089,7 +1096,7 @@ __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always)
     // a multi-system step walks the cells of the systems that search (k_live)
     const int nit = kLive ? cld(p.n_live + 1) : r.slot_hi - r.slot_lo;
     for (int it = first_cell<kLive>(nit); it < nit; it += gridDim.x) {
-        const int2 at = cell_at<kLive>(p, r, p.SRCH, it);
+        const int2 at = cell_at<kLive>(r, p.SRCH, it);
         const int slot = at.x, s = at.y;
         // metadata and parameters through scalar loads: this kernel writes none of
         // the fields it reads (only status bits, by atomics)
@@ -1192,10 +1199,7 @@ __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always)
 // mode is M_STEP (the fused step has code of its own: as a run-time value the mode
 // took scalar registers, spilled, throughout the kernel)
 template <int kLive, bool kStep>
-__global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_con_dis(Pool p, Range r, int32_t mode, const float* __restrict__ rX,
-                                                 const float* __restrict__ rY, const float* __restrict__ rZ,
-                                                 const float* __restrict__ rVX, const float* __restrict__ rVY,
-                                                 const float* __restrict__ rVZ, const float* __restrict__ rBB) {
+__global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_con_dis(Pool pk, Range r, int32_t mode) {
     __shared__ float sx[kSlots], sy[kSlots], sz[kSlots];
     __shared__ float svx[kSlots], svy[kSlots], svz[kSlots];
     __shared__ float snx[kSlots], sny[kSlots], snz[kSlots];  // friction normals
@@ -1206,14 +1210,18 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
     } u;
     const int tid = threadIdx.x;
     const bool node = tid < kNodes;
-    const MeshDev* mesh = p.mesh;
     constexpr bool fused = kStep;
     const bool forces = kStep || mode != M_PAIRS;
     const bool search = kStep || mode != M_BONDED;
     // a multi-system step walks the compact list of live slots (k_live)
-    const int nit = kLive ? cld(p.n_live) : r.slot_hi - r.slot_lo;
+    const int nit = kLive ? cld(pk.n_live) : r.slot_hi - r.slot_lo;
     for (int it = first_cell<kLive>(nit); it < nit; it += gridDim.x) {
-        const int2 at = cell_at<kLive>(p, r, p.LIVE, it);
+        CS3D_LOOP_POOL(p);
+        const MeshDev* mesh = p.mesh;
+        const float *rX = p.X, *rY = p.Y, *rZ = p.Z, *rVX = p.VAX, *rVY = p.VAY, *rVZ = p.VAZ, *rBB = p.BBOX;
+        asm volatile("" ::"s"(rX), "s"(rY), "s"(rZ), "s"(rVX), "s"(rVY), "s"(rVZ), "s"(mesh), "s"(p.NCAND), "s"(p.CAND),
+                     "s"(p.meta), "s"(p.prm));  // (in one batch)
+        const int2 at = cell_at<kLive>(r, p.LIVE, it);
         const int slot = at.x, s = at.y;
         // node data first (every slot of the range is allocated): their latency
         // overlaps the metadata reads
@@ -1632,7 +1640,7 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
     // a multi-system step walks the compact list of live slots (k_live)
     const int nit = kLive ? cld(p.n_live) : r.slot_hi - r.slot_lo;
     for (int it = first_cell<kLive>(nit); it < nit; it += gridDim.x) {
-        const int2 at = cell_at<kLive>(p, r, p.LIVE, it);
+        const int2 at = cell_at<kLive>(r, p.LIVE, it);
         const int slot = at.x, s = at.y;
         // node data first (every slot of the range is allocated): their latency
         // overlaps the metadata reads
@@ -2937,17 +2945,14 @@ void launch_search(const Pool& p, const Range& r, int always, hipStream_t st) {
     else
         launch(k_search<0>, dim3(g), dim3(192), st, p, r, always);
 }
-void launch_con(const Pool& p, const Range& r, int mode, bool use_va, hipStream_t st) {
-    const float* vx = use_va ? p.VAX : p.VX;
-    const float* vy = use_va ? p.VAY : p.VY;
-    const float* vz = use_va ? p.VAZ : p.VZ;
+void launch_con(const Pool& p, const Range& r, int mode, hipStream_t st) {
     const dim3 grid(grid_step(r, p.wg_per_cu)), block(192);
     if (mode != M_STEP)  // one system
-        launch(k_con_dis<0, false>, grid, block, st, p, r, mode, p.X, p.Y, p.Z, vx, vy, vz, p.BBOX);
+        launch(k_con_dis<0, false>, grid, block, st, p, r, mode);
     else if (r.live)
-        launch(k_con_dis<1, true>, grid, block, st, p, r, mode, p.X, p.Y, p.Z, vx, vy, vz, p.BBOX);
+        launch(k_con_dis<1, true>, grid, block, st, p, r, mode);
     else
-        launch(k_con_dis<0, true>, grid, block, st, p, r, mode, p.X, p.Y, p.Z, vx, vy, vz, p.BBOX);
+        launch(k_con_dis<0, true>, grid, block, st, p, r, mode);
 }
 // angles: 0 = systems without bending, 1 = with, -1 = both launches
 void launch_bonded(const Pool& p, const Range& r, int angles, hipStream_t st) {
