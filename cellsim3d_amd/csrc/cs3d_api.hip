@@ -360,7 +360,8 @@ bool any_correct_com(const cs3d_ctx* c, const Range& r) {
 // One step of the loop in GPUbounce.cu:1055-1506 as five launches:
 //   integrate  Integrate + ForwardTime + PressureUpdate; per-cell part of a grid
 //              rebuilt at the end of the last step; search bins (search steps)
-//   search     contact candidates (steps flagged by the previous step)
+//   search     contact candidates (steps flagged by the previous step); no launch where
+//              con_dis does it (small grids, search_in_con)
 //   con_dis    CalculateConForce + CalculateDisForce (post-Integrate velocities) +
 //              VelocityUpdateA/B
 //   dis_post   CalculateDisForce (end velocities) + CenterOfMass [+ volumes] +

@@ -79,8 +79,9 @@ struct SysMeta {
     int32_t need_search;  // search contact candidates this step: 0 no, 1 every cell, 2 only the
                           // cells near the cells listed in RSL (partial search)
     int32_t search_next;  // set during a step when the next step's drift takes a node pair_skin/2 away
-    int32_t n_reset;      // cells listed in RSL for the next partial search (moved past the skin or
-                          // divided); counts past kMaxPartial mean a full search
+    int32_t n_reset;      // cells that this step has listed in RSL so far (a node leaves the skin);
+                          // counts past kMaxPartial mean a full search
+    int32_t n_part;       // cells in RSL for the partial search of need_search 2 (at most kMaxPartial)
     float sys_cm[3];      // system centre subtracted at the end of the latest step (correct_com)
     int32_t shift_pending;  // 1 = the step that just ended computed sys_cm and its nodes are still to be
                             // shifted (set by the division phase, consumed by the shift kernel)

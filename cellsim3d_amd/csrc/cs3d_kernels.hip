@@ -27,6 +27,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -252,6 +253,12 @@ __device__ __forceinline__ uint32_t lane_index() {
     uint32_t t = threadIdx.x;
     asm volatile("" : "+v"(t));
     return t;
+}
+
+// v in a vector register: an address made from it is read by a vector load.
+__device__ __forceinline__ uint32_t vector_value(uint32_t v) {
+    asm volatile("" : "+v"(v));
+    return v;
 }
 
 // A value read from LDS that the compiler may not replace by a register copy of
@@ -665,7 +672,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
 // ascending in lst[0 .. n)[tid]; returns n.
 // ------------------------------------------------------------------------------
 template <class MP, class PP>
-__device__ int find_candidates(const Pool& p, MP M, PP P, int c, float X, float Y, float Z, int32_t (*lst)[kSlots],
+__device__ int find_candidates(CPool p, MP M, PP P, int c, float X, float Y, float Z, int32_t (*lst)[kSlots],
                                int tid, uint32_t& st) {
     int nc = 0;
     const float rc = P->attraction_range + P->pair_skin;
@@ -674,8 +681,8 @@ __device__ int find_candidates(const Pool& p, MP M, PP P, int c, float X, float 
     const int by = bin1(Y, M->bmin[1], M->bh, M->bdims[1]);
     const int bz = bin1(Z, M->bmin[2], M->bh, M->bdims[2]);
     const int bdx = M->bdims[0], bdy = M->bdims[1], bdz = M->bdims[2];
-    const int32_t* counts = p.bins + M->bbase;
-    const float4* ents = reinterpret_cast<const float4*>(p.bins + M->ebase);
+    const int32_t* counts = p->bins + M->bbase;
+    const float4* ents = reinterpret_cast<const float4*>(p->bins + M->ebase);
     auto consider = [&](const float4 en) {
         const int key = __float_as_int(en.w);
         if ((unsigned)(key - c * kSlots) < (unsigned)kSlots) return;  // a node of this cell
@@ -1079,16 +1086,92 @@ __device__ __forceinline__ void pair_pass(const int32_t* cand, uint64_t* mask, P
 // moved pair_skin/2 since the last search (or always, outside the fused step),
 // rebuild each node's sorted candidate list and remember the positions.
 // ------------------------------------------------------------------------------
+struct SearchLds {
+    int32_t lst[kPMax][kSlots];
+    float part[3][6];
+    int32_t wsum[3];
+    int32_t near;
+};
+
+// The search of one cell (every lane of the workgroup calls it) at its positions X,
+// Y, Z.  Returns whether the cell searched; then first, nc are this lane's entries
+// of the new list and total their number.  u is written only after a barrier that
+// ends its previous use, and is free when it returns.
+template <class MP, class PP>
+__device__ __forceinline__ bool search_cell(CPool p, SysMeta* M, MP MC, PP P, int slot, int c, int tid, bool always,
+                                            float X, float Y, float Z, SearchLds& u, int& first, int& nc, int& total) {
+    const bool node = tid < kNodes;
+    const size_t cb = (size_t)slot * kSlots;  // the cell's first node (uniform)
+    const uint32_t ln = lane_index();
+    bool reset = true;
+    if (!always && MC->need_search == 2) {
+        // Partial search, in search positions.  The cells listed in RSL (RESET: a
+        // node of the cell would leave the skin, or the cell divided) take their
+        // current positions as search positions; every other node is within
+        // pair_skin/2 of its search position.  Invariant: every list holds every
+        // node of another cell within attraction_range + pair_skin in search
+        // positions; with the pair_skin/2 bound it holds every node that is, or
+        // comes, within attraction_range before the next search.  The nodes were
+        // binned at their search positions (k_integrate), and SBOX holds the box of
+        // every cell's search positions (the listed cells' new boxes from
+        // k_integrate).  A cell whose box is farther than that radius from every
+        // listed cell's box keeps its list: the invariant holds for it with the new
+        // search positions.  The listed cells and the cells near them search again
+        // around their search positions, so their lists are as long as after a full
+        // search.
+        const bool own = p->RESET[slot] != 0;
+        if (!own) {
+            const float* ob = p->SBOX + (int64_t)slot * 6;
+            const float b[6] = {ob[0], ob[1], ob[2], ob[3], ob[4], ob[5]};
+            const int nr = MC->n_part;
+            const float mg = P->attraction_range + P->pair_skin;
+            bool hit = false;
+            if (tid < nr) {
+                const int q = p->RSL[MC->base + tid];
+                const float* o = p->SBOX + (int64_t)(MC->base + q) * 6;
+                hit = b[0] - mg <= o[1] && o[0] <= b[1] + mg && b[2] - mg <= o[3] && o[2] <= b[3] + mg &&
+                      b[4] - mg <= o[5] && o[4] <= b[5] + mg;
+            }
+            if (!__syncthreads_or(hit)) return false;
+            X = ldu(p->XBX + cb, ln); Y = ldu(p->XBY + cb, ln); Z = ldu(p->XBZ + cb, ln);
+        }
+        reset = own;
+    } else {
+        // full search: the current positions become the search positions; their box
+        // is kept for later partial searches
+        box_of_cell(X, Y, Z, node, u.part, p->SBOX + (int64_t)slot * 6);
+    }
+    uint32_t st = 0;
+    nc = node ? find_candidates(p, MC, P, c, X, Y, Z, u.lst, tid, st) : 0;
+    // the cell's candidates one after another in node order: an exclusive scan of
+    // the counts (shuffles within a wave, then the wave totals)
+    first = nc;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int t = __shfl_up(first, o);
+        if ((tid & 63) >= o) first += t;
+    }
+    if ((tid & 63) == 63) u.wsum[tid >> 6] = first;
+    __syncthreads();
+    first -= nc;
+    const int w0 = u.wsum[0], w1 = u.wsum[1];
+    total = w0 + w1 + u.wsum[2];
+    if (tid >= 64) first += w0;
+    if (tid >= 128) first += w1;
+    int32_t* cstore = p->CAND + (size_t)slot * kPMax * kSlots;
+    for (int i = 0; i < nc; ++i) stu(cstore, (uint32_t)(first + i), u.lst[i][tid]);
+    stu(p->NCAND + cb, ln, (first << kCandBits) | nc);  // the padding lanes hold the cell's total
+    if (node && reset) { stu(p->XBX + cb, ln, X); stu(p->XBY + cb, ln, Y); stu(p->XBZ + cb, ln, Z); }
+    if (st) flag(M, st);
+    __syncthreads();
+    return true;
+}
+
 // kLive: walk Pool::SRCH (a multi-system step: the cells of the systems that search)
 // instead of the range's slots
 template <int kLive>
 __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always) {
-    __shared__ int32_t lst[kPMax][kSlots];
-    __shared__ float part[3][6];
-    __shared__ int32_t wsum[3];
-    __shared__ int32_t near;
-    const int tid = threadIdx.x;
-    const bool node = tid < kNodes;
+    __shared__ SearchLds u;
     if (r.one_sys && !always) {  // one system: its flag decides for every workgroup
         const CMeta M0 = cmeta(p.meta + r.sys_lo);
         if (!M0->need_search || !sys_live(M0)) return;
@@ -1102,77 +1185,13 @@ __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always)
         // the fields it reads (only status bits, by atomics)
         SysMeta* M = p.meta + s;
         const CMeta MC = cmeta(M);
-        const CParams P = cparams(p.prm + s);
         int c;
         if (!cell_live(MC, slot, c) || !(always || MC->need_search)) continue;
-        const size_t cb = (size_t)slot * kSlots;  // the cell's first node (uniform)
+        const size_t cb = (size_t)slot * kSlots;
         const uint32_t ln = lane_index();
-        float X = ldu(p.X + cb, ln), Y = ldu(p.Y + cb, ln), Z = ldu(p.Z + cb, ln);
-        bool reset = true;
-        if (!always && MC->need_search == 2) {
-            // Partial search, in search positions.  The cells listed in RSL (RESET: a
-            // node of the cell would leave the skin, or the cell divided) take their
-            // current positions as search positions; every other node is within
-            // pair_skin/2 of its search position.  Invariant: every list holds every
-            // node of another cell within attraction_range + pair_skin in search
-            // positions; with the pair_skin/2 bound it holds every node that is, or
-            // comes, within attraction_range before the next search.  The nodes were
-            // binned at their search positions (k_integrate), and SBOX holds the box of
-            // every cell's search positions (the listed cells' new boxes from
-            // k_integrate).  A cell whose box is farther than that radius from every
-            // listed cell's box keeps its list: the invariant holds for it with the new
-            // search positions.  The listed cells and the cells near them search again
-            // around their search positions, so their lists are as long as after a full
-            // search.
-            const bool own = p.RESET[slot] != 0;
-            if (!own) {
-                const float* ob = p.SBOX + (int64_t)slot * 6;
-                const float b[6] = {ob[0], ob[1], ob[2], ob[3], ob[4], ob[5]};
-                const int nr = min(MC->n_reset, kMaxPartial);
-                const float mg = P->attraction_range + P->pair_skin;
-                bool hit = false;
-                if (tid < nr) {
-                    const int q = p.RSL[MC->base + tid];
-                    const float* o = p.SBOX + (int64_t)(MC->base + q) * 6;
-                    hit = b[0] - mg <= o[1] && o[0] <= b[1] + mg && b[2] - mg <= o[3] && o[2] <= b[3] + mg &&
-                          b[4] - mg <= o[5] && o[4] <= b[5] + mg;
-                }
-                if (tid == 0) near = 0;
-                __syncthreads();
-                if (hit) near = 1;
-                __syncthreads();
-                const bool go = near != 0;
-                __syncthreads();  // near is reset by the next cell
-                if (!go) continue;
-                X = ldu(p.XBX + cb, ln); Y = ldu(p.XBY + cb, ln); Z = ldu(p.XBZ + cb, ln);
-            }
-            reset = own;
-        } else {
-            // full search: the current positions become the search positions; their box
-            // is kept for later partial searches
-            box_of_cell(X, Y, Z, node, part, p.SBOX + (int64_t)slot * 6);
-        }
-        uint32_t st = 0;
-        const int nc = node ? find_candidates(p, MC, P, c, X, Y, Z, lst, tid, st) : 0;
-        // the cell's candidates one after another in node order: an exclusive scan of
-        // the counts (shuffles within a wave, then the wave totals)
-        int first = nc;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int t = __shfl_up(first, o);
-            if ((tid & 63) >= o) first += t;
-        }
-        if ((tid & 63) == 63) wsum[tid >> 6] = first;
-        __syncthreads();
-        first -= nc;
-        if (tid >= 64) first += wsum[0];
-        if (tid >= 128) first += wsum[1];
-        int32_t* cstore = p.CAND + (size_t)slot * kPMax * kSlots;
-        for (int i = 0; i < nc; ++i) stu(cstore, (uint32_t)(first + i), lst[i][tid]);
-        stu(p.NCAND + cb, ln, (first << kCandBits) | nc);  // the padding lanes hold the cell's total
-        if (node && reset) { stu(p.XBX + cb, ln, X); stu(p.XBY + cb, ln, Y); stu(p.XBZ + cb, ln, Z); }
-        if (st) flag(M, st);
-        __syncthreads();  // wsum is rewritten by the next cell
+        const float X = ldu(p.X + cb, ln), Y = ldu(p.Y + cb, ln), Z = ldu(p.Z + cb, ln);
+        int first, nc, total;
+        search_cell(pool_late(), M, MC, cparams(p.prm + s), slot, c, threadIdx.x, always, X, Y, Z, u, first, nc, total);
     }
 }
 
@@ -1197,17 +1216,44 @@ __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always)
 // at 2000 cells (2017 to 1088 at 20,000): 22.9 to 21.0 us and 248 to 224 us a launch.
 // kLive: walk Pool::LIVE (a multi-system step) instead of the range's slots; kStep:
 // mode is M_STEP (the fused step has code of its own: as a run-time value the mode
-// took scalar registers, spilled, throughout the kernel)
-template <int kLive, bool kStep>
-__global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_con_dis(Pool pk, Range r, int32_t mode) {
-    __shared__ float sx[kSlots], sy[kSlots], sz[kSlots];
-    __shared__ float svx[kSlots], svy[kSlots], svz[kSlots];
-    __shared__ float snx[kSlots], sny[kSlots], snz[kSlots];  // friction normals
-    __shared__ uint8_t owner[kSlots];
-    __shared__ union {
-        float angF[kNodes * 18];
-        PairLds pr;
-    } u;
+// took scalar registers, spilled, throughout the kernel); kSearch: with the step's
+// search (search_in_con)
+union ForceLds {
+    float angF[kNodes * 18];
+    PairLds pr;
+};
+struct ConLds {
+    float x[9][kSlots];  // positions, velocities and friction normals
+    uint8_t owner[kSlots];
+    ForceLds u;
+};
+union SharedLds {
+    ConLds c;
+    SearchLds s;
+};
+struct NoLds {};
+template <int kLive, bool kStep, bool kSearch>
+__global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(kSearch ? 4 : 6, 8))) void k_con_dis(Pool pk, Range r,
+                                                                                                        int32_t mode) {
+    // the search and the contact pass share LDS; without the search, arrays of their own
+    // (as parts of one object the compiler orders their accesses: 0.2 us at 2000 cells)
+    constexpr int kOwn = kSearch ? 1 : kSlots;
+    __shared__ float x0[kOwn], x1[kOwn], x2[kOwn], x3[kOwn], x4[kOwn], x5[kOwn], x6[kOwn], x7[kOwn], x8[kOwn];
+    __shared__ uint8_t own_owner[kOwn];
+    __shared__ std::conditional_t<kSearch, NoLds, ForceLds> own_u;
+    __shared__ std::conditional_t<kSearch, SharedLds, NoLds> mem;
+    float *sx = x0, *sy = x1, *sz = x2, *svx = x3, *svy = x4, *svz = x5, *snx = x6, *sny = x7, *snz = x8;
+    uint8_t* owner = own_owner;
+    if constexpr (kSearch) {
+        sx = mem.c.x[0]; sy = mem.c.x[1]; sz = mem.c.x[2];
+        svx = mem.c.x[3]; svy = mem.c.x[4]; svz = mem.c.x[5];
+        snx = mem.c.x[6]; sny = mem.c.x[7]; snz = mem.c.x[8];
+        owner = mem.c.owner;
+    }
+    ForceLds& u = [&]() -> ForceLds& {
+        if constexpr (kSearch) return mem.c.u;
+        else return own_u;
+    }();
     const int tid = threadIdx.x;
     const bool node = tid < kNodes;
     constexpr bool fused = kStep;
@@ -1215,6 +1261,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
     const bool search = kStep || mode != M_BONDED;
     // a multi-system step walks the compact list of live slots (k_live)
     const int nit = kLive ? cld(pk.n_live) : r.slot_hi - r.slot_lo;
+    int done = -1;  // kSearch: the iteration whose cell has searched
     for (int it = first_cell<kLive>(nit); it < nit; it += gridDim.x) {
         CS3D_LOOP_POOL(p);
         const MeshDev* mesh = p.mesh;
@@ -1236,7 +1283,9 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
         if (search) {
             ncf = ldu_now(p.NCAND + cb, ln);
             key0 = ldu_now(cand, ln);  // the first round's keys (in the list's room also where it is shorter)
-            total = cld(p.NCAND + cb + kNodes) >> kCandBits;  // entries of the list, from a padding lane
+            // entries of the list, from a padding lane (by a vector load where this kernel
+            // may have just written it: the scalar cache does not see that)
+            total = kSearch ? ldu_now(p.NCAND + cb, vector_value(kNodes)) : cld(p.NCAND + cb + kNodes) >> kCandBits;
         }
         const MeshRec mt = ldu(mesh->th, ln);
         const float sg = fused ? ldu(mesh->gs, ln).sign : 0.f;
@@ -1245,13 +1294,26 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
         // parameters and the fields of the metadata that this kernel does not write
         // (but for status bits, by atomics), through scalar loads
         const CMeta MC = cmeta(M);
+        const int32_t need = kSearch ? MC->need_search : 0;
+        if (kSearch) asm volatile("" ::"s"(need));  // (with the same round trip)
         int c;
         if (!cell_live(MC, slot, c)) continue;
         const int sbase = slot - c;
         const CParams P = cparams(p.prm + s);
+        if constexpr (kSearch) {
+            // the search of this step (search_in_con); the iteration then starts again
+            // with the new list, so that none of its registers live through the search
+            if (__builtin_expect(need && done != it, 0)) {
+                int f, n, t;
+                search_cell(pool_late(), M, MC, P, slot, c, lt, false, X, Y, Z, mem.s, f, n, t);
+                done = it;
+                it -= gridDim.x;
+                continue;
+            }
+        }
         sx[lt] = X; sy[lt] = Y; sz[lt] = Z;
         if (fused) { svx[lt] = vX; svy[lt] = vY; svz[lt] = vZ; }
-        if (fused && tid == 0) {  // the search of this step has used the reset list
+        if (fused && tid == 0) {  // this cell's search of this step is done; k_dis_post lists anew
             p.RESET[slot] = 0;
             if (c == 0) M->n_reset = 0;
         }
@@ -1307,6 +1369,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
                 }
             }
         }
+        if constexpr (kSearch) total = __builtin_amdgcn_readfirstlane(total) >> kCandBits;
         const int nc = ncf & ((1 << kCandBits) - 1), first = ncf >> kCandBits;
         float fdx = 0.f, fdy = 0.f, fdz = 0.f;
         if (search) fill_owners(owner, lt, first, nc, 0);
@@ -2333,7 +2396,7 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
                 }
             }
             M->need_search = full ? 1 : (nr > 0 ? 2 : 0);
-            M->n_reset = full ? 0 : nr;
+            M->n_part = full ? 0 : nr;
             M->search_next = 0;
         } else if (events > 0) {
             M->need_search = 1;
@@ -2938,7 +3001,17 @@ void launch_integrate(const Pool& p, const Range& r, int flags, int64_t step_ove
     else if (r.live) launch(k_integrate<1, true>, grid, block, st, p, r, flags, step_override);
     else launch(k_integrate<0, true>, grid, block, st, p, r, flags, step_override);
 }
+// Whether a step's search runs at the head of k_con_dis (a cell's search needs the bins
+// of k_integrate and nothing of another cell's search) instead of in a launch of its
+// own, which on the many steps that search nothing costs as much as a small kernel.
+// The search's LDS leaves room for 5 workgroups per CU instead of 8, so only where the
+// grid fits the chip at that: a step of 1 cell 18.2 instead of 19.3 us, of 8 cells 22.5
+// instead of 23.6, of 403 28.1 instead of 28.6, of 1000 29.7 instead of 30.5; with 2000
+// cells k_con_dis would take two rounds instead of one.
+static bool search_in_con(const Pool& p, const Range& r) { return grid_step(r, p.wg_per_cu) <= kSearchLive; }
+
 void launch_search(const Pool& p, const Range& r, int always, hipStream_t st) {
+    if (!always && search_in_con(p, r)) return;
     const int g = grid_step(r, p.wg_per_cu);
     if (r.live)
         launch(k_search<1>, dim3(g < kSearchLive ? g : kSearchLive), dim3(192), st, p, r, always);
@@ -2947,12 +3020,11 @@ void launch_search(const Pool& p, const Range& r, int always, hipStream_t st) {
 }
 void launch_con(const Pool& p, const Range& r, int mode, hipStream_t st) {
     const dim3 grid(grid_step(r, p.wg_per_cu)), block(192);
-    if (mode != M_STEP)  // one system
-        launch(k_con_dis<0, false>, grid, block, st, p, r, mode);
-    else if (r.live)
-        launch(k_con_dis<1, true>, grid, block, st, p, r, mode);
-    else
-        launch(k_con_dis<0, true>, grid, block, st, p, r, mode);
+    const bool search = search_in_con(p, r);
+    auto go = [&](auto kernel) { launch(kernel, grid, block, st, p, r, mode); };
+    if (mode != M_STEP) go(k_con_dis<0, false, false>);  // one system
+    else if (r.live) search ? go(k_con_dis<1, true, true>) : go(k_con_dis<1, true, false>);
+    else search ? go(k_con_dis<0, true, true>) : go(k_con_dis<0, true, false>);
 }
 // angles: 0 = systems without bending, 1 = with, -1 = both launches
 void launch_bonded(const Pool& p, const Range& r, int angles, hipStream_t st) {

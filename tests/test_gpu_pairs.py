@@ -6,7 +6,8 @@ pairs per cell), several rounds, nodes whose candidates straddle a round or a
 64-lane word, and lists near the 40-entry limit; and the bonds and angles at the
 edges of the short arithmetic (rest shape, crushed, stretched, bonds at and below
 its range); the division phase's flag test; reads of device memory; batches past one
-scan of the live list; grids smaller than their tissue."""
+scan of the live list; grids smaller than their tissue; the search with the contact
+pass or in its own launch."""
 import numpy as np
 import pytest
 
@@ -250,3 +251,38 @@ def test_grids_smaller_than_the_tissue(oracle_mesh, n, cap, both):
         for f, u, v in zip(fields, a, b):
             k = 2 * n * (1 if f == A.F_VOLUME else 192)
             assert np.array_equal(u[:k], v[:k], equal_nan=True), f
+
+
+@pytest.mark.parametrize("both", [False, True])
+def test_search_in_its_own_launch_or_with_the_contacts(oracle_mesh, both):
+    """1060 cells take more workgroups than a search with the contact pass is allowed, a cap
+    of 4 per CU fewer: the same states, through full and partial searches and divisions."""
+    from cellsim3d_amd import abi as A
+    from cellsim3d_amd import configs, engine
+    n = 1060
+    print("search place, both %d" % both, flush=True)
+    _, X, Y, Z, info = configs.lattice_tissue(n, 0.5, seed=9)
+    rng = np.random.default_rng(9)
+    V = [rng.normal(0, 1.0, n * 192).astype(np.float32) for _ in range(3)]
+    p = configs.base_params(2)
+    p.voxel_capacity = 64
+    p.pair_skin = 0.02
+    p.division_vol = np.float32(1.0005 * info["v0"])
+    p.div_time_steps = 1000
+    fields = (A.F_X, A.F_VY, A.F_FCZ, A.F_FDX, A.F_CANDCOUNT)
+    got = []
+    for cap in (0, 4):
+        with engine.Context(oracle_mesh, capacity_cells=5 * n, voxel_budget=1 << 22, bin_budget=1 << 29) as ctx:
+            if cap:
+                ctx.set_launch(cap)
+            systems = [ctx.add_system(p, X, Y, Z, n, max_cells=2 * n, voxels=1 << 14, V=V) for _ in range(2 if both else 1)]
+            for _ in range(4):
+                (ctx if both else systems[0]).step(13)
+                ctx.sync()
+                got.append([(s.info()[0], s.info()[2], [s.get(f) for f in fields]) for s in systems])
+    assert got[3][0][0] > n
+    for a, b in zip(got[:4], got[4:]):
+        for (na, sa, fa), (nb, sb, fb) in zip(a, b):
+            assert (na, sa) == (nb, sb)
+            for f, u, v in zip(fields, fa, fb):
+                assert np.array_equal(u[:na * 192], v[:na * 192], equal_nan=True), f
