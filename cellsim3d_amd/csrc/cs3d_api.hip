@@ -124,6 +124,7 @@ struct cs3d_ctx {
     cs3d_mesh mesh_host;  // the tables the context was created with (checkpoint check)
     // pinned staging ring of the reads (read_back), allocated at the first one
     char* stage = nullptr;
+    char* stage_small = nullptr;
     hipEvent_t stage_ev[4] = {nullptr, nullptr, nullptr, nullptr};
     void* scratch = nullptr;  // small device buffer of the per-kernel entry points (grown on demand)
     size_t scratch_bytes = 0;
@@ -199,13 +200,14 @@ int vox_blocks_of(cs3d_ctx* c, cs3d_sys s) {
 }
 
 // ---- reading device memory back -------------------------------------------------
-// A copy from the device into pageable memory costs 23 us up to 16 KB, 12 to 31 us to 50 KB
-// and runs at 17 GB/s from 1 MB on (measured on an MI355X).  Here one kernel writes
-// a list of pieces straight into a pinned ring (12 us for a small list, launch and
-// wait included; 51 GB/s), and the host copies them out: by itself below
-// kSerialRead, else with a few threads, which copy one slot of the ring while the
-// kernel fills the next (15.4 MB: 1.12 ms before, 0.38 ms).  One piece between 56 KB
-// and kSerialRead stays a plain copy (60 KB: 13.9 us against 16.9).
+// A copy from the device into pageable memory costs 21 to 25 us up to 16 KB, 10 to 20 us
+// to 256 KB and runs at 17 GB/s from 1 MB on (measured on an MI355X).  Here one kernel
+// writes a list of pieces straight into pinned memory (13 us for a small list, launch
+// and wait included; 51 GB/s), and the host copies them out: by itself below
+// kSerialRead, else with a few threads, which copy one slot of a ring while the
+// kernel fills the next (15.4 MB: 1.12 ms before, 0.38 ms).  One piece between 16 KB
+// and kSerialRead stays a plain copy (16,388 B: 9.9 us against 13.7; 16,384 B: 21.5
+// against 13.5).
 struct ReadSeg {
     const void* dev;
     void* host;
@@ -214,7 +216,8 @@ struct ReadSeg {
 constexpr size_t kSlotBytes = 2u << 20;  // a ring slot: 40 us of the link, long against a launch
 constexpr int kSlotsInRing = 4;
 constexpr size_t kSerialRead = 1u << 20;  // below, starting threads (45 us) costs more than it gives
-constexpr size_t kPlainFrom = 56u << 10;
+constexpr size_t kPlainFrom = 16u << 10;
+constexpr size_t kSmallBytes = 64u << 10;  // reads that fit this need not allocate the ring
 constexpr int kReaders = 4;
 
 struct ReadPiece {
@@ -222,16 +225,20 @@ struct ReadPiece {
     size_t off, bytes;  // offset in the slot
 };
 
-bool stage_ready(cs3d_ctx* c) {
-    if (c->stage) return true;
+// Pinned memory of the context for reads, made when first needed: a small piece, and
+// the ring for reads that do not fit that.
+bool stage_ready(cs3d_ctx* c, bool small) {
+    char*& at = small ? c->stage_small : c->stage;
+    if (at) return true;
     int before = c->device;
     (void)hipGetDevice(&before);
     void* q = nullptr;
     // coherent: what a finished kernel wrote is what the host reads
     bool ok = hipSetDevice(c->device) == hipSuccess &&
-              hipHostMalloc(&q, kSlotBytes * kSlotsInRing, hipHostMallocPortable | hipHostMallocCoherent) == hipSuccess;
+              hipHostMalloc(&q, small ? kSmallBytes : kSlotBytes * kSlotsInRing,
+                            hipHostMallocPortable | hipHostMallocCoherent) == hipSuccess;
     for (hipEvent_t& e : c->stage_ev) ok = ok && (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess);
-    if (ok) c->stage = static_cast<char*>(q);
+    if (ok) at = static_cast<char*>(q);
     else if (q) (void)hipHostFree(q);
     if (!ok) (void)hipGetLastError();
     (void)hipSetDevice(before);
@@ -253,7 +260,10 @@ cs3d_status read_back(cs3d_ctx* c, const ReadSeg* segs, int n_segs) {
     for (int i = 0; i < n_segs; ++i)
         words = words && segs[i].bytes % 4 == 0 && reinterpret_cast<uintptr_t>(segs[i].dev) % 4 == 0;
     const bool plain = n_segs == 1 && segs[0].bytes > kPlainFrom && segs[0].bytes < kSerialRead;
-    if (!words || plain || !stage_ready(c)) {
+    size_t room = 0;  // in a slot, with the alignment of the pieces
+    for (int i = 0; i < n_segs; ++i) room += (segs[i].bytes + 15) / 16 * 16;
+    const bool small = room <= kSmallBytes && n_segs <= kMaxGather;
+    if (!words || plain || !stage_ready(c, small)) {
         for (int i = 0; i < n_segs; ++i)
             if (segs[i].bytes)
                 HIPCHK(hipMemcpyAsync(segs[i].host, segs[i].dev, segs[i].bytes, hipMemcpyDeviceToHost, c->stream));
@@ -288,7 +298,7 @@ cs3d_status read_back(cs3d_ctx* c, const ReadSeg* segs, int n_segs) {
         HIPCHK(hipStreamSynchronize(c->stream));
         return CS3D_OK;
     }
-    auto slot = [&](int k) { return c->stage + (size_t)(k % kSlotsInRing) * kSlotBytes; };
+    auto slot = [&](int k) { return small ? c->stage_small : c->stage + (size_t)(k % kSlotsInRing) * kSlotBytes; };
     std::atomic<int> ready{0};            // slots whose data has arrived
     std::atomic<bool> stop{false};
     std::vector<std::atomic<int>> done(n);  // readers that have copied slot k
@@ -633,6 +643,7 @@ extern "C" cs3d_status cs3d_ctx_destroy(cs3d_ctx* c) {
     for (hipEvent_t e : c->stage_ev)
         if (e) (void)hipEventDestroy(e);
     if (c->stage) (void)hipHostFree(c->stage);
+    if (c->stage_small) (void)hipHostFree(c->stage_small);
     for (void* q : c->allocs) (void)hipFree(q);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
