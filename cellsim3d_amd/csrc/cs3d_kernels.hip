@@ -576,7 +576,10 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
         const int32_t rebuild = MC->rebuild;
         asm volatile("" ::"s"(b[0]), "s"(b[1]), "s"(b[2]), "s"(b[3]), "s"(b[4]), "s"(b[5]), "s"(rebuild));
         int c;
-        if (!cell_live(MC, slot, c)) continue;
+        if (!cell_live(MC, slot, c)) {
+            if (kLive) continue;
+            break;  // one system: neither is any cell after it
+        }
         const CPool q = pool_late();  // pointers read again where used (see pool_late)
         bool over = false;  // a voxel count beyond its capacity: looked at after the kick, which need not wait for it
         if ((flags & I_GRIDCOUNT) && rebuild && !(MC->status & CS3D_SYS_GRID_TOO_LARGE)) {
@@ -1186,7 +1189,10 @@ __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always)
         SysMeta* M = p.meta + s;
         const CMeta MC = cmeta(M);
         int c;
-        if (!cell_live(MC, slot, c) || !(always || MC->need_search)) continue;
+        if (!cell_live(MC, slot, c) || !(always || MC->need_search)) {
+            if (kLive) continue;
+            break;
+        }
         const size_t cb = (size_t)slot * kSlots;
         const uint32_t ln = lane_index();
         const float X = ldu(p.X + cb, ln), Y = ldu(p.Y + cb, ln), Z = ldu(p.Z + cb, ln);
@@ -1260,7 +1266,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(kSearch ? 4
     const bool forces = kStep || mode != M_PAIRS;
     const bool search = kStep || mode != M_BONDED;
     // a multi-system step walks the compact list of live slots (k_live)
-    const int nit = kLive ? cld(pk.n_live) : r.slot_hi - r.slot_lo;
+    int nit = kLive ? cld(pk.n_live) : r.slot_hi - r.slot_lo;
     int done = -1;  // kSearch: the iteration whose cell has searched
     for (int it = first_cell<kLive>(nit); it < nit; it += gridDim.x) {
         CS3D_LOOP_POOL(p);
@@ -1297,7 +1303,10 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(kSearch ? 4
         const int32_t need = kSearch ? MC->need_search : 0;
         if (kSearch) asm volatile("" ::"s"(need));  // (with the same round trip)
         int c;
-        if (!cell_live(MC, slot, c)) continue;
+        if (!cell_live(MC, slot, c)) {
+            if (!kLive) nit = 0;  // one system: neither is any cell after it
+            continue;
+        }
         const int sbase = slot - c;
         const CParams P = cparams(p.prm + s);
         if constexpr (kSearch) {
@@ -1737,7 +1746,10 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
         const CMeta MC = cmeta(M);
         const CParams P = cparams(p.prm + s);
         int c;
-        if (!cell_live(MC, slot, c)) continue;
+        if (!cell_live(MC, slot, c)) {
+            if (kLive) continue;
+            break;  // one system: neither is any cell after it
+        }
         const int nc = ncf & ((1 << kCandBits) - 1), first = ncf >> kCandBits;
         if (tid == 0) { moved = 0; okm[kRound / 64] = 0; }
         sx[lt] = X; sy[lt] = Y; sz[lt] = Z;
@@ -2535,7 +2547,10 @@ __global__ __launch_bounds__(192) void k_com_shift(Pool p, Range r) {
         const int s = sys_of(p, r, slot);
         if (s < 0) continue;
         const SysMeta* M = p.meta + s;
-        if (!M->shift_pending || slot - M->base >= M->n) continue;
+        if (!M->shift_pending || slot - M->base >= M->n) {
+            if (r.one_sys) break;
+            continue;
+        }
         const int64_t gi = (int64_t)slot * kSlots + tid;
         p.X[gi] = p.X[gi] - M->sys_cm[0];
         p.Y[gi] = p.Y[gi] - M->sys_cm[1];
@@ -2958,7 +2973,7 @@ static void launch(F kernel, dim3 grid, dim3 block, hipStream_t st, A... args) {
 
 // Grid of a step's cell kernel: a workgroup for each live cell that the host knows of
 // and a quarter more (cells that divide before it looks again; beyond the grid the
-// workgroups stride), at most 256 CUs x wg_per_cu if the caller set that.  One cell per
+// workgroups stride, up to the system's last live cell), at most 256 CUs x wg_per_cu if the caller set that.  One cell per
 // workgroup lets the dispatcher even out the load: at 20,000 cells k_con_dis takes
 // 156 us, with 4096 workgroups of 4 or 5 cells 183 us, with 2048 172 us, with 6144
 // 197 us (k_dis_post 94, 109, 103, 118).  A workgroup without a cell still costs its
@@ -3049,7 +3064,7 @@ void launch_divide(const Pool& p, const Range& r, int mode, hipStream_t st) {
     launch(k_sys_divide, dim3(ns < 1 ? 1 : (ns < kSysBlocks ? ns : kSysBlocks)), dim3(256), st, p, r, mode);
 }
 void launch_com_shift(const Pool& p, const Range& r, hipStream_t st) {
-    launch(k_com_shift, dim3(grid_step(r, p.wg_per_cu)), dim3(kSlots), st, p, r);
+    launch(k_com_shift, dim3(r.one_sys ? grid_step(r, p.wg_per_cu) : grid_cells(r, p.wg_per_cu)), dim3(kSlots), st, p, r);
 }
 void launch_grid(const Pool& p, const Range& r, int vox_blocks, hipStream_t st) {
     const int n = r.slot_hi - r.slot_lo;
