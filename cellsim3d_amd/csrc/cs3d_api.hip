@@ -23,6 +23,7 @@
 namespace cs3d {
 void launch_integrate(const Pool& p, const Range& r, int flags, int64_t step_override, hipStream_t st);
 void launch_search(const Pool& p, const Range& r, int always, hipStream_t st);
+int cells_covered(const Range& r);
 void launch_con(const Pool& p, const Range& r, int mode, hipStream_t st);
 void launch_dis(const Pool& p, const Range& r, int mode, int64_t step_override, int clear_bins, bool use_va,
                 hipStream_t st);
@@ -90,7 +91,6 @@ struct RangeAlloc {
 struct SysHost {
     bool used = false;
     int32_t base = 0, cap = 0;
-    int32_t n_seen = 0;  // live cells when the host last looked
     int64_t vreg = 0;  // voxel region offset
     int32_t vbudget = 0, vcap = 0;
     int64_t breg = 0;  // search-bin region offset
@@ -118,7 +118,7 @@ struct cs3d_ctx {
         hipGraphExec_t exec;
         int steps;
         bool shift;  // the captured steps include CorrectCoMMotion
-        int32_t live;  // Range::live_hint at the capture
+        int32_t grid;  // live cells that its grids cover without striding
     };
     std::map<int, GraphRec> graphs;  // target -> captured steps
     cs3d_mesh mesh_host;  // the tables the context was created with (checkpoint check)
@@ -160,6 +160,10 @@ void drop_graphs(cs3d_ctx* c, int target_only = -2) {
 
 bool valid_sys(cs3d_ctx* c, cs3d_sys s) { return c && s >= 0 && s < (int)c->sys.size() && c->sys[s].used; }
 
+// A system's live cells as of the latest division phase that has ended, or the last
+// look at its metadata (sizes grids, nothing else).
+int32_t seen(const cs3d_ctx* c, int s) { return *static_cast<const volatile int32_t*>(c->pool.seen + s); }
+
 Range range_of(cs3d_ctx* c, cs3d_sys s) {
     Range r;
     if (s == CS3D_ALL) {
@@ -173,7 +177,7 @@ Range range_of(cs3d_ctx* c, cs3d_sys s) {
         r.live = 0;
         int64_t n = 0;
         for (int i = 0; i < c->nsys_high; ++i)
-            if (c->sys[i].used) n += c->sys[i].n_seen;
+            if (c->sys[i].used) n += seen(c, i);
         r.live_hint = (int32_t)n;
     } else {
         r.slot_lo = c->sys[s].base;
@@ -182,7 +186,7 @@ Range range_of(cs3d_ctx* c, cs3d_sys s) {
         r.sys_hi = s + 1;
         r.one_sys = 1;
         r.live = 0;
-        r.live_hint = c->sys[s].n_seen;
+        r.live_hint = seen(c, s);
     }
     return r;
 }
@@ -350,14 +354,14 @@ cs3d_status read_back(cs3d_ctx* c, const ReadSeg* segs, int n_segs) {
 cs3d_status read_meta(cs3d_ctx* c, cs3d_sys s, SysMeta& m) {
     const ReadSeg seg{c->pool.meta + s, &m, sizeof(SysMeta)};
     const cs3d_status st = read_back(c, &seg, 1);
-    if (st == CS3D_OK) c->sys[s].n_seen = m.n;
+    if (st == CS3D_OK) c->pool.seen[s] = m.n;
     return st;
 }
 
 cs3d_status write_meta(cs3d_ctx* c, cs3d_sys s, const SysMeta& m) {
     HIPCHK(hipMemcpyAsync(c->pool.meta + s, &m, sizeof(SysMeta), hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
-    c->sys[s].n_seen = m.n;
+    c->pool.seen[s] = m.n;
     return CS3D_OK;
 }
 
@@ -620,6 +624,11 @@ extern "C" cs3d_status cs3d_ctx_create(int device, const cs3d_mesh* mesh, int64_
     if ((st = dalloc(c, p.slot_sys, capacity_cells)) != CS3D_OK) return cleanup(st);
     if ((st = dalloc(c, p.nsys, 1)) != CS3D_OK) return cleanup(st);
     if ((st = dalloc(c, p.meta, kMaxSys)) != CS3D_OK) return cleanup(st);
+    void* live = nullptr;  // coherent: the host reads it while kernels run
+    if (hipHostMalloc(&live, kMaxSys * sizeof(int32_t), hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess)
+        return cleanup(fail(CS3D_OUT_OF_MEMORY, "live counts"));
+    std::memset(live, 0, kMaxSys * sizeof(int32_t));
+    p.seen = static_cast<int32_t*>(live);
     cs3d_params* prm = nullptr;
     if ((st = dalloc(c, prm, kMaxSys)) != CS3D_OK) return cleanup(st);
     p.prm = prm;
@@ -642,6 +651,7 @@ extern "C" cs3d_status cs3d_ctx_destroy(cs3d_ctx* c) {
     drop_graphs(c);
     for (hipEvent_t e : c->stage_ev)
         if (e) (void)hipEventDestroy(e);
+    if (c->pool.seen) (void)hipHostFree(c->pool.seen);
     if (c->stage) (void)hipHostFree(c->stage);
     if (c->stage_small) (void)hipHostFree(c->stage_small);
     for (void* q : c->allocs) (void)hipFree(q);
@@ -694,7 +704,7 @@ cs3d_status room_add(cs3d_ctx* c, const cs3d_params* prm, int32_t n_cells, int32
     h.used = true;
     h.base = (int32_t)base;
     h.cap = max_cells;
-    h.n_seen = n_cells;
+    c->pool.seen[sid] = n_cells;
     h.vreg = vreg;
     h.vbudget = (int32_t)vb;
     h.vcap = vcap;
@@ -926,7 +936,7 @@ extern "C" cs3d_status cs3d_get_state(cs3d_ctx* c, cs3d_sys s, float* xyz, float
             if (cell_to(k, 0)) segs.push_back(ReadSeg{cell[k] + h.base, at, (size_t)h.cap * 4});
         const cs3d_status st = read_back(c, segs.data(), (int)segs.size());
         if (st != CS3D_OK) return st;
-        c->sys[s].n_seen = m.n;
+        c->pool.seen[s] = m.n;
         const size_t n = (size_t)m.n;
         for (int k = 0; k < 6; ++k)
             if (float* q = node_to(k, n)) std::memcpy(q, buf.data() + (size_t)k * h.cap * kSlots, n * kSlots * 4);
@@ -1191,7 +1201,7 @@ extern "C" cs3d_status cs3d_systems_poll(cs3d_ctx* c, int32_t first, int32_t cou
     if (const cs3d_status st = read_back(c, &seg, 1); st != CS3D_OK) return st;
     for (int32_t i = 0; i < count; ++i) {
         const bool used = c->sys[first + i].used;
-        if (used) c->sys[first + i].n_seen = m[i].n;
+        if (used) c->pool.seen[first + i] = m[i].n;
         if (n_cells) n_cells[i] = used ? m[i].n : -1;
         if (steps) steps[i] = used ? m[i].step : -1;
         if (status) status[i] = used ? m[i].status : 0u;
@@ -1365,8 +1375,9 @@ cs3d_status graph_of(cs3d_ctx* c, cs3d_sys s, const cs3d_ctx::GraphRec** out) {
     const Range r = range_of(c, s);
     auto it = c->graphs.find(s);
     // a tissue that has outgrown the grids of its capture (they would stride) is captured
-    // again; the factor keeps that rare
-    if (it != c->graphs.end() && r.live_hint > it->second.live + it->second.live / 2 + 64) {
+    // again: once for every quarter that it grows
+    if (it != c->graphs.end() && r.live_hint > it->second.grid) {
+        HIPCHK(hipStreamSynchronize(c->stream));
         drop_graphs(c, s);
         it = c->graphs.end();
     }
@@ -1385,7 +1396,7 @@ cs3d_status graph_of(cs3d_ctx* c, cs3d_sys s, const cs3d_ctx::GraphRec** out) {
             (void)hipGraphExecDestroy(ex);
             return fail(CS3D_HIP_ERROR, std::string("hipGraphUpload: ") + hipGetErrorString(e));
         }
-        it = c->graphs.emplace(s, cs3d_ctx::GraphRec{ex, c->graph_steps, any_correct_com(c, r), r.live_hint}).first;
+        it = c->graphs.emplace(s, cs3d_ctx::GraphRec{ex, c->graph_steps, any_correct_com(c, r), cells_covered(r)}).first;
     }
     *out = &it->second;
     return CS3D_OK;
@@ -1414,9 +1425,13 @@ extern "C" cs3d_status cs3d_step(cs3d_ctx* c, cs3d_sys s, int32_t n_steps) {
     int done = 0;
     if (c->use_graph && n_steps >= c->graph_steps) {
         const cs3d_ctx::GraphRec* g = nullptr;
-        cs3d_status st = graph_of(c, s, &g);
-        if (st != CS3D_OK) return st;
-        for (; done + g->steps <= n_steps; done += g->steps) HIPCHK(hipGraphLaunch(g->exec, c->stream));
+        do {
+            cs3d_status st = graph_of(c, s, &g);
+            if (st != CS3D_OK) return st;
+            if (done + g->steps > n_steps) break;
+            HIPCHK(hipGraphLaunch(g->exec, c->stream));
+            done += g->steps;
+        } while (done + g->steps <= n_steps);
     }
     for (; done < n_steps; ++done) enqueue_step(c, r, vb);
     HIPCHK(hipGetLastError());

@@ -152,6 +152,8 @@ struct Pool {
     int2* LIVE;      // {slot, system}[cap_cells]: live cells of the stepped systems (k_live)
     int2* SRCH;      // {slot, system}[cap_cells]: those of them whose system searches in this step
     int32_t* n_live; // int32[2]: entries of LIVE and SRCH
+    int32_t* seen;   // int32[kMaxSys], pinned host memory: live cells of each system, written by the
+                     // division phase of a step with divisions; the host sizes grids by it
     int32_t* EVL;
     int32_t* slot_sys;
     int32_t* nsys;   // int32[1]: system ids in use are below this (kernels over all systems read it, so a
@@ -170,7 +172,7 @@ struct Range {
     int32_t sys_lo, sys_hi;
     int32_t one_sys;  // 1: the range is exactly the slot range of system sys_lo
     int32_t live;     // 1: the cell kernels walk Pool::LIVE (built by k_live) instead of the slots
-    int32_t live_hint;  // host side: live cells as of the host's last look (sizes grids, nothing else)
+    int32_t live_hint;  // host side: live cells as far as the host knows (sizes grids, nothing else)
 };
 
 // A system entering its room (k_room_init): its metadata (room, voxel and bin

@@ -27,6 +27,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 #include <vector>
@@ -274,10 +275,13 @@ __device__ __forceinline__ float lds_reread(const float* a, int i) {
 // v mod 8; this maps the 8 XCDs to 8 contiguous runs of workgroup indices, so the
 // cells one XCD works on are neighbours in index and, for tissues placed in
 // order, in space: their partner gathers hit the XCD's own L2.  A bijection on
-// [0, gridDim.x).
+// [0, gridDim.x): on [0, live) if fewer cells than workgroups are known to be live, and
+// the identity beyond, or the last XCDs would have the workgroups without cells (2000
+// cells in a larger room, a grid of 2508: 18 us of k_con_dis became 25).
 constexpr int kXcds = 8;
-__device__ __forceinline__ int xcd_block() {
-    const int G = gridDim.x, v = blockIdx.x;
+__device__ __forceinline__ int xcd_block(int live = 0x7fffffff) {
+    const int G = min((int)gridDim.x, max(live, 1)), v = blockIdx.x;
+    if (v >= G) return v;
     const int q = G / kXcds, rem = G % kXcds;
     const int k = v % kXcds, j = v / kXcds;
     return k * q + min(k, rem) + j;
@@ -285,8 +289,8 @@ __device__ __forceinline__ int xcd_block() {
 
 // The first iteration of a cell kernel's loop over nit cells.  The grid over a range of
 // slots has at most one workgroup per slot, so its loop need not be entered by a test.
-template <int kLive> __device__ __forceinline__ int first_cell(int nit) {
-    const int it = xcd_block();
+template <int kLive> __device__ __forceinline__ int first_cell(int nit, const Range& r) {
+    const int it = xcd_block(r.live_hint);
     if (!kLive) __builtin_assume(it < nit);
     return it;
 }
@@ -548,7 +552,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
     const bool node = tid < kNodes;
     // a multi-system step walks the compact list of live slots (k_live)
     const int nit = kLive ? cld(p.n_live) : r.slot_hi - r.slot_lo;
-    for (int it = first_cell<kLive>(nit); it < nit; it += gridDim.x) {
+    for (int it = first_cell<kLive>(nit, r); it < nit; it += gridDim.x) {
         const int2 at = cell_at<kLive>(r, p.LIVE, it);
         const int slot = at.x, s = at.y;
         // the cell's node data are loaded before the system checks (every slot of the
@@ -1181,7 +1185,7 @@ __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always)
     }
     // a multi-system step walks the cells of the systems that search (k_live)
     const int nit = kLive ? cld(p.n_live + 1) : r.slot_hi - r.slot_lo;
-    for (int it = first_cell<kLive>(nit); it < nit; it += gridDim.x) {
+    for (int it = first_cell<kLive>(nit, r); it < nit; it += gridDim.x) {
         const int2 at = cell_at<kLive>(r, p.SRCH, it);
         const int slot = at.x, s = at.y;
         // metadata and parameters through scalar loads: this kernel writes none of
@@ -1268,7 +1272,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(kSearch ? 4
     // a multi-system step walks the compact list of live slots (k_live)
     int nit = kLive ? cld(pk.n_live) : r.slot_hi - r.slot_lo;
     int done = -1;  // kSearch: the iteration whose cell has searched
-    for (int it = first_cell<kLive>(nit); it < nit; it += gridDim.x) {
+    for (int it = first_cell<kLive>(nit, r); it < nit; it += gridDim.x) {
         CS3D_LOOP_POOL(p);
         const MeshDev* mesh = p.mesh;
         const float *rX = p.X, *rY = p.Y, *rZ = p.Z, *rVX = p.VAX, *rVY = p.VAY, *rVZ = p.VAZ, *rBB = p.BBOX;
@@ -1711,7 +1715,7 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
     constexpr bool fused = kStep;
     // a multi-system step walks the compact list of live slots (k_live)
     const int nit = kLive ? cld(p.n_live) : r.slot_hi - r.slot_lo;
-    for (int it = first_cell<kLive>(nit); it < nit; it += gridDim.x) {
+    for (int it = first_cell<kLive>(nit, r); it < nit; it += gridDim.x) {
         const int2 at = cell_at<kLive>(r, p.LIVE, it);
         const int slot = at.x, s = at.y;
         // node data first (every slot of the range is allocated): their latency
@@ -2300,6 +2304,7 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
             }
         }
         __syncthreads();
+        if (tid == 0) late->seen[s] = ncur;
     }
     const int events = ncur - n0;
     const bool rebuild = step_mode && (events > 0 || due);
@@ -2978,9 +2983,14 @@ static void launch(F kernel, dim3 grid, dim3 block, hipStream_t st, A... args) {
 // 156 us, with 4096 workgroups of 4 or 5 cells 183 us, with 2048 172 us, with 6144
 // 197 us (k_dis_post 94, 109, 103, 118).  A workgroup without a cell still costs its
 // dispatch, 2 to 3 ns, so rooms far larger than their tissue are not launched whole.
+constexpr int kMinGrid = 256;  // one workgroup per CU: a small tissue's growth needs no wider grid
+int cells_covered(const Range& r) {
+    const int64_t slots = r.slot_hi - r.slot_lo, n = (int64_t)r.live_hint + r.live_hint / 4 + 8;
+    return (int)std::min(slots, std::max<int64_t>(n, kMinGrid));
+}
 static int grid_step(const Range& r, int per_cu) {
-    const int64_t slots = r.slot_hi - r.slot_lo, live = (int64_t)r.live_hint + r.live_hint / 4 + 8;
-    const int64_t n = live < slots ? live : slots, cap = per_cu > 0 ? 256 * (int64_t)per_cu : n;
+    const int n = cells_covered(r);
+    const int64_t cap = per_cu > 0 ? 256 * (int64_t)per_cu : n;
     return (int)(n < 1 ? 1 : (n < cap ? n : cap));
 }
 // Grid of the other cell kernels: one workgroup per slot up to 4096, then they stride.
