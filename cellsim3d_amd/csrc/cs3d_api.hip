@@ -371,7 +371,7 @@ bool any_correct_com(const cs3d_ctx* c, const Range& r) {
     return false;
 }
 
-// One step of the loop in GPUbounce.cu:1055-1506 as five launches:
+// One step of the loop in GPUbounce.cu:1055-1506 as four launches, or five:
 //   integrate  Integrate + ForwardTime + PressureUpdate; per-cell part of a grid
 //              rebuilt at the end of the last step; search bins (search steps)
 //   search     contact candidates (steps flagged by the previous step); no launch where
@@ -381,10 +381,10 @@ bool any_correct_com(const cs3d_ctx* c, const Range& r) {
 //   dis_post   CalculateDisForce (end velocities) + CenterOfMass [+ volumes] +
 //              bounding_boxes + next-step search decision
 //   divide     division phase, step bookkeeping, extent and grid geometry
-//              [+ CorrectCoMMotion, a sixth launch, for systems with correct_com]
+//              [+ CorrectCoMMotion, a launch of its own, for systems with correct_com]
 //
-// A step of several systems first lists their live cell slots (k_live); the four
-// cell kernels of the step walk that list.  The division phase adds daughters after
+// A step of several systems first lists their live cell slots (k_live); the cell
+// kernels of the step walk that list.  The division phase adds daughters after
 // them, which the next step's list holds.
 void enqueue_step_phase(cs3d_ctx* c, const Range& r, int phase) {
     const Pool& p = c->pool;

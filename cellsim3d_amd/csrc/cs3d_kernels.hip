@@ -15,14 +15,14 @@
 // search bins of that edge (find_candidates).  The list is rebuilt only on steps where some
 // node has moved pair_skin/2 since the last search, so it always contains every
 // node now within attraction_range; after divisions only the lists near the divided
-// cells are rebuilt (k_search's partial search).  Every step then applies the reference's own
-// tests to the candidates in (cell, node) order -- the order of the reference's
-// loops: the distance test, voxel-list membership and the bbox test
-// (accept_forces).  Voxel-list membership is evaluated arithmetically: makeNNlist
+// cells are rebuilt (the partial search of search_cell).  Every step then applies the
+// reference's own tests to the candidates in (cell, node) order -- the order of the
+// reference's loops: the distance test, voxel-list membership and the bbox test
+// (pair_terms).  Voxel-list membership is evaluated arithmetically: makeNNlist
 // puts cell b into voxel v exactly when v lies in the voxel range of b's bbox
 // widened by attraction_range (propagatebound.cu:224-259), so the same range test
-// on the same bbox and grid answers "b in list(v)".  The accepted pairs are
-// stored for the second friction pass.
+// on the same bbox and grid answers "b in list(v)".  One bit per candidate keeps
+// which pairs were accepted, for the second friction pass.
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -1224,6 +1224,8 @@ __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always)
 // barriers.  Pairs on lanes instead of a loop over each node's candidates, and the
 // angles' short arithmetic, took it from 1577 to 1127 vector instructions per wave
 // at 2000 cells (2017 to 1088 at 20,000): 22.9 to 21.0 us and 248 to 224 us a launch.
+// With friction on accept bits, grids of one workgroup per cell and the entry chain
+// cut (sys_live, CS3D_LOOP_POOL) it takes 18 and 137 us.
 // kLive: walk Pool::LIVE (a multi-system step) instead of the range's slots; kStep:
 // mode is M_STEP (the fused step has code of its own: as a run-time value the mode
 // took scalar registers, spilled, throughout the kernel); kSearch: with the step's

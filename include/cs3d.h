@@ -285,7 +285,7 @@ cs3d_status cs3d_set_graph(cs3d_ctx* ctx, int32_t enable);
 cs3d_status cs3d_set_graph_steps(cs3d_ctx* ctx, int32_t steps);
 /* Launch shape of the cell kernels: at most 256 x wg_per_cu workgroups (one
  * cell each; beyond that a workgroup strides over several cells).  Without a call
- * the step's kernels launch one workgroup per live cell, the others as with 16.
+ * the step's kernels launch about one workgroup per live cell, the others as with 16.
  * No counterpart in the reference (one block per cell, GPUbounce.cu:1059-1164);
  * set by the ensemble autotuner. */
 cs3d_status cs3d_set_launch(cs3d_ctx* ctx, int32_t wg_per_cu);
@@ -305,8 +305,9 @@ cs3d_status cs3d_systems_work(cs3d_ctx* ctx, int32_t first, int32_t count, int64
  * valid when systems are added or removed.  No counterpart in the reference. */
 cs3d_status cs3d_graph_prepare(cs3d_ctx* ctx, cs3d_sys sys);
 
-/* Phases of one step, in launch order (one kernel launch each; the division phase adds
- * CorrectCoMMotion for systems with correct_com). */
+/* Phases of one step, in launch order (one kernel launch each; a small grid's search is
+ * part of the next phase's launch and reads 0; the division phase adds CorrectCoMMotion
+ * for systems with correct_com). */
 #define CS3D_PHASES 5
 #define CS3D_PH_INTEGRATE 0  /* Integrate + ForwardTime + PressureUpdate; adoption of the bboxes and
                                 voxel counts of a grid rebuilt at the end of the previous step;
