@@ -58,7 +58,10 @@ struct SysMeta {
     int32_t active;     // 1 = stepped by cs3d_step
     int64_t step;       // completed steps
     int64_t horizon;    // stop after this many steps (-1 = none)
-    uint32_t status;    // CS3D_SYS_* bits (sticky)
+    uint32_t status;    // CS3D_SYS_* bits (sticky); a fused step changes it in its division phase only
+    uint32_t raised[4];  // status bits found by each phase of the current fused step (R_*): a phase stops for
+                        // what the phases before it found, so that it runs for all cells of a system or none;
+                        // merged into status, and zero again, by the division phase
     int32_t rebuild;    // fused step: 1 = the grid was rebuilt at the end of the last step and its
                         // per-cell part (bbox adoption, voxel counts) is still to be done by the
                         // next step; explicit grid kernels: 1 = rebuild now
@@ -93,6 +96,11 @@ struct SysMeta {
     int32_t kick_fast;    // 1: the constants above reproduce the divisions exactly
     cs3d_ranmar_state rng;
 };
+
+// The phases of a fused step that find status bits (SysMeta::raised), in their order;
+// as a count: the phases that have ended when that one runs.
+enum { R_INTEGRATE = 0, R_SEARCH = 1, R_CON = 2, R_POST = 3, R_PHASES = 4 };
+static_assert(R_PHASES == sizeof(SysMeta::raised) / sizeof(uint32_t), "a word per phase");
 
 // Fills the kick constants of a system with particle mass m and time step dt and
 // checks them exhaustively (on the host; results are cached per (m, dt)).
@@ -148,6 +156,8 @@ struct Pool {
                      // searches, and by k_integrate for RESET cells before a partial search)
     int8_t* RESET;   // int8[cap_cells]: 1 = the cell takes its current positions as search positions at
                      // the next partial search (a node left the skin, or the cell divided)
+    float* KEEP;     // float[cap_cells * 9 * 192]: V, F_con and F_ran before the contact pass of a step that
+                     // searches at its head (put back if the search overflows)
     int32_t* RSL;    // int32[cap_cells]: per system, the local indices of its RESET cells (n_reset)
     int2* LIVE;      // {slot, system}[cap_cells]: live cells of the stepped systems (k_live)
     int2* SRCH;      // {slot, system}[cap_cells]: those of them whose system searches in this step

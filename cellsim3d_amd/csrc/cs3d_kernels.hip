@@ -51,23 +51,33 @@ __device__ __forceinline__ int sys_of(const Pool& p, const Range& r, int slot) {
 // k_integrate.  With it in three, and the division kernel's arguments and metadata read
 // in one batch each, a step took 24.4 instead of 25.6 us at 8 cells, 29.6 instead of
 // 30.9 at 403 and 40.5 instead of 42.3 at 2000.
-template <class MP> __device__ __forceinline__ bool sys_live(MP m) {
+// kEnded: phases of this step that have ended (SysMeta::raised of them stops it).
+template <int kEnded = 0, class MP> __device__ __forceinline__ bool sys_live(MP m) {
     // every field read at once, no short-circuit branches: one memory round trip
     const int32_t active = m->active;
     const int64_t horizon = m->horizon, step = m->step;
-    const uint32_t status = m->status;
-    return (active != 0) & ((horizon < 0) | (step < horizon)) & !(status & CS3D_SYS_FATAL_MASK);
+    uint32_t stop = m->status;
+#pragma unroll
+    for (int k = 0; k < kEnded; ++k) stop |= m->raised[k];
+    return (active != 0) & ((horizon < 0) | (step < horizon)) & !(stop & CS3D_SYS_FATAL_MASK);
 }
 
-// Whether cell slot `slot` of the system is stepped; c: its local index.
-template <class MP> __device__ __forceinline__ bool cell_live(MP m, int slot, int& c) {
+// Whether cell slot `slot` of the system is stepped; c: its local index.  In a fused
+// step no word that it reads changes during the launch, so the waves of a workgroup,
+// which read apart from each other, decide alike, and so do all cells of the system.
+template <int kEnded, class MP> __device__ __forceinline__ bool cell_live(MP m, int slot, int& c) {
     const int32_t base = m->base, n = m->n;
     c = slot - base;
-    return sys_live(m) & (c < n);
+    return sys_live<kEnded>(m) & (c < n);
 }
 
-__device__ __forceinline__ void flag(SysMeta* m, uint32_t bits) {
-    if (bits) atomicOr(&m->status, bits);
+// Status bits found by a kernel: in phase kPhase of a fused step beside the status (the
+// division phase merges them at the end of the step), by an entry point into it.
+template <bool kStep, int kPhase> __device__ __forceinline__ uint32_t* status_word(SysMeta* m) {
+    return kStep ? &m->raised[kPhase] : &m->status;
+}
+__device__ __forceinline__ void flag(uint32_t* word, uint32_t bits) {
+    if (bits) atomicOr(word, bits);
 }
 
 // Loads and stores at a uniform base pointer plus a 32-bit element index: the
@@ -580,10 +590,11 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
         const int32_t rebuild = MC->rebuild;
         asm volatile("" ::"s"(b[0]), "s"(b[1]), "s"(b[2]), "s"(b[3]), "s"(b[4]), "s"(b[5]), "s"(rebuild));
         int c;
-        if (!cell_live(MC, slot, c)) {
+        if (!cell_live<R_INTEGRATE>(MC, slot, c)) {
             if (kLive) continue;
             break;  // one system: neither is any cell after it
         }
+        uint32_t* word = status_word<kStep, R_INTEGRATE>(M);
         const CPool q = pool_late();  // pointers read again where used (see pool_late)
         bool over = false;  // a voxel count beyond its capacity: looked at after the kick, which need not wait for it
         if ((flags & I_GRIDCOUNT) && rebuild && !(MC->status & CS3D_SYS_GRID_TOO_LARGE)) {
@@ -640,7 +651,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
                     float4* ent = reinterpret_cast<float4*>(q->bins + MC->ebase);
                     ent[(int64_t)b * kBCap + k] = make_float4(qx, qy, qz, __int_as_float(c * kSlots + tid));
                 } else {
-                    flag(M, CS3D_SYS_BIN_OVERFLOW);
+                    flag(word, CS3D_SYS_BIN_OVERFLOW);
                 }
             }
         }
@@ -663,7 +674,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
             q->P[slot] = pr;
         }
         if (__any(over) && (tid & 63) == __ffsll((unsigned long long)__ballot(over)) - 1)
-            atomicOr(&M->status, (uint32_t)CS3D_SYS_VOXEL_OVERFLOW);
+            atomicOr(word, (uint32_t)CS3D_SYS_VOXEL_OVERFLOW);
         if (kick && (flags & I_IFSEARCH) && MC->need_search == 2 && q->RESET[slot]) {
             // a cell that divided or left the skin in the last step publishes the box of
             // its new positions: the partial search re-searches the cells within reach
@@ -1101,11 +1112,11 @@ struct SearchLds {
 };
 
 // The search of one cell (every lane of the workgroup calls it) at its positions X,
-// Y, Z.  Returns whether the cell searched; then first, nc are this lane's entries
+// Y, Z (word: where an overflow is noted).  Returns whether the cell searched; then first, nc are this lane's entries
 // of the new list and total their number.  u is written only after a barrier that
 // ends its previous use, and is free when it returns.
 template <class MP, class PP>
-__device__ __forceinline__ bool search_cell(CPool p, SysMeta* M, MP MC, PP P, int slot, int c, int tid, bool always,
+__device__ __forceinline__ bool search_cell(CPool p, uint32_t* word, MP MC, PP P, int slot, int c, int tid, bool always,
                                             float X, float Y, float Z, SearchLds& u, int& first, int& nc, int& total) {
     const bool node = tid < kNodes;
     const size_t cb = (size_t)slot * kSlots;  // the cell's first node (uniform)
@@ -1169,7 +1180,7 @@ __device__ __forceinline__ bool search_cell(CPool p, SysMeta* M, MP MC, PP P, in
     for (int i = 0; i < nc; ++i) stu(cstore, (uint32_t)(first + i), u.lst[i][tid]);
     stu(p->NCAND + cb, ln, (first << kCandBits) | nc);  // the padding lanes hold the cell's total
     if (node && reset) { stu(p->XBX + cb, ln, X); stu(p->XBY + cb, ln, Y); stu(p->XBZ + cb, ln, Z); }
-    if (st) flag(M, st);
+    if (st) flag(word, st);
     __syncthreads();
     return true;
 }
@@ -1181,7 +1192,7 @@ __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always)
     __shared__ SearchLds u;
     if (r.one_sys && !always) {  // one system: its flag decides for every workgroup
         const CMeta M0 = cmeta(p.meta + r.sys_lo);
-        if (!M0->need_search || !sys_live(M0)) return;
+        if (!M0->need_search || !sys_live<R_SEARCH>(M0)) return;
     }
     // a multi-system step walks the cells of the systems that search (k_live)
     const int nit = kLive ? cld(p.n_live + 1) : r.slot_hi - r.slot_lo;
@@ -1193,7 +1204,7 @@ __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always)
         SysMeta* M = p.meta + s;
         const CMeta MC = cmeta(M);
         int c;
-        if (!cell_live(MC, slot, c) || !(always || MC->need_search)) {
+        if (!cell_live<R_SEARCH>(MC, slot, c) || !(always || MC->need_search)) {
             if (kLive) continue;
             break;
         }
@@ -1201,8 +1212,28 @@ __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always)
         const uint32_t ln = lane_index();
         const float X = ldu(p.X + cb, ln), Y = ldu(p.Y + cb, ln), Z = ldu(p.Z + cb, ln);
         int first, nc, total;
-        search_cell(pool_late(), M, MC, cparams(p.prm + s), slot, c, threadIdx.x, always, X, Y, Z, u, first, nc, total);
+        uint32_t* word = always ? status_word<false, R_SEARCH>(M) : status_word<true, R_SEARCH>(M);
+        search_cell(pool_late(), word, MC, cparams(p.prm + s), slot, c, threadIdx.x, always, X, Y, Z, u, first, nc,
+                    total);
     }
+}
+
+// A step whose candidate search overflows ends there: no velocity, force or random
+// force of it is kept.  Where the search runs at the head of k_con_dis the cells of the
+// system cannot know of each other's overflow, so on a step that searches each keeps
+// what the contact pass writes over (keep_cell), and the division phase puts it back
+// (take_back_cell) in a system that overflowed.
+template <class F> __device__ __forceinline__ void kept_arrays(CPool p, bool rands, F&& f) {
+    float* const a[9] = {p->VX, p->VY, p->VZ, p->FCX, p->FCY, p->FCZ, p->FRX, p->FRY, p->FRZ};
+    for (int k = 0; k < (rands ? 9 : 6); ++k) f(a[k], (uint32_t)(k * kSlots));
+}
+__device__ __forceinline__ void keep_cell(CPool p, bool rands, int slot, uint32_t ln) {
+    const size_t cb = (size_t)slot * kSlots;
+    kept_arrays(p, rands, [&](float* a, uint32_t at) { stu(p->KEEP + 9 * cb, at + ln, ldu(a + cb, ln)); });
+}
+__device__ __forceinline__ void take_back_cell(CPool p, bool rands, int slot, uint32_t ln) {
+    const size_t cb = (size_t)slot * kSlots;
+    kept_arrays(p, rands, [&](float* a, uint32_t at) { stu(a + cb, ln, ldu(p->KEEP + 9 * cb, at + ln)); });
 }
 
 // ------------------------------------------------------------------------------
@@ -1309,10 +1340,11 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(kSearch ? 4
         const int32_t need = kSearch ? MC->need_search : 0;
         if (kSearch) asm volatile("" ::"s"(need));  // (with the same round trip)
         int c;
-        if (!cell_live(MC, slot, c)) {
+        if (!cell_live<kStep ? R_CON : 0>(MC, slot, c)) {
             if (!kLive) nit = 0;  // one system: neither is any cell after it
             continue;
         }
+        uint32_t* word = status_word<kStep, R_CON>(M);
         const int sbase = slot - c;
         const CParams P = cparams(p.prm + s);
         if constexpr (kSearch) {
@@ -1320,7 +1352,8 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(kSearch ? 4
             // with the new list, so that none of its registers live through the search
             if (__builtin_expect(need && done != it, 0)) {
                 int f, n, t;
-                search_cell(pool_late(), M, MC, P, slot, c, lt, false, X, Y, Z, mem.s, f, n, t);
+                keep_cell(pool_late(), P->add_rands != 0, slot, ln);
+                search_cell(pool_late(), word, MC, P, slot, c, lt, false, X, Y, Z, mem.s, f, n, t);
                 done = it;
                 it -= gridDim.x;
                 continue;
@@ -1517,7 +1550,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(kSearch ? 4
             const CPool q = pool_late();
             stu(q->FCX + cb, ln, FX); stu(q->FCY + cb, ln, FY); stu(q->FCZ + cb, ln, FZ);
         }
-        if (st) flag(M, st);
+        if (st) flag(word, st);
         __syncthreads();
     }
 }
@@ -1641,7 +1674,7 @@ __global__ __launch_bounds__(192) void k_bonded(Pool p, Range r) {
                 }
                 p.FCX[gi] = FX; p.FCY[gi] = FY; p.FCZ[gi] = FZ;
             }
-            if (st) flag(M, st);
+            if (st) flag(&M->status, st);
             __syncthreads();
         }
         X = Xn; Y = Yn; Z = Zn;
@@ -1752,7 +1785,7 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
         const CMeta MC = cmeta(M);
         const CParams P = cparams(p.prm + s);
         int c;
-        if (!cell_live(MC, slot, c)) {
+        if (!cell_live<kStep ? R_POST : 0>(MC, slot, c)) {
             if (kLive) continue;
             break;  // one system: neither is any cell after it
         }
@@ -1991,7 +2024,7 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
                 }
             }
         }
-        if (st) flag(M, st);
+        if (st) flag(status_word<kStep, R_POST>(M), st);
         __syncthreads();
     }
 }
@@ -2107,7 +2140,10 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
     const CParams PC = cparams(p.prm + s);
     const int32_t m_active = MC->active, n0 = MC->n, base = MC->base, cap = MC->cap;
     const int64_t m_step = MC->step, m_horizon = MC->horizon, m_cell_steps = MC->cell_steps;
-    const uint32_t m_status = MC->status;
+    uint32_t raised[R_PHASES];
+#pragma unroll
+    for (int k = 0; k < R_PHASES; ++k) raised[k] = MC->raised[k];
+    uint32_t m_status = MC->status;
     const int32_t m_nreset = MC->n_reset, m_search_next = MC->search_next;
     const int64_t div_time = PC->div_time_steps;
     const int32_t m_gint = PC->grid_interval, m_ccom = PC->correct_com;
@@ -2119,6 +2155,24 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
     asm volatile("" ::"s"(div_time), "s"(m_gint), "s"(m_ccom), "s"(PC->do_pop_model), "s"(PC->growth_rate),
                  "s"(m_grid.DL), "s"(m_grid.ar), "s"(m_grid.skin), "s"(m_grid.vbudget), "s"(m_grid.bbudget), "s"(m_vbase));
     const float m_rgrowth = rgrowth(PC, n0);
+    // what the phases of this step found becomes status (a candidate overflow in the
+    // contact pass ended the step there: nothing else that was found in it counts)
+    uint32_t found = 0;
+#pragma unroll
+    for (int k = 0; k < R_PHASES; ++k) found |= raised[k];
+    if (__builtin_expect(found != 0, 0)) {
+        if (raised[R_CON] & CS3D_SYS_CAND_OVERFLOW) {
+            found = CS3D_SYS_CAND_OVERFLOW;
+            for (int c = 0; c < n0; ++c)
+                if (tid < kSlots) take_back_cell(pool_late(), PC->add_rands != 0, base + c, (uint32_t)tid);
+        }
+        m_status |= found;
+        __syncthreads();  // every wave has read them
+        if (tid == 0) {
+            M->status = m_status;
+            for (int k = 0; k < R_PHASES; ++k) M->raised[k] = 0;
+        }
+    }
     const bool live = m_active && (m_horizon < 0 || m_step < m_horizon) && !(m_status & CS3D_SYS_FATAL_MASK);
     // a stopped system keeps a pending grid adoption: its bboxes are adopted when it
     // resumes or when a caller reads the grid
