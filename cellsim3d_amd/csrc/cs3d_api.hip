@@ -1648,7 +1648,7 @@ extern "C" cs3d_status cs3d_time_kernel(cs3d_ctx* c, cs3d_sys s, int32_t which, 
     auto launch = [&]() {
         if (which == 0) launch_bonded(c->pool, r, c->sys[s].prm.constrain_angles ? 1 : 0, c->stream);
         else if (which == 1) launch_dis(c->pool, r, M_COM, 0, 0, false, c->stream);
-        else launch_search(c->pool, r, 1, c->stream);
+        else launch_search(c->pool, r, kSearchAgain, c->stream);
     };
     // the timed search replaces the candidates that the accept bits belong to
     if (which == 2) make_pairs(c, s);

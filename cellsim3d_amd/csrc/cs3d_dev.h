@@ -9,7 +9,8 @@
 //                int32[cap_cells * 6]    voxel range of the contact-rule bbox (kept with it)
 //   pair lists   int32[cap_cells * kPMax * 192]  contact partners of each node, (cell, node)
 //                ascending, k-major per cell, and int32[cap_cells * 192] their count: made
-//                from the candidates and their accept bits when a caller reads them
+//                from the candidates and their accept bits when a caller reads them (until the
+//                contact pass after a search is done, the room holds what that search replaced)
 //                int32[cap_cells * kPMax * 192]  contact candidates (within attraction_range + skin
 //                at the last search): per cell one flat list, node after node, + per node the
 //                count (low kCandBits bits) and the index of its first entry (above them); behind the
@@ -43,7 +44,13 @@ static_assert(kPMax < (1 << kCandBits), "a node's candidate count fits its bits"
 // tests of the latest contact pass (entry j is bit j % 64 of word j / 64).
 constexpr int kMaskAt = kPMax * kNodes;
 constexpr int kMaskWords = (kMaskAt + kSlots - 1) / kSlots * (kSlots / 64);
-static_assert(kMaskAt % 2 == 0 && kMaskAt + 2 * kMaskWords <= kPMax * kSlots, "the mask fits behind the list");
+// Behind the bits, one word.  0: list and bits belong together.  1: the list has been
+// searched anew; the one that the latest contact pass used is held, with its bits at the
+// same places, in the cell's room of PAIRS, its counts in NPAIR.  2: the partner lists
+// have been made of that.
+constexpr int kHeldAt = kMaskAt + 2 * kMaskWords;
+static_assert(kMaskAt % 2 == 0 && kHeldAt < kPMax * kSlots, "the mask and the word fit behind the list");
+constexpr int kSearchAgain = 2;  // k_search: a search for its own sake, whose list no contact pass uses
 constexpr int kBCap = CS3D_BIN_CAP;  // nodes per search bin
 constexpr int kMaxSys = 4096;        // systems per context
 constexpr int kMaxPartial = 192;     // listed cells beyond which the next search is a full one (at most the

@@ -1099,6 +1099,26 @@ __device__ __forceinline__ void pair_pass(const int32_t* cand, uint64_t* mask, P
     }
 }
 
+// A search replaces the candidates that the accept bits of the latest contact pass belong
+// to.  Until the next pass is done the old list, counts and bits stay in the cell's room
+// of the partner lists (kHeldAt 1; on a step k_dis_post ends it), so that a step that ends
+// at its search leaves the partners that a caller reads as they were.  key0, ncf, total:
+// the list's entry of this lane, the lane's NCAND word and the list's length.  Every lane
+// of the workgroup calls it; the candidates may be written after the next barrier.
+__device__ __forceinline__ void hold_partners(CPool p, int slot, int tid, int key0, int ncf, int total) {
+    int32_t* cand = p->CAND + (size_t)slot * (kPMax * kSlots);
+    int32_t* held = p->PAIRS + (size_t)slot * (kPMax * kSlots);
+    if (tid < kMaskWords) pair_mask(p->PAIRS, slot)[tid] = pair_mask(p->CAND, slot)[tid];
+    held[tid] = key0;
+#pragma unroll 1
+    for (int e = kSlots + tid; e < total; e += kSlots) held[e] = cand[e];
+    p->NPAIR[(size_t)slot * kSlots + tid] = ncf;
+    if (tid == 0) cand[kHeldAt] = 1;
+}
+__device__ __forceinline__ void release_partners(CPool p, int slot) {
+    p->CAND[(size_t)slot * (kPMax * kSlots) + kHeldAt] = 0;
+}
+
 // ------------------------------------------------------------------------------
 // Contact-candidate search (one cell per workgroup): on systems whose nodes
 // moved pair_skin/2 since the last search (or always, outside the fused step),
@@ -1114,10 +1134,12 @@ struct SearchLds {
 // The search of one cell (every lane of the workgroup calls it) at its positions X,
 // Y, Z (word: where an overflow is noted).  Returns whether the cell searched; then first, nc are this lane's entries
 // of the new list and total their number.  u is written only after a barrier that
-// ends its previous use, and is free when it returns.
+// ends its previous use, and is free when it returns.  hold: hold_partners with key0,
+// ncf and oldn is still to be done (where the cell searches).
 template <class MP, class PP>
 __device__ __forceinline__ bool search_cell(CPool p, uint32_t* word, MP MC, PP P, int slot, int c, int tid, bool always,
-                                            float X, float Y, float Z, SearchLds& u, int& first, int& nc, int& total) {
+                                            float X, float Y, float Z, bool hold, int key0, int ncf, int oldn,
+                                            SearchLds& u, int& first, int& nc, int& total) {
     const bool node = tid < kNodes;
     const size_t cb = (size_t)slot * kSlots;  // the cell's first node (uniform)
     const uint32_t ln = lane_index();
@@ -1159,6 +1181,7 @@ __device__ __forceinline__ bool search_cell(CPool p, uint32_t* word, MP MC, PP P
         // is kept for later partial searches
         box_of_cell(X, Y, Z, node, u.part, p->SBOX + (int64_t)slot * 6);
     }
+    if (hold) hold_partners(p, slot, tid, key0, ncf, oldn);
     uint32_t st = 0;
     nc = node ? find_candidates(p, MC, P, c, X, Y, Z, u.lst, tid, st) : 0;
     // the cell's candidates one after another in node order: an exclusive scan of
@@ -1211,10 +1234,13 @@ __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always)
         const size_t cb = (size_t)slot * kSlots;
         const uint32_t ln = lane_index();
         const float X = ldu(p.X + cb, ln), Y = ldu(p.Y + cb, ln), Z = ldu(p.Z + cb, ln);
+        const bool hold = always != kSearchAgain;
+        const int key0 = ldu(p.CAND + cb * kPMax, ln), ncf = ldu(p.NCAND + cb, ln);
+        const int oldn = cld(p.NCAND + cb + kNodes) >> kCandBits;
         int first, nc, total;
         uint32_t* word = always ? status_word<false, R_SEARCH>(M) : status_word<true, R_SEARCH>(M);
-        search_cell(pool_late(), word, MC, cparams(p.prm + s), slot, c, threadIdx.x, always, X, Y, Z, u, first, nc,
-                    total);
+        search_cell(pool_late(), word, MC, cparams(p.prm + s), slot, c, threadIdx.x, always, X, Y, Z, hold, key0, ncf, oldn,
+                    u, first, nc, total);
     }
 }
 
@@ -1223,19 +1249,38 @@ __global__ __launch_bounds__(192) void k_search(Pool p, Range r, int32_t always)
 // system cannot know of each other's overflow, so on a step that searches each keeps
 // what the contact pass writes over (keep_cell), and the division phase puts it back
 // (take_back_cell) in a system that overflowed.
-template <class F> __device__ __forceinline__ void kept_arrays(CPool p, bool rands, F&& f) {
-    float* const a[9] = {p->VX, p->VY, p->VZ, p->FCX, p->FCY, p->FCZ, p->FRX, p->FRY, p->FRZ};
-    for (int k = 0; k < (rands ? 9 : 6); ++k) f(a[k], (uint32_t)(k * kSlots));
-}
-__device__ __forceinline__ void keep_cell(CPool p, bool rands, int slot, uint32_t ln) {
+struct Kept {
+    float v[9];
+};
+__device__ __forceinline__ Kept load_kept(CPool p, bool rands, int slot, uint32_t ln) {
     const size_t cb = (size_t)slot * kSlots;
-    kept_arrays(p, rands, [&](float* a, uint32_t at) { stu(p->KEEP + 9 * cb, at + ln, ldu(a + cb, ln)); });
+    Kept k;
+    k.v[0] = ldu(p->VX + cb, ln); k.v[1] = ldu(p->VY + cb, ln); k.v[2] = ldu(p->VZ + cb, ln);
+    k.v[3] = ldu(p->FCX + cb, ln); k.v[4] = ldu(p->FCY + cb, ln); k.v[5] = ldu(p->FCZ + cb, ln);
+    k.v[6] = k.v[7] = k.v[8] = 0.f;
+    if (rands) { k.v[6] = ldu(p->FRX + cb, ln); k.v[7] = ldu(p->FRY + cb, ln); k.v[8] = ldu(p->FRZ + cb, ln); }
+    return k;
+}
+__device__ __forceinline__ void keep_cell(CPool p, const Kept& k, int slot, uint32_t ln) {
+    float* q = p->KEEP + (size_t)slot * (9 * kSlots);
+#pragma unroll
+    for (int a = 0; a < 9; ++a) stu(q, a * kSlots + ln, k.v[a]);
 }
 __device__ __forceinline__ void take_back_cell(CPool p, bool rands, int slot, uint32_t ln) {
     const size_t cb = (size_t)slot * kSlots;
-    kept_arrays(p, rands, [&](float* a, uint32_t at) { stu(a + cb, ln, ldu(p->KEEP + 9 * cb, at + ln)); });
+    const float* q = p->KEEP + 9 * cb;
+    float* const to[9] = {p->VX, p->VY, p->VZ, p->FCX, p->FCY, p->FCZ, p->FRX, p->FRY, p->FRZ};
+    for (int a = 0; a < (rands ? 9 : 6); ++a) stu(to[a] + cb, ln, ldu(q, a * kSlots + ln));
 }
 
+// Both before a search at the head of k_con_dis; a call, since inlined it takes registers
+// from the step's common path (8 cells 23.0 against 23.15 us a step, 403 28.2 against 28.5).
+__attribute__((noinline)) __device__ void hold_and_keep(CPool p, bool rands, int slot, uint32_t ln, int key0, int ncf,
+                                                        int total) {
+    const Kept kept = load_kept(p, rands, slot, ln);
+    hold_partners(p, slot, (int)ln, key0, ncf, total);
+    keep_cell(p, kept, slot, ln);
+}
 // ------------------------------------------------------------------------------
 // Conservative force (CalculateConForce, propagate.cu:183-520) fused with the
 // first dissipative force (CalculateDisForce with the post-Integrate
@@ -1338,9 +1383,10 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(kSearch ? 4
         // (but for status bits, by atomics), through scalar loads
         const CMeta MC = cmeta(M);
         const int32_t need = kSearch ? MC->need_search : 0;
-        if (kSearch) asm volatile("" ::"s"(need));  // (with the same round trip)
         int c;
-        if (!cell_live<kStep ? R_CON : 0>(MC, slot, c)) {
+        const bool live = cell_live<kStep ? R_CON : 0>(MC, slot, c);
+        if (kSearch) asm volatile("" ::"s"(need), "s"(c), "s"((int)live));  // (with the same round trip)
+        if (!live) {
             if (!kLive) nit = 0;  // one system: neither is any cell after it
             continue;
         }
@@ -1352,8 +1398,10 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(kSearch ? 4
             // with the new list, so that none of its registers live through the search
             if (__builtin_expect(need && done != it, 0)) {
                 int f, n, t;
-                keep_cell(pool_late(), P->add_rands != 0, slot, ln);
-                search_cell(pool_late(), word, MC, P, slot, c, lt, false, X, Y, Z, mem.s, f, n, t);
+                hold_and_keep(pool_late(), P->add_rands != 0, slot, ln, key0, ncf,
+                              __builtin_amdgcn_readfirstlane(total) >> kCandBits);
+                __syncthreads();
+                search_cell(pool_late(), word, MC, P, slot, c, lt, false, X, Y, Z, false, 0, 0, 0, mem.s, f, n, t);
                 done = it;
                 it -= gridDim.x;
                 continue;
@@ -1365,6 +1413,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(kSearch ? 4
             p.RESET[slot] = 0;
             if (c == 0) M->n_reset = 0;
         }
+        if (!kStep && tid == 0) release_partners(pool_late(), slot);
         __syncthreads();
         uint32_t st = 0;
         const bool angles = forces && P->constrain_angles;
@@ -1949,6 +1998,7 @@ __global__ __launch_bounds__(192) void k_dis_post(Pool p, Range r, int32_t mode,
             const int64_t lo = (int64_t)c * per, hi = min(nb, lo + per);
             int32_t* counts = pool_late()->bins + MC->bbase;
             for (int64_t b = lo + tid; b < hi; b += blockDim.x) counts[b] = 0;
+            if (kStep && tid == 0) release_partners(pool_late(), slot);
         }
         const int64_t stepno = step_override >= 0 ? step_override : MC->step + 1;
         const bool do_vol = mode == M_VOLUMES || (kStep && stepno <= P->div_time_steps && rgrowth(P, MC->n) > 0.0f);
@@ -2161,10 +2211,13 @@ __device__ void divide_system(const Pool& p, int s, int32_t mode) {
 #pragma unroll
     for (int k = 0; k < R_PHASES; ++k) found |= raised[k];
     if (__builtin_expect(found != 0, 0)) {
-        if (raised[R_CON] & CS3D_SYS_CAND_OVERFLOW) {
+        const bool over = raised[R_CON] & CS3D_SYS_CAND_OVERFLOW;
+        if (over) {
             found = CS3D_SYS_CAND_OVERFLOW;
             for (int c = 0; c < n0; ++c)
                 if (tid < kSlots) take_back_cell(pool_late(), PC->add_rands != 0, base + c, (uint32_t)tid);
+        } else if (raised[R_CON]) {  // the contact pass is done, but no k_dis_post followed
+            for (int c = tid; c < n0; c += blockDim.x) release_partners(pool_late(), base + c);
         }
         m_status |= found;
         __syncthreads();  // every wave has read them
@@ -2787,22 +2840,38 @@ __global__ __launch_bounds__(192) void k_grid_adopt(Pool p, Range r) {
 }
 
 // The partner lists that callers read (CS3D_F_PAIRS, CS3D_F_PAIRCOUNT): each live
-// node's accepted candidates, ascending, k-major per cell.
+// node's accepted candidates, ascending, k-major per cell, from the candidates and their
+// accept bits, or from what a search holds of them (hold_partners) in the lists' own room.
 __global__ __launch_bounds__(192) void k_pairs_list(Pool p, Range r) {
+    __shared__ int32_t list[kMaskAt];
+    __shared__ uint64_t bits[kMaskWords];
     const int tid = threadIdx.x;
     for (int slot = r.slot_lo + blockIdx.x; slot < r.slot_hi; slot += gridDim.x) {
         const int s = sys_of(p, r, slot);
-        if (s < 0 || tid >= kNodes) continue;
+        if (s < 0) continue;
         const SysMeta* M = p.meta + s;
         if (slot - M->base >= M->n) continue;
-        const int ncf = p.NCAND[(int64_t)slot * kSlots + tid];
-        const int nc = ncf & ((1 << kCandBits) - 1), first = ncf >> kCandBits;
-        const int32_t* cand = p.CAND + (int64_t)slot * kPMax * kSlots;
-        const uint64_t* mask = pair_mask(p.CAND, slot);
-        int np = 0;
-        for (int j = first; j < first + nc; ++j)
-            if (mask[j >> 6] >> (j & 63) & 1) p.PAIRS[((int64_t)slot * kPMax + np++) * kSlots + tid] = cand[j];
-        p.NPAIR[(int64_t)slot * kSlots + tid] = np;
+        const size_t cb = (size_t)slot * kSlots;
+        int32_t* cand = p.CAND + cb * kPMax;
+        const int held = cand[kHeldAt];
+        __syncthreads();  // every lane has read it (and the cell before is done)
+        if (held == 2) continue;  // the lists were made of it
+        const int32_t* counts = held ? p.NPAIR : p.NCAND;
+        const int32_t* from = held ? p.PAIRS + cb * kPMax : cand;
+        const int ncf = counts[cb + tid], total = counts[cb + kNodes] >> kCandBits;
+        for (int e = tid; e < total; e += kSlots) list[e] = from[e];
+        if (tid < kMaskWords) bits[tid] = pair_mask(held ? p.PAIRS : p.CAND, slot)[tid];
+        __syncthreads();
+        if (tid < kNodes) {
+            const int nc = ncf & ((1 << kCandBits) - 1), first = ncf >> kCandBits;
+            int np = 0;
+            for (int j = first; j < first + nc; ++j)
+                if (bits[j >> 6] >> (j & 63) & 1) p.PAIRS[cb * kPMax + np++ * kSlots + tid] = list[j];
+            p.NPAIR[cb + tid] = np;
+        } else {
+            p.NPAIR[cb + tid] = 0;
+        }
+        if (tid == 0 && held) cand[kHeldAt] = 2;
     }
 }
 
