@@ -23,7 +23,7 @@
 namespace cs3d {
 void launch_integrate(const Pool& p, const Range& r, int flags, int64_t step_override, hipStream_t st);
 void launch_search(const Pool& p, const Range& r, int always, hipStream_t st);
-int cells_covered(const Range& r);
+int32_t cells_covered(const Pool& p, const Range& r);
 void launch_con(const Pool& p, const Range& r, int mode, hipStream_t st);
 void launch_dis(const Pool& p, const Range& r, int mode, int64_t step_override, int clear_bins, bool use_va,
                 hipStream_t st);
@@ -116,11 +116,11 @@ struct cs3d_ctx {
     int graph_steps = 10;
     struct GraphRec {
         hipGraphExec_t exec;
-        int steps;
         bool shift;  // the captured steps include CorrectCoMMotion
-        int32_t grid;  // live cells that its grids cover without striding
+        int32_t covers;  // live cells up to which no wider grid would be launched
     };
-    std::map<int, GraphRec> graphs;  // target -> captured steps
+    // target -> captured steps, one record for each width of the grids, ascending
+    std::map<int, std::vector<GraphRec>> graphs;
     cs3d_mesh mesh_host;  // the tables the context was created with (checkpoint check)
     // pinned staging ring of the reads (read_back), allocated at the first one
     char* stage = nullptr;
@@ -150,7 +150,7 @@ template <class T> cs3d_status dalloc(cs3d_ctx* c, T*& p, int64_t count) {
 void drop_graphs(cs3d_ctx* c, int target_only = -2) {
     for (auto it = c->graphs.begin(); it != c->graphs.end();) {
         if (target_only == -2 || it->first == target_only) {
-            (void)hipGraphExecDestroy(it->second.exec);
+            for (const cs3d_ctx::GraphRec& g : it->second) (void)hipGraphExecDestroy(g.exec);
             it = c->graphs.erase(it);
         } else {
             ++it;
@@ -747,7 +747,7 @@ cs3d_status room_add(cs3d_ctx* c, const cs3d_params* prm, int32_t n_cells, int32
     HIPCHK(hipGetLastError());
     // a captured all-systems step without CorrectCoMMotion cannot serve this system
     auto g = c->graphs.find(CS3D_ALL);
-    if (prm->correct_com && g != c->graphs.end() && !g->second.shift) drop_graphs(c, CS3D_ALL);
+    if (prm->correct_com && g != c->graphs.end() && !g->second.front().shift) drop_graphs(c, CS3D_ALL);
     *out = sid;
     return CS3D_OK;
 }
@@ -1370,36 +1370,35 @@ extern "C" cs3d_status cs3d_step_timed(cs3d_ctx* c, cs3d_sys s, int32_t n_steps,
 }
 
 namespace {
-// The captured graph_steps steps of a target, captured, instantiated and
-// uploaded on first use.
-cs3d_status graph_of(cs3d_ctx* c, cs3d_sys s, const cs3d_ctx::GraphRec** out) {
-    const Range r = range_of(c, s);
+// The captured graph_steps steps of a target, with grids for the range's live cells:
+// captured, instantiated and uploaded on first use.  A tissue that outgrows its grids,
+// which would stride, is captured again with wider ones (once for every quarter that it
+// grows) beside the graphs that may still run: nothing waits for the stream.
+cs3d_status graph_of(cs3d_ctx* c, cs3d_sys s, const Range& r, cs3d_ctx::GraphRec* out) {
     auto it = c->graphs.find(s);
-    // a tissue that has outgrown the grids of its capture (they would stride) is captured
-    // again: once for every quarter that it grows
-    if (it != c->graphs.end() && r.live_hint > it->second.grid) {
-        HIPCHK(hipStreamSynchronize(c->stream));
-        drop_graphs(c, s);
-        it = c->graphs.end();
+    if (it != c->graphs.end())
+        for (const cs3d_ctx::GraphRec& g : it->second)
+            if (r.live_hint <= g.covers) {
+                *out = g;
+                return CS3D_OK;
+            }
+    const int vb = vox_blocks_of(c, s);
+    hipGraph_t g = nullptr;
+    HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+    for (int k = 0; k < c->graph_steps; ++k) enqueue_step(c, r, vb);
+    HIPCHK(hipStreamEndCapture(c->stream, &g));
+    hipGraphExec_t ex = nullptr;
+    hipError_t e = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(g);
+    if (e != hipSuccess) return fail(CS3D_HIP_ERROR, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
+    e = hipGraphUpload(ex, c->stream);
+    if (e != hipSuccess) {
+        (void)hipGraphExecDestroy(ex);
+        return fail(CS3D_HIP_ERROR, std::string("hipGraphUpload: ") + hipGetErrorString(e));
     }
-    if (it == c->graphs.end()) {
-        const int vb = vox_blocks_of(c, s);
-        hipGraph_t g = nullptr;
-        HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        for (int k = 0; k < c->graph_steps; ++k) enqueue_step(c, r, vb);
-        HIPCHK(hipStreamEndCapture(c->stream, &g));
-        hipGraphExec_t ex = nullptr;
-        hipError_t e = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        if (e != hipSuccess) return fail(CS3D_HIP_ERROR, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
-        e = hipGraphUpload(ex, c->stream);
-        if (e != hipSuccess) {
-            (void)hipGraphExecDestroy(ex);
-            return fail(CS3D_HIP_ERROR, std::string("hipGraphUpload: ") + hipGetErrorString(e));
-        }
-        it = c->graphs.emplace(s, cs3d_ctx::GraphRec{ex, c->graph_steps, any_correct_com(c, r), cells_covered(r)}).first;
-    }
-    *out = &it->second;
+    // (a new record covers more than those before it)
+    *out = cs3d_ctx::GraphRec{ex, any_correct_com(c, r), cells_covered(c->pool, r)};
+    c->graphs[s].push_back(*out);
     return CS3D_OK;
 }
 }  // namespace
@@ -1408,9 +1407,14 @@ extern "C" cs3d_status cs3d_graph_prepare(cs3d_ctx* c, cs3d_sys s) {
     if (!c) return fail(CS3D_INVALID_ARG, "NULL context");
     if (s != CS3D_ALL && !valid_sys(c, s)) return fail(CS3D_INVALID_ARG, "unknown system");
     if (!c->use_graph) return CS3D_OK;
-    const cs3d_ctx::GraphRec* g = nullptr;
-    cs3d_status st = graph_of(c, s, &g);
-    if (st != CS3D_OK) return st;
+    // for the cells that are live and for every width that the room can come to need
+    Range r = range_of(c, s);
+    cs3d_ctx::GraphRec g;
+    do {
+        const cs3d_status st = graph_of(c, s, r, &g);
+        if (st != CS3D_OK) return st;
+        if (g.covers < std::numeric_limits<int32_t>::max()) r.live_hint = g.covers + 1;
+    } while (g.covers < std::numeric_limits<int32_t>::max());
     HIPCHK(hipStreamSynchronize(c->stream));
     return CS3D_OK;
 }
@@ -1425,14 +1429,12 @@ extern "C" cs3d_status cs3d_step(cs3d_ctx* c, cs3d_sys s, int32_t n_steps) {
     pairs_stale(c, s);
     int done = 0;
     if (c->use_graph && n_steps >= c->graph_steps) {
-        const cs3d_ctx::GraphRec* g = nullptr;
-        do {
-            cs3d_status st = graph_of(c, s, &g);
+        cs3d_ctx::GraphRec g;
+        for (; done + c->graph_steps <= n_steps; done += c->graph_steps) {
+            cs3d_status st = graph_of(c, s, range_of(c, s), &g);
             if (st != CS3D_OK) return st;
-            if (done + g->steps > n_steps) break;
-            HIPCHK(hipGraphLaunch(g->exec, c->stream));
-            done += g->steps;
-        } while (done + g->steps <= n_steps);
+            HIPCHK(hipGraphLaunch(g.exec, c->stream));
+        }
     }
     for (; done < n_steps; ++done) enqueue_step(c, r, vb);
     HIPCHK(hipGetLastError());

@@ -28,6 +28,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <limits>
 #include <type_traits>
 #include <utility>
 #include <vector>
@@ -3109,14 +3110,21 @@ static void launch(F kernel, dim3 grid, dim3 block, hipStream_t st, A... args) {
 // 197 us (k_dis_post 94, 109, 103, 118).  A workgroup without a cell still costs its
 // dispatch, 2 to 3 ns, so rooms far larger than their tissue are not launched whole.
 constexpr int kMinGrid = 256;  // one workgroup per CU: a small tissue's growth needs no wider grid
-int cells_covered(const Range& r) {
+static int grid_cover(const Range& r) {
     const int64_t slots = r.slot_hi - r.slot_lo, n = (int64_t)r.live_hint + r.live_hint / 4 + 8;
     return (int)std::min(slots, std::max<int64_t>(n, kMinGrid));
 }
 static int grid_step(const Range& r, int per_cu) {
-    const int n = cells_covered(r);
+    const int n = grid_cover(r);
     const int64_t cap = per_cu > 0 ? 256 * (int64_t)per_cu : n;
     return (int)(n < 1 ? 1 : (n < cap ? n : cap));
+}
+// Live cells up to which a step launches no wider grid than now: without bound where
+// the room or the caller's cap already ends it.
+int32_t cells_covered(const Pool& p, const Range& r) {
+    const int n = grid_cover(r);
+    const bool widest = n >= r.slot_hi - r.slot_lo || (p.wg_per_cu > 0 && n >= 256 * (int64_t)p.wg_per_cu);
+    return widest ? std::numeric_limits<int32_t>::max() : n;
 }
 // Grid of the other cell kernels: one workgroup per slot up to 4096, then they stride.
 static int grid_cells(const Range& r, int per_cu) {
