@@ -406,7 +406,7 @@ void enqueue_step_phase(cs3d_ctx* c, const Range& r, int phase) {
     }
 }
 
-void enqueue_step(cs3d_ctx* c, const Range& r, int /*vb*/) {
+void enqueue_step(cs3d_ctx* c, const Range& r) {
     for (int q = 0; q < CS3D_PHASES; ++q) enqueue_step_phase(c, r, q);
 }
 
@@ -1364,8 +1364,10 @@ extern "C" cs3d_status cs3d_step_timed(cs3d_ctx* c, cs3d_sys s, int32_t n_steps,
     if (r.slot_hi <= r.slot_lo || r.sys_hi <= r.sys_lo) return CS3D_OK;
     pairs_stale(c, s);
     cs3d_status st = CS3D_OK;
-    for (int k = 0; k < n_steps && st == CS3D_OK; ++k)
-        st = timed_groups(c, CS3D_PHASES, [&](int q) { enqueue_step_phase(c, r, q); }, phase_ms);
+    for (int k = 0; k < n_steps && st == CS3D_OK; ++k) {
+        const Range now = range_of(c, s);  // (grids follow the live cells)
+        st = timed_groups(c, CS3D_PHASES, [&](int q) { enqueue_step_phase(c, now, q); }, phase_ms);
+    }
     return st;
 }
 
@@ -1382,10 +1384,9 @@ cs3d_status graph_of(cs3d_ctx* c, cs3d_sys s, const Range& r, cs3d_ctx::GraphRec
                 *out = g;
                 return CS3D_OK;
             }
-    const int vb = vox_blocks_of(c, s);
     hipGraph_t g = nullptr;
     HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    for (int k = 0; k < c->graph_steps; ++k) enqueue_step(c, r, vb);
+    for (int k = 0; k < c->graph_steps; ++k) enqueue_step(c, r);
     HIPCHK(hipStreamEndCapture(c->stream, &g));
     hipGraphExec_t ex = nullptr;
     hipError_t e = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
@@ -1424,8 +1425,6 @@ extern "C" cs3d_status cs3d_step(cs3d_ctx* c, cs3d_sys s, int32_t n_steps) {
     if (s != CS3D_ALL && !valid_sys(c, s)) return fail(CS3D_INVALID_ARG, "unknown system");
     if (n_steps <= 0) return CS3D_OK;
     if (s == CS3D_ALL && c->nsys_high == 0) return CS3D_OK;
-    const Range r = range_of(c, s);
-    const int vb = vox_blocks_of(c, s);
     pairs_stale(c, s);
     int done = 0;
     if (c->use_graph && n_steps >= c->graph_steps) {
@@ -1436,7 +1435,7 @@ extern "C" cs3d_status cs3d_step(cs3d_ctx* c, cs3d_sys s, int32_t n_steps) {
             HIPCHK(hipGraphLaunch(g.exec, c->stream));
         }
     }
-    for (; done < n_steps; ++done) enqueue_step(c, r, vb);
+    for (; done < n_steps; ++done) enqueue_step(c, range_of(c, s));  // (grids follow the live cells)
     HIPCHK(hipGetLastError());
     return CS3D_OK;
 }

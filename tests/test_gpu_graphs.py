@@ -82,3 +82,38 @@ def test_growth_past_the_captured_grids(oracle_mesh, n, cap, both, prepared):
     for a, b in zip(*got):
         for f, u, v in zip(fields, a, b):
             assert np.array_equal(u, v), f
+
+
+def test_eager_steps_widen_their_grids(oracle_mesh):
+    """One long call without graphs: its first step doubles the tissue, past the grids of
+    its start, and the later ones take grids for what they find.  2000 steps take less than
+    1.25 times those of a host that has looked (1.5 times on the grids of the start, 1.1
+    with the first of them enqueued before the division is seen), and give the same state."""
+    from cellsim3d_amd import abi as A
+    from cellsim3d_amd import configs, engine
+    print("eager grids", flush=True)
+    n, steps = 204, 2000
+    p, X, Y, Z = _dividing(A, configs, n, 1)
+    p.grid_interval = 10
+    took, state = {True: [], False: []}, []
+    with engine.Context(oracle_mesh, capacity_cells=8 * n, voxel_budget=1 << 22, bin_budget=1 << 28) as ctx:
+        ctx.set_graph(False)
+        for rep in range(3):
+            for looked in (True, False):
+                s = ctx.add_system(p, X, Y, Z, n, max_cells=8 * n, voxels=1 << 14)
+                if looked:
+                    s.step(1)
+                ctx.sync()
+                s.info()
+                t = time.perf_counter()
+                s.step(steps - looked)
+                ctx.sync()
+                took[looked].append((time.perf_counter() - t) / (steps - looked))
+                assert s.info() == (2 * n, steps, 0)
+                if rep == 0:
+                    state.append([s.get(f) for f in (A.F_X, A.F_VY, A.F_FDZ)])
+                s.remove()
+    print({k: [round(1e6 * x, 1) for x in v] for k, v in took.items()}, flush=True)
+    for a, b in zip(*state):
+        assert np.array_equal(a, b)
+    assert min(took[False]) < 1.25 * min(took[True])
