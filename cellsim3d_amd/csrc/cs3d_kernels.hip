@@ -2171,8 +2171,9 @@ __device__ __forceinline__ void block_minmax12(float* v, float (*part)[12], floa
 }
 
 // Division phase of system s by one 256-lane workgroup (every lane calls it; the
-// early returns depend on the system only, so the workgroup stays together).
-__device__ void divide_system(const Pool& p, int s, int32_t mode) {
+// early returns depend on the system only, so the workgroup stays together).  Part of its
+// kernel: pool_late reads the kernel's own arguments, which a called function has not.
+__device__ __forceinline__ void divide_system(const Pool& p, int s, int32_t mode) {
     __shared__ int32_t wsum[4];
     __shared__ int32_t nev, ncur, stop;
     __shared__ float nrm[3];
