@@ -122,9 +122,10 @@ struct cs3d_ctx {
     // target -> captured steps, one record for each width of the grids, ascending
     std::map<int, std::vector<GraphRec>> graphs;
     cs3d_mesh mesh_host;  // the tables the context was created with (checkpoint check)
-    // pinned staging ring of the reads (read_back), allocated at the first one
-    char* stage = nullptr;
+    // pinned memory of the reads (read_back): a small piece behind the live counts
+    // (Pool::seen), and a ring made at the first large read
     char* stage_small = nullptr;
+    char* stage = nullptr;
     hipEvent_t stage_ev[4] = {nullptr, nullptr, nullptr, nullptr};
     void* scratch = nullptr;  // small device buffer of the per-kernel entry points (grown on demand)
     size_t scratch_bytes = 0;
@@ -229,20 +230,17 @@ struct ReadPiece {
     size_t off, bytes;  // offset in the slot
 };
 
-// Pinned memory of the context for reads, made when first needed: a small piece, and
-// the ring for reads that do not fit that.
-bool stage_ready(cs3d_ctx* c, bool small) {
-    char*& at = small ? c->stage_small : c->stage;
-    if (at) return true;
+// The ring of the context's large reads, made when first needed.
+bool ring_ready(cs3d_ctx* c) {
+    if (c->stage) return true;
     int before = c->device;
     (void)hipGetDevice(&before);
     void* q = nullptr;
     // coherent: what a finished kernel wrote is what the host reads
     bool ok = hipSetDevice(c->device) == hipSuccess &&
-              hipHostMalloc(&q, small ? kSmallBytes : kSlotBytes * kSlotsInRing,
-                            hipHostMallocPortable | hipHostMallocCoherent) == hipSuccess;
+              hipHostMalloc(&q, kSlotBytes * kSlotsInRing, hipHostMallocPortable | hipHostMallocCoherent) == hipSuccess;
     for (hipEvent_t& e : c->stage_ev) ok = ok && (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess);
-    if (ok) at = static_cast<char*>(q);
+    if (ok) c->stage = static_cast<char*>(q);
     else if (q) (void)hipHostFree(q);
     if (!ok) (void)hipGetLastError();
     (void)hipSetDevice(before);
@@ -267,7 +265,7 @@ cs3d_status read_back(cs3d_ctx* c, const ReadSeg* segs, int n_segs) {
     size_t room = 0;  // in a slot, with the alignment of the pieces
     for (int i = 0; i < n_segs; ++i) room += (segs[i].bytes + 15) / 16 * 16;
     const bool small = room <= kSmallBytes && n_segs <= kMaxGather;
-    if (!words || plain || !stage_ready(c, small)) {
+    if (!words || plain || !(small || ring_ready(c))) {
         for (int i = 0; i < n_segs; ++i)
             if (segs[i].bytes)
                 HIPCHK(hipMemcpyAsync(segs[i].host, segs[i].dev, segs[i].bytes, hipMemcpyDeviceToHost, c->stream));
@@ -337,9 +335,9 @@ cs3d_status read_back(cs3d_ctx* c, const ReadSeg* segs, int n_segs) {
                 while (done[issued - kSlotsInRing].load(std::memory_order_acquire) < want) std::this_thread::yield();
             launch_gather(lists[issued], slot(issued), c->stream);
             e = hipGetLastError();
-            if (e == hipSuccess) e = hipEventRecord(c->stage_ev[issued % kSlotsInRing], c->stream);
+            if (e == hipSuccess && !small) e = hipEventRecord(c->stage_ev[issued % kSlotsInRing], c->stream);
         }
-        if (e == hipSuccess) e = hipEventSynchronize(c->stage_ev[k % kSlotsInRing]);
+        if (e == hipSuccess) e = small ? hipStreamSynchronize(c->stream) : hipEventSynchronize(c->stage_ev[k % kSlotsInRing]);
         if (e != hipSuccess) break;
         if (k == 0 && total >= kSerialRead) start_readers();
         if (want) ready.store(k + 1, std::memory_order_release);
@@ -626,10 +624,12 @@ extern "C" cs3d_status cs3d_ctx_create(int device, const cs3d_mesh* mesh, int64_
     if ((st = dalloc(c, p.nsys, 1)) != CS3D_OK) return cleanup(st);
     if ((st = dalloc(c, p.meta, kMaxSys)) != CS3D_OK) return cleanup(st);
     void* live = nullptr;  // coherent: the host reads it while kernels run
-    if (hipHostMalloc(&live, kMaxSys * sizeof(int32_t), hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess)
+    if (hipHostMalloc(&live, kMaxSys * sizeof(int32_t) + kSmallBytes, hipHostMallocPortable | hipHostMallocCoherent) !=
+        hipSuccess)
         return cleanup(fail(CS3D_OUT_OF_MEMORY, "live counts"));
     std::memset(live, 0, kMaxSys * sizeof(int32_t));
     p.seen = static_cast<int32_t*>(live);
+    c->stage_small = static_cast<char*>(live) + kMaxSys * sizeof(int32_t);
     cs3d_params* prm = nullptr;
     if ((st = dalloc(c, prm, kMaxSys)) != CS3D_OK) return cleanup(st);
     p.prm = prm;
@@ -654,7 +654,6 @@ extern "C" cs3d_status cs3d_ctx_destroy(cs3d_ctx* c) {
         if (e) (void)hipEventDestroy(e);
     if (c->pool.seen) (void)hipHostFree(c->pool.seen);
     if (c->stage) (void)hipHostFree(c->stage);
-    if (c->stage_small) (void)hipHostFree(c->stage_small);
     for (void* q : c->allocs) (void)hipFree(q);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
