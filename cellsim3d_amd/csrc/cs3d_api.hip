@@ -9,7 +9,9 @@
 #include <cstring>
 #include <limits>
 #include <map>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <string>
 #include <system_error>
 #include <thread>
@@ -213,22 +215,12 @@ int vox_blocks_of(cs3d_ctx* c, cs3d_sys s) {
 // kernel fills the next (15.4 MB: 1.12 ms before, 0.38 ms).  One piece between 16 KB
 // and kSerialRead stays a plain copy (16,388 B: 9.9 us against 13.7; 16,384 B: 21.5
 // against 13.5).
-struct ReadSeg {
-    const void* dev;
-    void* host;
-    size_t bytes;
-};
 constexpr size_t kSlotBytes = 2u << 20;  // a ring slot: 40 us of the link, long against a launch
 constexpr int kSlotsInRing = 4;
 constexpr size_t kSerialRead = 1u << 20;  // below, starting threads (45 us) costs more than it gives
 constexpr size_t kPlainFrom = 16u << 10;
 constexpr size_t kSmallBytes = 64u << 10;  // reads that fit this need not allocate the ring
 constexpr int kReaders = 4;
-
-struct ReadPiece {
-    char* host;
-    size_t off, bytes;  // offset in the slot
-};
 
 // The ring of the context's large reads, made when first needed.
 bool ring_ready(cs3d_ctx* c) {
@@ -265,37 +257,15 @@ cs3d_status read_back(cs3d_ctx* c, const ReadSeg* segs, int n_segs) {
     size_t room = 0;  // in a slot, with the alignment of the pieces
     for (int i = 0; i < n_segs; ++i) room += (segs[i].bytes + 15) / 16 * 16;
     const bool small = room <= kSmallBytes && n_segs <= kMaxGather;
-    if (!words || plain || !(small || ring_ready(c))) {
+    ReadPlan plan;
+    if (!words || plain || !(small || ring_ready(c)) || !plan_reads(segs, n_segs, kSlotBytes, plan)) {
         for (int i = 0; i < n_segs; ++i)
             if (segs[i].bytes)
                 HIPCHK(hipMemcpyAsync(segs[i].host, segs[i].dev, segs[i].bytes, hipMemcpyDeviceToHost, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
         return CS3D_OK;
     }
-    // the segments cut into slots (each piece 16-byte aligned in its slot)
-    std::vector<GatherList> lists;
-    std::vector<std::vector<ReadPiece>> pieces;
-    size_t used = kSlotBytes, total = 0;
-    for (int i = 0; i < n_segs; ++i) {
-        total += segs[i].bytes;
-        for (size_t at = 0; at < segs[i].bytes;) {
-            if (used + 16 > kSlotBytes || lists.back().n == kMaxGather) {
-                lists.emplace_back();
-                lists.back().n = 0;
-                pieces.emplace_back();
-                used = 0;
-            }
-            const size_t len = std::min(segs[i].bytes - at, kSlotBytes - used);
-            GatherList& g = lists.back();
-            g.src[g.n] = reinterpret_cast<const uint32_t*>(static_cast<const char*>(segs[i].dev) + at);
-            g.dst[g.n] = (uint32_t)(used / 4);
-            g.words[g.n++] = (uint32_t)(len / 4);
-            pieces.back().push_back(ReadPiece{static_cast<char*>(segs[i].host) + at, used, len});
-            used += (len + 15) / 16 * 16;
-            at += len;
-        }
-    }
-    const int n = (int)lists.size();
+    const int n = (int)plan.lists.size();
     if (n == 0) {
         HIPCHK(hipStreamSynchronize(c->stream));
         return CS3D_OK;
@@ -303,8 +273,6 @@ cs3d_status read_back(cs3d_ctx* c, const ReadSeg* segs, int n_segs) {
     auto slot = [&](int k) { return small ? c->stage_small : c->stage + (size_t)(k % kSlotsInRing) * kSlotBytes; };
     std::atomic<int> ready{0};            // slots whose data has arrived
     std::atomic<bool> stop{false};
-    std::vector<std::atomic<int>> done(n);  // readers that have copied slot k
-    for (auto& d : done) d.store(0, std::memory_order_relaxed);
     std::vector<std::thread> readers;
     int want = 0;
     auto start_readers = [&] {  // once data is there: the stream may hold steps still to run, and readers spin
@@ -317,8 +285,8 @@ cs3d_status read_back(cs3d_ctx* c, const ReadSeg* segs, int n_segs) {
                             if (stop.load(std::memory_order_relaxed)) return;
                             std::this_thread::yield();
                         }
-                        copy_share(pieces[k], slot(k), t, kReaders);
-                        done[k].fetch_add(1, std::memory_order_release);
+                        copy_share(plan.pieces[k], slot(k), t, kReaders);
+                        plan.done[k].fetch_add(1, std::memory_order_release);
                     }
                 });
             want = kReaders;
@@ -332,16 +300,16 @@ cs3d_status read_back(cs3d_ctx* c, const ReadSeg* segs, int n_segs) {
     for (int issued = 0, k = 0; k < n && e == hipSuccess; ++k) {
         for (; issued < n && issued < k + kSlotsInRing && e == hipSuccess; ++issued) {
             if (issued >= kSlotsInRing && want)
-                while (done[issued - kSlotsInRing].load(std::memory_order_acquire) < want) std::this_thread::yield();
-            launch_gather(lists[issued], slot(issued), c->stream);
+                while (plan.done[issued - kSlotsInRing].load(std::memory_order_acquire) < want) std::this_thread::yield();
+            launch_gather(plan.lists[issued], slot(issued), c->stream);
             e = hipGetLastError();
             if (e == hipSuccess && !small) e = hipEventRecord(c->stage_ev[issued % kSlotsInRing], c->stream);
         }
         if (e == hipSuccess) e = small ? hipStreamSynchronize(c->stream) : hipEventSynchronize(c->stage_ev[k % kSlotsInRing]);
         if (e != hipSuccess) break;
-        if (k == 0 && total >= kSerialRead) start_readers();
+        if (k == 0 && plan.total >= kSerialRead) start_readers();
         if (want) ready.store(k + 1, std::memory_order_release);
-        else copy_share(pieces[k], slot(k), 0, 1);
+        else copy_share(plan.pieces[k], slot(k), 0, 1);
     }
     if (e != hipSuccess) stop.store(true);
     for (auto& t : readers) t.join();
@@ -923,34 +891,36 @@ extern "C" cs3d_status cs3d_get_state(cs3d_ctx* c, cs3d_sys s, float* xyz, float
         return cell_out[1] ? cell_out[1] + (k - 1) * n : nullptr;
     };
     SysMeta m;
-    std::vector<ReadSeg> segs;
-    const size_t room = (size_t)h.cap * (6 * kSlots + 5) * sizeof(float);
-    if (room <= kSerialRead / 2) {
+    ReadSeg segs[12];
+    int n_segs = 0;
+    const size_t room = (size_t)h.cap * (6 * kSlots + 5);  // words
+    std::unique_ptr<float[]> buf;
+    if (room * sizeof(float) <= kSerialRead / 2) buf.reset(new (std::nothrow) float[room]);
+    if (buf) {
         // a small room: all of it with the metadata in one read, the live part copied out
-        std::vector<float> buf((size_t)h.cap * (6 * kSlots + 5));
-        float* at = buf.data();
-        segs.push_back(ReadSeg{p.meta + s, &m, sizeof(m)});
+        float* at = buf.get();
+        segs[n_segs++] = ReadSeg{p.meta + s, &m, sizeof(m)};
         for (int k = 0; k < 6; ++k, at += (size_t)h.cap * kSlots)
-            if (node_out[k / 3]) segs.push_back(ReadSeg{node[k] + (int64_t)h.base * kSlots, at, (size_t)h.cap * kSlots * 4});
+            if (node_out[k / 3]) segs[n_segs++] = ReadSeg{node[k] + (int64_t)h.base * kSlots, at, (size_t)h.cap * kSlots * 4};
         for (int k = 0; k < 5; ++k, at += h.cap)
-            if (cell_to(k, 0)) segs.push_back(ReadSeg{cell[k] + h.base, at, (size_t)h.cap * 4});
-        const cs3d_status st = read_back(c, segs.data(), (int)segs.size());
+            if (cell_to(k, 0)) segs[n_segs++] = ReadSeg{cell[k] + h.base, at, (size_t)h.cap * 4};
+        const cs3d_status st = read_back(c, segs, n_segs);
         if (st != CS3D_OK) return st;
         c->pool.seen[s] = m.n;
         const size_t n = (size_t)m.n;
         for (int k = 0; k < 6; ++k)
-            if (float* q = node_to(k, n)) std::memcpy(q, buf.data() + (size_t)k * h.cap * kSlots, n * kSlots * 4);
+            if (float* q = node_to(k, n)) std::memcpy(q, buf.get() + (size_t)k * h.cap * kSlots, n * kSlots * 4);
         for (int k = 0; k < 5; ++k)
-            if (float* q = cell_to(k, n)) std::memcpy(q, buf.data() + (size_t)h.cap * (6 * kSlots + k), n * 4);
+            if (float* q = cell_to(k, n)) std::memcpy(q, buf.get() + (size_t)h.cap * (6 * kSlots + k), n * 4);
     } else {
         cs3d_status st = read_meta(c, s, m);
         if (st != CS3D_OK) return st;
         const size_t n = (size_t)m.n;
         for (int k = 0; k < 6; ++k)
-            if (float* q = node_to(k, n)) segs.push_back(ReadSeg{node[k] + (int64_t)h.base * kSlots, q, n * kSlots * 4});
+            if (float* q = node_to(k, n)) segs[n_segs++] = ReadSeg{node[k] + (int64_t)h.base * kSlots, q, n * kSlots * 4};
         for (int k = 0; k < 5; ++k)
-            if (float* q = cell_to(k, n)) segs.push_back(ReadSeg{cell[k] + h.base, q, n * 4});
-        st = read_back(c, segs.data(), (int)segs.size());
+            if (float* q = cell_to(k, n)) segs[n_segs++] = ReadSeg{cell[k] + h.base, q, n * 4};
+        st = read_back(c, segs, n_segs);
         if (st != CS3D_OK) return st;
     }
     if (n_cells) *n_cells = m.n;

@@ -29,6 +29,7 @@
 #include <stdint.h>
 
 #include "../../include/cs3d.h"
+#include "cs3d_read.h"
 #include "cs3d_theta.h"
 
 namespace cs3d {
@@ -198,15 +199,6 @@ struct RoomInit {
     SysMeta meta;
     cs3d_params prm;
     int32_t sys, nsys;
-};
-
-// Pieces of device memory that one launch copies into a buffer (k_gather).
-constexpr int kMaxGather = 16;
-struct GatherList {
-    const uint32_t* src[kMaxGather];
-    uint32_t dst[kMaxGather];    // first word in the buffer, a multiple of 4
-    uint32_t words[kMaxGather];
-    int32_t n;
 };
 
 // kernel modes
