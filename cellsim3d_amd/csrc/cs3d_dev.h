@@ -205,7 +205,6 @@ struct RoomInit {
 enum : int32_t {
     M_STEP = 0,        // fused step path (state flags decided on the device)
     M_CON = 1,         // CalculateConForce only -> FC
-    M_BONDED = 2,      // spring + pressure + angle only -> FC
     M_DIS_V = 3,       // CalculateDisForce with V -> FD
     M_DIS_VA = 4,      // CalculateDisForce with VA -> FD
     M_COM = 5,         // CenterOfMass only

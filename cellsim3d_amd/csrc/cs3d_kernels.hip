@@ -1129,7 +1129,6 @@ struct SearchLds {
     int32_t lst[kPMax][kSlots];
     float part[3][6];
     int32_t wsum[3];
-    int32_t near;
 };
 
 // The search of one cell (every lane of the workgroup calls it) at its positions X,
@@ -1287,8 +1286,7 @@ __attribute__((noinline)) __device__ void hold_and_keep(CPool p, bool rands, int
 // first dissipative force (CalculateDisForce with the post-Integrate
 // velocities, propagate.cu:523-665) and VelocityUpdateA/B (propagate.cu:714-736),
 // over the stored contact candidates.  Modes: M_STEP (FC, V, accepted
-// partners), M_CON / M_INIT (FC, accepted partners), M_BONDED (spring +
-// pressure + angle -> FC), M_PAIRS (accepted partners only).
+// partners), M_CON / M_INIT (FC, accepted partners), M_PAIRS (accepted partners only).
 // ------------------------------------------------------------------------------
 // 6 waves per SIMD (80 VGPRs, 20,064 B of LDS): 2048 workgroups fit on the chip at
 // once, so 2000 cells run in one round instead of 1.5 (at 4 waves the kernel took
@@ -1347,7 +1345,6 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(kSearch ? 4
     const bool node = tid < kNodes;
     constexpr bool fused = kStep;
     const bool forces = kStep || mode != M_PAIRS;
-    const bool search = kStep || mode != M_BONDED;
     // a multi-system step walks the compact list of live slots (k_live)
     int nit = kLive ? cld(pk.n_live) : r.slot_hi - r.slot_lo;
     int done = -1;  // kSearch: the iteration whose cell has searched
@@ -1368,14 +1365,11 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(kSearch ? 4
         float vX = 0.f, vY = 0.f, vZ = 0.f;
         if (fused) { vX = ldu_now(rVX + cb, ln); vY = ldu_now(rVY + cb, ln); vZ = ldu_now(rVZ + cb, ln); }
         const int32_t* cand = p.CAND + (size_t)slot * kPMax * kSlots;  // the cell's candidate list (uniform)
-        int ncf = 0, key0 = 0, total = 0;
-        if (search) {
-            ncf = ldu_now(p.NCAND + cb, ln);
-            key0 = ldu_now(cand, ln);  // the first round's keys (in the list's room also where it is shorter)
-            // entries of the list, from a padding lane (by a vector load where this kernel
-            // may have just written it: the scalar cache does not see that)
-            total = kSearch ? ldu_now(p.NCAND + cb, vector_value(kNodes)) : cld(p.NCAND + cb + kNodes) >> kCandBits;
-        }
+        const int ncf = ldu_now(p.NCAND + cb, ln);
+        const int key0 = ldu_now(cand, ln);  // the first round's keys (in the list's room also where it is shorter)
+        // entries of the list, from a padding lane (by a vector load where this kernel
+        // may have just written it: the scalar cache does not see that)
+        int total = kSearch ? ldu_now(p.NCAND + cb, vector_value(kNodes)) : cld(p.NCAND + cb + kNodes) >> kCandBits;
         const MeshRec mt = ldu(mesh->th, ln);
         const float sg = fused ? ldu(mesh->gs, ln).sign : 0.f;
         const MeshRec r0 = ldu(mesh->r0, ln), ir0 = ldu(mesh->ir0, ln);
@@ -1470,7 +1464,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(kSearch ? 4
         if constexpr (kSearch) total = __builtin_amdgcn_readfirstlane(total) >> kCandBits;
         const int nc = ncf & ((1 << kCandBits) - 1), first = ncf >> kCandBits;
         float fdx = 0.f, fdy = 0.f, fdz = 0.f;
-        if (search) fill_owners(owner, lt, first, nc, 0);
+        fill_owners(owner, lt, first, nc, 0);
         if (fused && node) {
             const float vix = svx[lt], viy = svy[lt], viz = svz[lt];
             const float gint = P->internal_damping;
@@ -1549,7 +1543,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(kSearch ? 4
                 pair_pass<false, false>(cand, mask, in, lt, first, nc, total, u.pr, owner, R, k, sx, sy, sz,
                                              svx, svy, svz, snx, sny, snz, arr, cfx, cfy, cfz, fdx, fdy, fdz);
         }
-        if (search && node) {
+        if (node) {
             const float X = lds_reread(sx, lt), Y = lds_reread(sy, lt), Z = lds_reread(sz, lt);
             if (fused) {
                 const float vix = svx[lt], viy = svy[lt], viz = svz[lt];
@@ -3105,11 +3099,12 @@ static void launch(F kernel, dim3 grid, dim3 block, hipStream_t st, A... args) {
 
 // Grid of a step's cell kernel: a workgroup for each live cell that the host knows of
 // and a quarter more (cells that divide before it looks again; beyond the grid the
-// workgroups stride, up to the system's last live cell), at most 256 CUs x wg_per_cu if the caller set that.  One cell per
-// workgroup lets the dispatcher even out the load: at 20,000 cells k_con_dis takes
-// 156 us, with 4096 workgroups of 4 or 5 cells 183 us, with 2048 172 us, with 6144
-// 197 us (k_dis_post 94, 109, 103, 118).  A workgroup without a cell still costs its
-// dispatch, 2 to 3 ns, so rooms far larger than their tissue are not launched whole.
+// workgroups stride, up to the system's last live cell), at most 256 CUs x wg_per_cu if
+// the caller set that.  One cell per workgroup lets the dispatcher even out the load: at
+// 20,000 cells k_con_dis takes 138 us, with 2048 workgroups 160, with 4096 161, with 6144
+// 174, with 16,384 209 (k_dis_post 90; 100, 105, 113, 135).  A workgroup without a cell
+// still costs its dispatch, 2 to 3 ns, so rooms far larger than their tissue are not
+// launched whole.
 constexpr int kMinGrid = 256;  // one workgroup per CU: a small tissue's growth needs no wider grid
 static int grid_cover(const Range& r) {
     const int64_t slots = r.slot_hi - r.slot_lo, n = (int64_t)r.live_hint + r.live_hint / 4 + 8;
@@ -3164,8 +3159,8 @@ void launch_integrate(const Pool& p, const Range& r, int flags, int64_t step_ove
 // of k_integrate and nothing of another cell's search) instead of in a launch of its
 // own, which on the many steps that search nothing costs as much as a small kernel.
 // The search's LDS leaves room for 5 workgroups per CU instead of 8, so only where the
-// grid fits the chip at that: a step of 1 cell 18.2 instead of 19.3 us, of 8 cells 22.5
-// instead of 23.6, of 403 28.1 instead of 28.6, of 1000 29.7 instead of 30.5; with 2000
+// grid fits the chip at that: a step of 1 cell 18.4 instead of 19.5 us, of 8 cells 22.9
+// instead of 23.7, of 403 28.2 instead of 28.7, of 1000 33.1 instead of 34.0; with 2000
 // cells k_con_dis would take two rounds instead of one.
 static bool search_in_con(const Pool& p, const Range& r) { return grid_step(r, p.wg_per_cu) <= kSearchLive; }
 

@@ -6,7 +6,8 @@
 // rounded quotient, and returns whether that fixes the float: where
 // theta - 2^-37 and theta + 2^-37 round to the same float, every value between
 // them does (rounding is monotone), so (float)cs3d_acos(...) is that float.  The
-// callers take the general path otherwise, which about one angle in 2^14 needs.
+// callers take the general path otherwise, which one angle in 2^13 needs below 2 rad and
+// one in 2^14 above (the boundaries lie 2^-23 and 2^-22 apart).
 //
 // Method.  t = x + 0.425 with x = idk * y, y = 1/(den + 1e-3) from a float
 // reciprocal estimate and one Newton step in double (relative error below 2^-43: the
