@@ -299,10 +299,12 @@ cs3d_status cs3d_systems_poll(cs3d_ctx* ctx, int32_t first, int32_t count, int32
  * ids), counted on the device at the end of every step, so growing systems are
  * counted with their actual cell counts.  No counterpart in the reference. */
 cs3d_status cs3d_systems_work(cs3d_ctx* ctx, int32_t first, int32_t count, int64_t* cell_steps);
-/* Captures, instantiates and uploads the HIP graph that cs3d_step replays for
- * `sys` (or CS3D_ALL) without running it, so that a timed region holds replays
- * only.  The all-systems graph reads the systems in use on the device and stays
- * valid when systems are added or removed.  No counterpart in the reference. */
+/* Captures, instantiates and uploads the HIP graphs that cs3d_step replays for
+ * `sys` (or CS3D_ALL) without running them, one for each width of the grids that
+ * the room can come to need (for each quarter that a tissue grows), so that a timed
+ * region holds replays only.  The all-systems graphs read the systems in use on the
+ * device and stay valid when systems are added or removed.  No counterpart in the
+ * reference. */
 cs3d_status cs3d_graph_prepare(cs3d_ctx* ctx, cs3d_sys sys);
 
 /* Phases of one step, in launch order (one kernel launch each; a small grid's search is
